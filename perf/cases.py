@@ -235,6 +235,8 @@ def prepare(c, seed):
         _set_transform(at, seed, layers)
         if c["kind"] == "prefill":
             st["rotated"] = torch.zeros_like(st["q"])
+    if not c["one_call"]:  # a forward pass holds the tensors of each layer
+        st["layer"] = list(zip(*(st[name] for name in ("q", "k", "v", "rotated", "out") if name in st)))
     st["attn"] = at
     return st
 
@@ -244,25 +246,23 @@ def run(st):
     if c["kind"] == "sample":
         st["sampler"].sample_to_id_and_score_buffer(st["logits"], st["ids"], st["scores"])
         return {"ids": st["ids"], "scores": st["scores"]}
-    at, layers, q, out = st["attn"], c["layers"], st["q"], st["out"]
+    at, q, out = st["attn"], st["q"], st["out"]
     if c["kind"] == "decode":
         lens = st["lens"]
         if c["one_call"]:
-            at.decode(0, lens, q, out, n_layers=layers)
+            at.decode(0, lens, q, out, n_layers=c["layers"])
         elif c["step"]:
-            k, v = st["k"], st["v"]
-            for layer in range(layers):
-                at.decode_step(layer, lens, q[layer], k[layer], v[layer], out[layer])
+            for layer, (q, k, v, o) in enumerate(st["layer"]):
+                at.decode_step(layer, lens, q, k, v, o)
         else:
-            for layer in range(layers):
-                at.decode(layer, lens, q[layer], out[layer])
+            for layer, (q, o) in enumerate(st["layer"]):
+                at.decode(layer, lens, q, o)
         return out
     n, start = c["rows"], c["start"]
     if c["one_call"]:
-        at.prefill(0, 0, start, n, q, out, n_layers=layers)
+        at.prefill(0, 0, start, n, q, out, n_layers=c["layers"])
         return out
-    k, v, rotated = st["k"], st["v"], st["rotated"]
-    for layer in range(layers):
-        at.pre_attention(layer, 0, start, q[layer], k[layer], v[layer], rotated[layer])
-        at.prefill(layer, 0, start, n, rotated[layer], out[layer])
-    return {"queries": rotated, "out": out}
+    for layer, (q, k, v, rotated, o) in enumerate(st["layer"]):
+        at.pre_attention(layer, 0, start, q, k, v, rotated)
+        at.prefill(layer, 0, start, n, rotated, o)
+    return {"queries": st["rotated"], "out": out}
