@@ -339,7 +339,11 @@ float mi355_attn_last_kernel_ms(mi355_attn* handle);
  *   "decode_waves"     1, 2 or 4 waves per decode workgroup, 0 (default) = chosen
  *                      from the number of workgroups of the launch
  *   "rowwise_prefill"  0/1 run prefill row by row through the decode kernel
- *                      (the only path for an fp32 cache)
+ *   "prefill_short"    the prefill kernel for short calls, one 16-column tile of
+ *                      positions x query heads per workgroup: 1 always, 0 never, -1
+ *                      (default): by rule, where none of the options below asks for
+ *                      another kernel (an fp32 cache, which the tiled kernels do not
+ *                      take: always)
  *   "prefill_i8_min_rows" int8 cache: prefill calls of fewer rows run row by row
  *                      (default 16)
  *   "prefill_i8_stage_mib" int8 cache: limit of the staging area for half planes,

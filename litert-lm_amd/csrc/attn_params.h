@@ -181,6 +181,21 @@ constexpr int kPrefillQueues = 2;                     // ticket queues; workgrou
 constexpr int kPrefillOrderUnits = 128;               // entries of PrefillArgs::unit_order
 constexpr int kPrefillSchedInts = kPrefillQueues + 1;  // + count of workgroups that are done
 
+// Arguments of prefill_short_kernel (passed by value).
+struct PrefillShortArgs {
+  const void* q;  // [n_layers][n][hq][D] io dtype
+  void* out;
+  const uint8_t* cache;
+  const float* scales;  // int8 cache only
+  CacheGeom geom;
+  int32_t hq, group;
+  int32_t layer_begin, n_layers;
+  int32_t seq, q_pos0, n;
+  int32_t rows_log2;  // positions per workgroup (log2): prefill_short_rows_log2(group)
+  float scale, softcap;
+  int32_t window[kInlineLayers];  // of layers layer_begin .. layer_begin + n_layers - 1
+};
+
 struct KvCopyArgs {
   uint8_t* cache;
   CacheGeom geom;

@@ -68,6 +68,13 @@ int prefill_plan_probe(int n_layers, int n, int q_pos0, int hq, int hkv, const i
 hipError_t launch_prefill(const PrefillArgs& args, int kv_dtype, int io_dtype, PrefillPlans* plans,
                           hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
 
+// The kernel for short calls (prefill_short.hip): any cache and activation type, up to kInlineLayers layers.
+int prefill_short_rows_log2(int group);  // log2 of the positions a workgroup takes
+// The rule: window[0 .. n_layers) are the windows of the call's layers. Host only.
+bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, int n_layers, int q_pos0, int n);
+hipError_t launch_prefill_short(const PrefillShortArgs& args, int kv_dtype, int io_dtype, hipStream_t stream,
+                                hipEvent_t ev0, hipEvent_t ev1);
+
 // Scatter n boundary-layout rows into the cache planes / gather them back.
 hipError_t launch_kv_append(const KvCopyArgs& args, hipStream_t stream);
 hipError_t launch_kv_read(const KvCopyArgs& args, hipStream_t stream);

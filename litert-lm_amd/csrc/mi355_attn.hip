@@ -100,6 +100,7 @@ struct mi355_attn {
   size_t kv_stage_bytes = 0;
   int prefill_i8_min_rows = 16;  // int8 cache: calls of fewer rows take the row-wise path
   int prefill_i8_stage_mib = 2048;  // int8 cache: limit of the staging area (a pass covers as many layers as fit, at least one)
+  int prefill_short = -1;      // the kernel for short calls: 1 always, 0 never, < 0 by rule
   int prefill_key_split = -1;  // < 0 by rule, 0 off, > 0 key blocks per work item
   int prefill_rows16 = -1;     // which prefill kernel: 1 the one on 16x16x32 MFMAs, 0 the one on 32x32x16, < 0 by rule
   // the step before attention: per-layer constants in HBM and what is switched on
@@ -441,6 +442,16 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   return stage_out_end(h, 1, out, io_bytes, error_msg);
 }
 
+// Whether a prefill call runs on the kernel for short calls (prefill_short.hip): option prefill_short, or by rule where
+// no option asks for a particular one of the other kernels.
+bool takes_short_prefill(const mi355_attn* h, int layer_begin, int n_layers, int q_pos0, int n) {
+  if (n_layers > kInlineLayers || n > 65535 || h->prefill_short == 0) return false;
+  if (h->prefill_short == 1) return true;
+  if (h->prefill_rows16 >= 0 || h->prefill_key_split >= 0 || h->prefill_workgroups > 0) return false;
+  return prefill_short_wanted(h->cfg.kv_dtype, h->cfg.num_q_heads, h->cfg.num_kv_heads, h->window.data() + layer_begin,
+                              n_layers, q_pos0, n);
+}
+
 int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_pos0, int n, const void* q,
                  void* out, char** error_msg) {
   if (!h) return fail(error_msg, MI355_ATTN_INVALID_ARGUMENT, "null handle");
@@ -491,6 +502,30 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
         }
       }
     }
+  }
+  // (An int8 call that has to take the row-wise path - few rows, or recorded without a staging area - still does. A
+  // float32 cache has no tiled kernel; there `rowwise` stands for the option alone.)
+  if (!(i8 ? rowwise : h->rowwise_prefill) && takes_short_prefill(h, layer_begin, n_layers, q_pos0, n)) {
+    PrefillShortArgs a{};
+    a.q = dq;
+    a.out = dout;
+    a.cache = h->cache;
+    a.scales = h->scales;
+    a.geom = h->geom;
+    a.hq = h->cfg.num_q_heads;
+    a.group = h->cfg.num_q_heads / h->cfg.num_kv_heads;
+    a.layer_begin = layer_begin;
+    a.n_layers = n_layers;
+    a.seq = seq;
+    a.q_pos0 = q_pos0;
+    a.n = n;
+    a.rows_log2 = prefill_short_rows_log2(a.group);
+    a.scale = h->cfg.scale;
+    a.softcap = h->cfg.softcap;
+    for (int i = 0; i < n_layers; ++i) a.window[i] = h->window[layer_begin + i];
+    HIP_OR_RETURN(launch_prefill_short(a, h->cfg.kv_dtype, h->cfg.io_dtype, h->stream, e0, e1));
+    h->timed = h->timing;
+    return stage_out_end(h, 1, out, io_bytes, error_msg);
   }
   const size_t layer_io_bytes = (size_t)n * h->cfg.num_q_heads * h->cfg.head_dim * io_size(h);
   for (int l0 = 0; !rowwise && l0 < n_layers; l0 += layers_per_pass) {
@@ -1113,6 +1148,9 @@ int mi355_attn_set_option(mi355_attn* h, const char* name, int32_t value) {
   } else if (!strcmp(name, "prefill_i8_min_rows")) {
     if (value < 1) return MI355_ATTN_INVALID_ARGUMENT;
     h->prefill_i8_min_rows = value;
+  } else if (!strcmp(name, "prefill_short")) {
+    if (value < -1 || value > 1) return MI355_ATTN_INVALID_ARGUMENT;
+    h->prefill_short = value;
   } else if (!strcmp(name, "prefill_key_split")) {
     if (value < -1 || value > 4096) return MI355_ATTN_INVALID_ARGUMENT;
     h->prefill_key_split = value;
