@@ -1,12 +1,12 @@
 #!/usr/bin/env python3
-"""Build-time check of the decode kernels' device assembly.
+"""Build-time check of the device assembly of the kernels that stream K / V blocks into registers.
 
-The decode kernels keep up to 128 registers of K / V buffer loads in flight while they set up the query
+The decode kernels (and the prefill kernel for short calls, which is built from the same pieces) keep up to 128 registers of K / V buffer loads in flight while they set up the query
 operands (and, in the fused step, norm and rotate the new token's rows). That is laid out for straight-line
 code: a function call inside a kernel (s_swappc_b64 / s_setpc_b64 to a callee) would have to save those
 registers around the call, and scratch memory (register spills, a stack) would put memory traffic and waits
 into the block loop. This script reads the device assembly (hipcc -S) and fails if any instantiation of
-decode_attn_kernel or decode_merge_kernel contains a call, uses scratch memory or spills registers.
+decode_attn_kernel, decode_merge_kernel or prefill_short_kernel contains a call, uses scratch memory or spills registers.
 
 It also looks for one miscompilation that this compiler has produced in these kernels: the register allocator
 handing registers of a loaded V operand group (four registers, one matrix-instruction operand) to the softmax as
@@ -55,9 +55,9 @@ def torn_operands(body):
 
 def main(path):
     asm = open(path).read()
-    names = re.findall(r"^(_ZN5mi355\w*decode_(?:attn|merge)_kernel\w+):", asm, re.M)
+    names = re.findall(r"^(_ZN5mi355\w*(?:decode_(?:attn|merge)|prefill_short)_kernel\w+):", asm, re.M)
     if not names:
-        sys.exit(f"{path}: no decode kernel found")
+        sys.exit(f"{path}: no kernel to check found")
     bad = 0
     for name in names:
         body = re.search(r"^" + re.escape(name) + r":(.*?)\.Lfunc_end", asm, re.S | re.M).group(1)
@@ -69,7 +69,7 @@ def main(path):
         for line, operand, kinds in torn_operands(body):
             print(f"{name}: line {line}: matrix-instruction operand {operand} last written by {kinds}: live registers reused?")
             bad += 1
-    meta = re.findall(r"\.name:\s+(_ZN5mi355\w*decode_(?:attn|merge)_kernel\w+)\n(.*?)\.wavefront_size", asm, re.S)
+    meta = re.findall(r"\.name:\s+(_ZN5mi355\w*(?:decode_(?:attn|merge)|prefill_short)_kernel\w+)\n(.*?)\.wavefront_size", asm, re.S)
     if len(meta) != len(names):
         print(f"{path}: {len(names)} kernels but {len(meta)} metadata records")
         bad += 1
@@ -87,7 +87,7 @@ def main(path):
             bad += 1
     if bad:
         sys.exit(1)
-    print(f"{path}: {len(names)} decode kernel instantiations: no calls, no scratch memory, no vector register spills, no torn matrix operands")
+    print(f"{path}: {len(names)} kernel instantiations: no calls, no scratch memory, no vector register spills, no torn matrix operands")
 
 
 if __name__ == "__main__":

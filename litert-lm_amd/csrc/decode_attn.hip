@@ -39,19 +39,25 @@ namespace {
 // room for two waves per SIMD next to the 128 registers of K/V data in flight.
 // q_rows: the `group` query rows of this KV head, [group][D] (in HBM, or in LDS when the kernel has
 // produced them itself).
-template <int KV, int IO, int D>
-__device__ __forceinline__ void stage_q(u4* sm_q, const DecodeArgs& a, const typename IoT<IO>::type* q_rows, int kvh,
-                                        int seq, int layer, int lane) {
-  constexpr int NQ = KV == kF32 ? D / 16 : D / 32;
+template <int KV, int D>
+constexpr int query_steps() { return KV == kF32 ? D / 16 : D / 32; }
+
+template <int KV, int IO, int D, int NQ>
+__device__ __forceinline__ void load_q(u4 (&w)[NQ], const DecodeArgs& a, const typename IoT<IO>::type* q_rows,
+                                       int kvh, int seq, int layer, int lane) {
   const int n = lane & 15, g = lane >> 4;
   const bool live = n < a.group;
   const float* ks = KV == kI8 ? a.scales + a.geom.scale_offset(layer, seq, 0, kvh) : nullptr;
   const typename IoT<IO>::type* qrow = q_rows + (live ? n : 0) * D;
 #pragma unroll
-  for (int step = 0; step < NQ; ++step) {
-    const u4 w = q_operand<KV, IO, D>(qrow, ks, step, g);
-    sm_q[step * 64 + lane] = live ? w : u4{0, 0, 0, 0};
-  }
+  for (int step = 0; step < NQ; ++step) w[step] = q_operand<KV, IO, D>(qrow, ks, step, g);
+}
+
+template <int NQ>
+__device__ __forceinline__ void store_q(u4* sm_q, const u4 (&w)[NQ], int group, int lane) {
+  const bool live = (lane & 15) < group;
+#pragma unroll
+  for (int step = 0; step < NQ; ++step) sm_q[step * 64 + lane] = live ? w[step] : u4{0, 0, 0, 0};
 }
 
 // One wave's share of a partition: blocks first, first + step, ... < blk_end of
@@ -63,22 +69,16 @@ __device__ __forceinline__ void stage_q(u4* sm_q, const DecodeArgs& a, const typ
 // operands in sm_q while those loads were under way.
 // patch_blk: a block one of whose rows is not in the cache yet (-1: none); patch(kreg, vreg) puts that
 // row into the block's registers once they are loaded.
+//
+// The loads are issued on every path (`first` is wave-uniform: the caller has taken it through readfirstlane, and it is
+// the very value the block loop starts from): a wave that streams nothing comes with a resource of no bytes, from which
+// the loads return zeros without a trip to memory. Behind a branch of their own, the waits for whatever was loaded
+// before them would have to be waits for everything.
 template <int D>
 __device__ __forceinline__ void request_first_block(u4 (&kreg)[D / 16], u4 (&vreg)[D / 16], __amdgpu_buffer_rsrc_t krsrc,
-                                                    __amdgpu_buffer_rsrc_t vrsrc, bool streams, int first, int lane) {
-  // `first` is wave-uniform (the caller has taken it through readfirstlane) and is the very value the block
-  // loop starts from. A wave that streams nothing gets zeros, so that the registers hold defined values on
-  // every path.
-  if (streams) {
-    load_plane_block<D>(kreg, krsrc, first * (64 * D), lane * 16);
-    load_plane_block<D>(vreg, vrsrc, first * (64 * D), lane * 16);
-  } else {
-    const u4 zero = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) kreg[i] = zero;
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) vreg[i] = zero;
-  }
+                                                    __amdgpu_buffer_rsrc_t vrsrc, int first, int lane) {
+  load_plane_block<D>(kreg, krsrc, first * (64 * D), lane * 16);
+  load_plane_block<D>(vreg, vrsrc, first * (64 * D), lane * 16);
 }
 
 template <int KV, int IO, int D, class Patch>
@@ -141,8 +141,8 @@ __device__ __forceinline__ void stream_blocks(const DecodeArgs& a, __amdgpu_buff
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int i = 0; i < 4; ++i) bm = fmaxf(bm, s[T][i]);
-    bm = wave_xor_max(bm, 16);
-    bm = wave_xor_max(bm, 32);
+    bm = wave_xor_max<16>(bm);
+    bm = wave_xor_max<32>(bm);
     const float m_new = fmaxf(m_run, bm);
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
     const float alpha = fast_exp2(m_run - m_use);
@@ -275,7 +275,7 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
   static_assert(!PRE || INL, "the fused step needs the items in the argument block");
   constexpr int NWP = decode_wg_waves<NW, PRE>();  // waves of the workgroup; the first NW do the attention
   constexpr int VB = KvT<KV>::VB, NL = D / 16;
-  constexpr int NQ = KV == kF32 ? D / 16 : D / 32;
+  constexpr int NQ = query_steps<KV, D>();
   extern __shared__ float smem[];
 
   const int lane = threadIdx.x & 63;
@@ -325,18 +325,19 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
   if (p_lo >= p_hi) return;  // empty partition: uniform over the workgroup
 
   const uint8_t* kplane = cache + ((((int64_t)layer * max_seqs + seq) * hkv + kvh) * 2) * plane_bytes;  // geom.plane_offset
-  const __amdgpu_buffer_rsrc_t krsrc = plane_resource(kplane, plane_bytes);
-  const __amdgpu_buffer_rsrc_t vrsrc = plane_resource(kplane + plane_bytes, plane_bytes);
   const int blk_end = (p_hi + VB - 1) / VB;
+  const int first_blk = __builtin_amdgcn_readfirstlane(p_lo / VB + wave);
+  const int64_t streamed = wave < NW && first_blk < blk_end ? plane_bytes : 0;  // (a helper wave of a PRE workgroup streams nothing)
+  const __amdgpu_buffer_rsrc_t krsrc = plane_resource(kplane, streamed);
+  const __amdgpu_buffer_rsrc_t vrsrc = plane_resource(kplane + plane_bytes, streamed);
 
   u4* sm_q = reinterpret_cast<u4*>(smem) + wave * (NQ * 64);
   float m_run, l_run;
   f4 acc[NL];
   using io_t = typename IoT<IO>::type;
-  // The first block's loads go out before anything else (a helper wave of a PRE workgroup streams nothing).
+  // What the queries are made from is asked for first, the first block right behind it: loads complete in the order
+  // they were issued, so the queries are normed, rotated and staged while the block is still on its way.
   u4 kreg[NL], vreg[NL];
-  const int first_blk = __builtin_amdgcn_readfirstlane(p_lo / VB + wave);
-  request_first_block<D>(kreg, vreg, krsrc, vrsrc, wave < NW && first_blk < blk_end, first_blk, lane);
   if constexpr (PRE) {
     static_assert(D == kRowD, "row helpers are written for head_dim 256");
     constexpr int ESZ = KV == kF32 ? 4 : (KV == kI8 ? 1 : 2);
@@ -356,7 +357,8 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
       constexpr int kMaxRows = (kMaxGroup + 2 + NWP - 1) / NWP;
       const int d0 = 2 * lane, d1 = D / 2 + 2 * lane;
       float xs[kMaxRows][4];
-      // every row of this wave in flight before the first is waited for
+      float2 w0[kMaxRows], w1[kMaxRows], freq = {0.f, 0.f};
+      // every row of this wave, its norm's weights and the frequencies in flight before the first is waited for
 #pragma unroll
       for (int r = 0; r < kMaxRows; ++r) {
         const int row = wave + r * NWP;
@@ -365,17 +367,27 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
           const int64_t base = row < G ? ((int64_t)b * a.hq + kvh * G + row) * D : ((int64_t)b * hkv + kvh) * D;
           load_pair<IO>(src, base + d0, xs[r][0], xs[r][1]);
           load_pair<IO>(src, base + d1, xs[r][2], xs[r][3]);
+          const float* weights = row_weights(a.pre_constants, row < G ? 0 : (row == G ? 1 : 2), a.pre_q_scaled != 0, a.pre_k_scaled != 0);
+          w0[r] = w1[r] = float2{0.f, 0.f};
+          if (weights) {
+            w0[r] = *reinterpret_cast<const float2*>(weights + d0);
+            w1[r] = *reinterpret_cast<const float2*>(weights + d1);
+          }
         }
       }
-      const RowAngles ang = row_angles(a.pre_rope ? a.pre_constants : nullptr, t, lane);
+      if (a.pre_rope) freq = *reinterpret_cast<const float2*>(a.pre_constants + d0);
+      __builtin_amdgcn_sched_barrier(0);
+      request_first_block<D>(kreg, vreg, krsrc, vrsrc, first_blk, lane);
+      __builtin_amdgcn_sched_barrier(0);
+      const RowAngles ang = row_angles(a.pre_rope != 0, freq, t);
 #pragma unroll
       for (int r = 0; r < kMaxRows; ++r) {
         const int row = wave + r * NWP;
         if (row < nrows) {
           const int kind = row < G ? 0 : (row == G ? 1 : 2);
           const bool norm = kind == 0 ? a.pre_norm_q != 0 : (kind == 1 ? a.pre_norm_k != 0 : a.pre_norm_v != 0);
-          transform_row(xs[r], norm, row_weights(a.pre_constants, kind, a.pre_q_scaled != 0, a.pre_k_scaled != 0),
-                        a.pre_weight_offset, a.pre_eps, a.pre_rope != 0 && kind != 2, ang, lane);
+          const bool weighted = kind == 0 ? a.pre_q_scaled != 0 : (kind == 1 && a.pre_k_scaled != 0);
+          transform_row(xs[r], norm, weighted, w0[r], w1[r], a.pre_weight_offset, a.pre_eps, a.pre_rope != 0 && kind != 2, ang);
           if (kind == 0) {
             uint8_t* dst = reinterpret_cast<uint8_t*>(sm_rows + row * D);
             store_pair<IO>(dst + d0 * sizeof(io_t), xs[r][0], xs[r][1]);
@@ -390,9 +402,12 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
         }
       }
     }
-    __syncthreads();
+    // (a barrier for LDS alone: __syncthreads() would also wait for the block under way)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (wave >= NW) return;  // a helper wave: its share of the rows, nothing else
-    stage_q<KV, IO, D>(sm_q, a, sm_rows, kvh, seq, layer, lane);
+    u4 qw[NQ];
+    load_q<KV, IO, D>(qw, a, sm_rows, kvh, seq, layer, lane);
+    store_q(sm_q, qw, a.group, lane);
     // Row t in the registers of its block. K: chunk c of the row is the 16 bytes of lane (t % 16, g) in load
     // (t % VB) / 16 * KPT + j with c = 4 j + g. V: element d of the row sits in lane (d % 16, (t % 16) / 4), load
     // d / 16, at element slot 4 * ((t % VB) / 16) + t % 4 of the lane's 16 bytes.
@@ -438,13 +453,20 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
                              patch, lane, m_run, l_run, acc);
   } else {
     const io_t* q_rows = reinterpret_cast<const io_t*>(a.q) + ((int64_t)item * a.hq + kvh * a.group) * D;
-    stage_q<KV, IO, D>(sm_q, a, q_rows, kvh, seq, layer, lane);
+    u4 qw[NQ];
+    // (queries that are converted on the way would be waited for before the block is asked for: the block goes first)
+    if constexpr (KV == IO) load_q<KV, IO, D>(qw, a, q_rows, kvh, seq, layer, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    request_first_block<D>(kreg, vreg, krsrc, vrsrc, first_blk, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (KV != IO) load_q<KV, IO, D>(qw, a, q_rows, kvh, seq, layer, lane);
+    store_q(sm_q, qw, a.group, lane);
     auto patch = [](u4 (&)[NL], u4 (&)[NL]) {};
     stream_blocks<KV, IO, D>(a, krsrc, vrsrc, kreg, vreg, first_blk, blk_end, NW, vlo, p_hi, sm_q, -1, patch, lane, m_run,
                              l_run, acc);
   }
-  float l_tot = wave_xor_add(l_run, 16);
-  l_tot = wave_xor_add(l_tot, 32);
+  float l_tot = wave_xor_add<16>(l_run);
+  l_tot = wave_xor_add<32>(l_tot);
 
   const int G = a.group;
   if constexpr (NW == 1) {
@@ -525,7 +547,7 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
 template <int KV, int IO, int D, int NW, bool INL, bool PRE = false>
 hipError_t launch_inl(const DecodeArgs& a, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
   const dim3 grid(a.n_layers, a.batch, a.num_splits * a.geom.hkv);
-  constexpr int NQ = KV == kF32 ? D / 16 : D / 32;
+  constexpr int NQ = query_steps<KV, D>();
   const size_t lds = (size_t)NW * NQ * 64 * 16 + (size_t)NW * a.group * (D + 2) * sizeof(float) +
                      (PRE ? (size_t)a.group * D * sizeof(typename IoT<IO>::type) + 2 * (size_t)D * a.geom.esize : 0);
   // ev0/ev1 are attached to the dispatch itself: they carry the kernel's own

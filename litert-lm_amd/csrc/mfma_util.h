@@ -106,8 +106,43 @@ __device__ __forceinline__ float fast_tanh(float y) {
   return copysignf(r, y);
 }
 
-__device__ __forceinline__ float wave_xor_max(float v, int mask) { return fmaxf(v, __shfl_xor(v, mask, 64)); }
-__device__ __forceinline__ float wave_xor_add(float v, int mask) { return v + __shfl_xor(v, mask, 64); }
+// Reductions over lanes a power of two apart, on the vector ALU: the DPP modes and the row swaps of gfx950 cost a few
+// cycles each where a trip through the LDS crossbar (__shfl_xor) takes over a hundred. Every lane ends up with the same
+// sum of the same two operands as with a xor shuffle, bit for bit. All 64 lanes must be active.
+__device__ __forceinline__ float2 wave_swap16(float v) {  // {even row, odd row} of each pair of 16-lane rows
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return float2{__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ float2 wave_swap32(float v) {  // {lower half, upper half} of the wave
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return float2{__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+template <int MASK>
+__device__ __forceinline__ float wave_xor_max(float v) {
+  static_assert(MASK == 16 || MASK == 32, "rows or halves of a wave");
+  const float2 r = MASK == 16 ? wave_swap16(v) : wave_swap32(v);
+  return fmaxf(r.x, r.y);
+}
+template <int MASK>
+__device__ __forceinline__ float wave_xor_add(float v) {
+  static_assert(MASK == 16 || MASK == 32, "rows or halves of a wave");
+  const float2 r = MASK == 16 ? wave_swap16(v) : wave_swap32(v);
+  return r.x + r.y;
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+// The sum over all lanes, in every lane, in the order of a butterfly with xor distances 1, 2, 4, 8, 16, 32 (the mirrors
+// pair a lane with one of the partner group, whose lanes all hold the same sum by then).
+__device__ __forceinline__ float wave_sum(float v) {
+  v = dpp_add<0xB1>(v);   // quad_perm 1 0 3 2
+  v = dpp_add<0x4E>(v);   // quad_perm 2 3 0 1
+  v = dpp_add<0x141>(v);  // row_half_mirror
+  v = dpp_add<0x140>(v);  // row_mirror
+  v = wave_xor_add<16>(v);
+  return wave_xor_add<32>(v);
+}
 
 }  // namespace mi355
 #endif  // LITERT_LM_AMD_CSRC_MFMA_UTIL_H_

@@ -51,14 +51,19 @@ __global__ void __launch_bounds__(64 * kRowsPerWg) pre_attention_kernel(const Pr
   load_pair<IO>(src, base + d0, x[0], x[1]);
   load_pair<IO>(src, base + d1, x[2], x[3]);
 
-  // sine / cosine of the lane's two angles first: they depend on the position
-  // only, so their ~200 instructions run while the row's loads are in flight
+  // everything the row needs comes in one trip to memory: its channels, the norm's weights, the rotary frequencies
   const int t = a.pos + i;
   const bool rotate = a.rope && kind != 2;
-  const RowAngles ang = row_angles(rotate ? a.constants : nullptr, t, lane);
   const bool norm = kind == 0 ? a.norm_q != 0 : (kind == 1 ? a.norm_k != 0 : a.norm_v != 0);
-  transform_row(x, norm, row_weights(a.constants, kind, a.q_scaled != 0, a.k_scaled != 0), a.weight_offset, a.eps, rotate,
-                ang, lane);
+  const float* weights = row_weights(a.constants, kind, a.q_scaled != 0, a.k_scaled != 0);
+  float2 w0 = {0.f, 0.f}, w1 = {0.f, 0.f}, freq = {0.f, 0.f};
+  if (weights) {
+    w0 = *reinterpret_cast<const float2*>(weights + d0);
+    w1 = *reinterpret_cast<const float2*>(weights + d1);
+  }
+  if (rotate) freq = *reinterpret_cast<const float2*>(a.constants + d0);
+  const RowAngles ang = row_angles(rotate, freq, t);
+  transform_row(x, norm, weights != nullptr, w0, w1, a.weight_offset, a.eps, rotate, ang);
 
   if (kind == 0) {
     uint8_t* out = reinterpret_cast<uint8_t*>(a.q_out);

@@ -75,15 +75,14 @@ __device__ __forceinline__ int quantise(float x, float scale) {
 }
 
 // Sine / cosine of the lane's two angles at position t (they depend on the position only);
-// inv_freq: the layer's [128] rotary frequencies, nullptr: no rotation.
+// f: the layer's rotary frequencies of pairs 2l, 2l+1.
 struct RowAngles {
   float s0, c0, s1, c1;
 };
-__device__ __forceinline__ RowAngles row_angles(const float* inv_freq, int t, int lane) {
+__device__ __forceinline__ RowAngles row_angles(bool rotate, float2 f, int t) {
 #pragma clang fp contract(off)
   RowAngles r{0.f, 1.f, 0.f, 1.f};
-  if (inv_freq) {
-    const float2 f = *reinterpret_cast<const float2*>(inv_freq + 2 * lane);  // frequencies of pairs 2l, 2l+1
+  if (rotate) {
     sincosf((float)t * f.x, &r.s0, &r.c0);
     sincosf((float)t * f.y, &r.s1, &r.c1);
   }
@@ -91,21 +90,18 @@ __device__ __forceinline__ RowAngles row_angles(const float* inv_freq, int t, in
 }
 
 // x = the lane's channels 2l, 2l+1, 128+2l, 128+2l+1 of one row. norm: RMS-normalise the row (eps inside the
-// root), then scale channel d by weight_offset + weights[d] when weights != nullptr; rotate: apply `ang`.
+// root), then, if weighted, scale channel d by weight_offset + the weight of d, of which the lane brings its four (w0:
+// channels 2l, 2l+1, w1: 128+2l, 128+2l+1; loaded together with the row, so that the norm does not end in another
+// trip to memory); rotate: apply `ang`.
 // (Flags and pointers come as plain values: picked out of a struct by the row's kind, the struct ends up in
 // memory and the kernel several times slower.)
-__device__ __forceinline__ void transform_row(float (&x)[4], bool norm, const float* weights, float weight_offset,
-                                              float eps, bool rotate, const RowAngles& ang, int lane) {
+__device__ __forceinline__ void transform_row(float (&x)[4], bool norm, bool weighted, float2 w0, float2 w1,
+                                              float weight_offset, float eps, bool rotate, const RowAngles& ang) {
 #pragma clang fp contract(off)
-  const int d0 = 2 * lane, d1 = kRowD / 2 + 2 * lane;
   if (norm) {
-    float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+    const float ss = wave_sum((x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]));
     const float r = 1.0f / sqrtf(ss * (1.0f / kRowD) + eps);
-    if (weights) {
-      const float2 w0 = *reinterpret_cast<const float2*>(weights + d0);
-      const float2 w1 = *reinterpret_cast<const float2*>(weights + d1);
+    if (weighted) {
       x[0] = x[0] * r * (weight_offset + w0.x);
       x[1] = x[1] * r * (weight_offset + w0.y);
       x[2] = x[2] * r * (weight_offset + w1.x);

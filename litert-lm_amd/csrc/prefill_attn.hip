@@ -550,7 +550,7 @@ __global__ void __launch_bounds__(kWaves * 64) prefill_attn_kernel(const Prefill
     constexpr int kRowStrideF = 4 * D + 16;
     static_assert(2 * (kStretch * kRowStrideF) <= (kStages + kStages - 1) * kBlockBytes, "patches 0, 1 before the ticket");
     uint8_t* const patch = smem + wave * (kStretch * kRowStrideF) + (wave >= 2 ? 16384 : 0);
-    const float l_tot = wave_xor_add(l_run0, 32);
+    const float l_tot = wave_xor_add<32>(l_run0);
 #pragma unroll
     for (int dp = 0; dp < NDP; ++dp) {
 #pragma unroll
@@ -579,7 +579,7 @@ __global__ void __launch_bounds__(kWaves * 64) prefill_attn_kernel(const Prefill
     // float32 rows: the same route as the parts of a split tile, normalised, to the output
     constexpr int kRowStrideF = 4 * D + 16;
     uint8_t* const patch = smem + wave * (kStretch * kRowStrideF) + (wave >= 2 ? 16384 : 0);
-    const float l_tot = wave_xor_add(l_run0, 32);
+    const float l_tot = wave_xor_add<32>(l_run0);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
 #pragma unroll
     for (int dp = 0; dp < NDP; ++dp) {
@@ -604,7 +604,7 @@ __global__ void __launch_bounds__(kWaves * 64) prefill_attn_kernel(const Prefill
   } else {
     constexpr int kRowStride = 2 * D + 16;
     uint8_t* const patch = smem + wave * (kStretch * kRowStride);
-    const float l_tot = wave_xor_add(l_run0, 32);
+    const float l_tot = wave_xor_add<32>(l_run0);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
 #pragma unroll
     for (int dp = 0; dp < NDP; ++dp) {
@@ -917,8 +917,8 @@ __global__ void __launch_bounds__(kWaves16 * 64, 2) prefill_attn16_kernel(const 
         // The four lanes of a query compare notes only when one of them has seen a score that
         // exceeds the reference by more than the slack: rare after the first blocks.
         if (__any(bm > m_run[u] + kRescaleSlack)) {
-          bm = wave_xor_max(bm, 16);
-          bm = wave_xor_max(bm, 32);
+          bm = wave_xor_max<16>(bm);
+          bm = wave_xor_max<32>(bm);
         }
         const float m_new = bm > m_run[u] + kRescaleSlack ? bm : m_run[u];
         // (the reference starts at a finite kNoKeyYet, not at -inf: exp2(m_run - m_new) is then 0 when the first
@@ -990,8 +990,8 @@ __global__ void __launch_bounds__(kWaves16 * 64, 2) prefill_attn16_kernel(const 
     stores_after_q = 0;
 #pragma unroll
     for (int u = 0; u < kSub16; ++u) {
-      float l_tot = wave_xor_add(l_run[u], 16);
-      l_tot = wave_xor_add(l_tot, 32);
+      float l_tot = wave_xor_add<16>(l_run[u]);
+      l_tot = wave_xor_add<32>(l_tot);
       const int row = my_pos0 + kRows16 * u + n - a.q_pos0;
       // (lane n = 0 has a row to store: the wave issues the sub-tile's store instructions, NL / 2 of 16 bytes, NL
       // for float32 output, or NL + 1 for a part of a split tile)

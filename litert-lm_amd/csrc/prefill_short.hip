@@ -83,36 +83,34 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
   const int64_t q_elem = (((int64_t)li * a.n + row) * a.hq + kvh * a.group + (live ? head : 0)) * D;
 
   const uint8_t* kplane = a.cache + a.geom.plane_offset(layer, a.seq, kvh, 0);
-  const __amdgpu_buffer_rsrc_t krsrc = plane_resource(kplane, a.geom.plane_bytes);
-  const __amdgpu_buffer_rsrc_t vrsrc = plane_resource(kplane + a.geom.plane_bytes, a.geom.plane_bytes);
+  int blk = blk0 + wave;
+  // (a wave without a block has a resource of no bytes: its first loads return zeros without a trip to memory; behind a
+  // branch, the wait for the queries would have to be a wait for everything)
+  const int64_t streamed = blk < blk_end ? a.geom.plane_bytes : 0;
+  const __amdgpu_buffer_rsrc_t krsrc = plane_resource(kplane, streamed);
+  const __amdgpu_buffer_rsrc_t vrsrc = plane_resource(kplane + a.geom.plane_bytes, streamed);
 
-  // This wave's share of the query operands goes first, then its first K and V blocks: the wait for the former
-  // leaves the latter under way.
+  // This wave's share of the query operands goes first, then its first K and V blocks: the wait for the former leaves
+  // the latter under way. (Queries that are converted on the way would be waited for before the blocks are asked for:
+  // then the blocks go first.)
   static_assert(NQ % NW == 0, "every wave stages the same number of operands");
   constexpr int kQPerWave = NQ / NW;
   u4 qw[kQPerWave];
-  {
+  auto load_queries = [&]() {
     const float* ks = KV == kI8 ? a.scales + a.geom.scale_offset(layer, a.seq, 0, kvh) : nullptr;
     const io_t* qrow = reinterpret_cast<const io_t*>(a.q) + q_elem;
 #pragma unroll
-    for (int s = 0; s < kQPerWave; ++s) {
-      const u4 w = q_operand<KV, IO, D>(qrow, ks, wave * kQPerWave + s, g);
-      qw[s] = live ? w : u4{0, 0, 0, 0};
-    }
-  }
+    for (int s = 0; s < kQPerWave; ++s) qw[s] = q_operand<KV, IO, D>(qrow, ks, wave * kQPerWave + s, g);
+  };
+  if constexpr (KV == IO) load_queries();
   __builtin_amdgcn_sched_barrier(0);
   u4 kreg[NL], vreg[NL];
-  int blk = blk0 + wave;
-  if (blk < blk_end) {
-    load_plane_block<D, kCachedLoad>(kreg, krsrc, blk * kBlockBytes, lane * 16);
-    load_plane_block<D, kCachedLoad>(vreg, vrsrc, blk * kBlockBytes, lane * 16);
-  } else {
-#pragma unroll
-    for (int i = 0; i < NL; ++i) kreg[i] = vreg[i] = u4{0, 0, 0, 0};
-  }
+  load_plane_block<D, kCachedLoad>(kreg, krsrc, blk * kBlockBytes, lane * 16);
+  load_plane_block<D, kCachedLoad>(vreg, vrsrc, blk * kBlockBytes, lane * 16);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (KV != IO) load_queries();
 #pragma unroll
-  for (int s = 0; s < kQPerWave; ++s) sm_q[(wave * kQPerWave + s) * 64 + lane] = qw[s];
+  for (int s = 0; s < kQPerWave; ++s) sm_q[(wave * kQPerWave + s) * 64 + lane] = live ? qw[s] : u4{0, 0, 0, 0};
   // (a barrier for LDS alone: __syncthreads() would also wait for the blocks under way)
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
@@ -155,8 +153,8 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int i = 0; i < 4; ++i) bm = fmaxf(bm, s[T][i]);
-    bm = wave_xor_max(bm, 16);
-    bm = wave_xor_max(bm, 32);
+    bm = wave_xor_max<16>(bm);
+    bm = wave_xor_max<32>(bm);
     const float m_new = fmaxf(m_run, bm);
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
     const float alpha = fast_exp2(m_run - m_use);
@@ -177,8 +175,8 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
     if (nxt < blk_end) load_plane_block<D, kCachedLoad>(vreg, vrsrc, nxt * kBlockBytes, lane * 16);
     blk = nxt;
   }
-  float l_tot = wave_xor_add(l_run, 16);
-  l_tot = wave_xor_add(l_tot, 32);
+  float l_tot = wave_xor_add<16>(l_run);
+  l_tot = wave_xor_add<32>(l_tot);
 
   // Merge the waves that had a block: accumulators and (max, sum) through LDS, then a wave per column and 4 channels
   // per lane, so that whole rows leave.
