@@ -165,15 +165,16 @@ struct PrefillArgs {
   const int32_t* host_window;  // host copy of layer_window (for the ordering), may be null
   int32_t use_order;
   // Key split (launches with fewer work items than compute units): a work item covers at most kchunk
-  // key blocks of its tile, tiles with more blocks are cut into up to smax items whose unnormalised
+  // key blocks of its tile, tiles with more blocks are cut into up to smax items of equal length whose unnormalised
   // fp32 accumulators and (max, sum) pairs go to ws_acc / ws_ml, [layer][row][head][smax] x head_dim
   // and x 2 floats, and prefill_merge_kernel combines them. kchunk == 0: off.
   int32_t kchunk, smax;
+  int32_t direct;  // != 0: the kernel on 16x16x32 MFMAs with a workgroup per item, no plan
   float* ws_acc;
   float* ws_ml;
   int32_t rows16;  // 1: the kernel on 16x16x32 MFMAs, two workgroups per compute unit; 0: the one on 32x32x16; < 0: by rule
   // Work plan of the kernel on 16x16x32 MFMAs (device memory): [workgroups + 1] offsets into the item list, then
-  // two words per item, (unit, tile | part << 20), each workgroup's items in the order it runs them.
+  // two words per item, (unit, tile | part << 20), each workgroup's items in the order it runs them. nullptr: a direct launch.
   const int32_t* plan;
   uint16_t unit_order[128];
 };

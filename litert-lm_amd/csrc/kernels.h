@@ -24,12 +24,13 @@ bool prefill_supported(int kv_dtype, int io_dtype, int head_dim);
 // Bytes of half planes that a prefill over an int8 cache stages for `n_layers` layers of a call ending at row `end`.
 int64_t prefill_i8_stage_bytes(const CacheGeom& geom, int n_layers, int end);
 
-// Key split of a prefill launch (PrefillArgs::kchunk / smax): none (kchunk 0) unless the launch has
-// fewer work items than three quarters of the compute units; then at most 8 items per tile of at
-// least 4 key blocks each. option > 0 forces that many key blocks per item (tests), option 0 is off,
-// option < 0 the rule above. Reads n_layers, geom.hkv, group, n, q_pos0, layer_begin, host_window.
+// Key split of a prefill launch (PrefillArgs::kchunk / smax / direct): none (kchunk 0) unless the launch has fewer work
+// items than three quarters of the compute units; then at most 8 items per tile of at least 4 key blocks each, as many
+// and on the kernel that the measured times say. option > 0 forces that many key blocks per item (tests), option 0 is
+// off, option < 0 the rule. Reads n_layers, geom.hkv, group, n, q_pos0, layer_begin, host_window, rows16, max_workgroups.
 struct PrefillSplit {
   int kchunk = 0, smax = 1;
+  bool direct = false;  // on 16x16x32 MFMAs, a workgroup per item and no plan
   size_t rows = 0;  // rows of the workspace: n_layers * n * hq * smax
 };
 PrefillSplit plan_prefill_split(const PrefillArgs& args, int option);

@@ -584,6 +584,7 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
       }
       a.kchunk = split.kchunk;
       a.smax = split.smax;
+      a.direct = split.direct;
       a.ws_acc = h->d_pf_acc;
       a.ws_ml = h->d_pf_ml;
     }

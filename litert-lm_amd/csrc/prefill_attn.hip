@@ -66,6 +66,14 @@ struct El<kBF16> {
   static __device__ __forceinline__ f16v mfma(vec8 a, vec8 b, f16v c) { return mfma32_bf16(a, b, c); }
 };
 
+// Key blocks of one work item of a tile of nblk blocks, cut into as few parts of at most kchunk blocks as do, all of the
+// same length to a block (cut every kchunk blocks, the last part of a tile could be a single block, which costs an item
+// and a part of the merge like any other).
+MI355_HD int tile_chunk(int nblk, int kchunk) {
+  const int parts = (nblk + kchunk - 1) / kchunk;
+  return (nblk + parts - 1) / parts;
+}
+
 // Output element type: the cache's own 16-bit type, or float32 for float32 activations (the queries of such a
 // call are rounded to the cache's type by convert_queries_kernel before the attention kernel runs).
 template <int OUT>
@@ -174,8 +182,8 @@ __global__ void __launch_bounds__(kWaves * 64) prefill_attn_kernel(const Prefill
   // A ticket of a queue with qcnt units is (tile, part, unit), tile-major: a
   // queue's longest key loops first. Key blocks of a tile: from the first one the
   // window of its first row reaches to the one holding the diagonal of its last
-  // valid row; part p of a split tile covers blocks [p * kchunk, (p + 1) * kchunk)
-  // of those.
+  // valid row; part p of a split tile covers blocks [p * chunk, (p + 1) * chunk)
+  // of those, chunk = tile_chunk(blocks, kchunk).
   struct Item { int li, kvh, hb, tile, part, layer, window, wg_pos0, kb_lo, nblk_tile; };
   auto item_of = [&](int qx, int ticket) {
     Item it;
@@ -246,8 +254,9 @@ __global__ void __launch_bounds__(kWaves * 64) prefill_attn_kernel(const Prefill
   // Key blocks the workgroup walks (every wave walks all of them; blocks outside
   // a row's range are masked): the tile's, or this part of them.
   const bool split_tile = smax > 1 && it.nblk_tile > a.kchunk;
-  const int kb_lo = it.kb_lo + (smax > 1 ? it.part * a.kchunk : 0);
-  const int nblk = smax > 1 ? min(a.kchunk, it.nblk_tile - it.part * a.kchunk) : it.nblk_tile;
+  const int chunk = split_tile ? tile_chunk(it.nblk_tile, a.kchunk) : it.nblk_tile;
+  const int kb_lo = it.kb_lo + it.part * chunk;
+  const int nblk = min(chunk, it.nblk_tile - it.part * chunk);
 
   // A K or V block travels HBM/L2 -> LDS without touching registers: every
   // wave issues kXfers of the 16 wave-wide 1 KiB transfers of a block; the data
@@ -704,19 +713,31 @@ __global__ void __launch_bounds__(kWaves16 * 64, 2) prefill_attn16_kernel(const 
   const float c = CAP ? 1.f : a.scale * kLog2e;
   const int pos_end = a.q_pos0 + a.n;
 
-  // This workgroup's items, in the order the host planned them (no queue, no ticket: every wave reads the list).
+  // This workgroup's items, in the order the host planned them (no queue, no ticket: every wave reads the list). A direct
+  // launch (no plan) has a workgroup per item, unit fastest, then part, then tile from the longest down: with the number
+  // of units x parts a multiple or a divisor of 8, the workgroups of an XCD then walk the same key blocks at the same
+  // time, and its L2 serves all of them but the first.
   const int32_t* const plan_items = a.plan + gridDim.x + 1;
-  const int item_end = scalar_load(a.plan + blockIdx.x + 1);
+  const int item_end = a.plan ? scalar_load(a.plan + blockIdx.x + 1) : (int)blockIdx.x + 1;
+  const int units = a.n_layers * per_layer;
 
   struct Item { int li, kvh, layer, window, wg_pos0, part, head, my_pos0, kb0, nblk; bool split; };
   auto item_at = [&](int idx) {
     Item it;
     // (read through the scalar cache: a vector load here would make every item wait for all memory
     // operations under way, the previous item's stores included)
-    const int u = scalar_load(plan_items + 2 * idx);
-    const int w1 = scalar_load(plan_items + 2 * idx + 1);
-    const int tile = w1 & 0xFFFFF;
-    it.part = w1 >> 20;
+    int u, tile;
+    if (a.plan) {
+      u = scalar_load(plan_items + 2 * idx);
+      const int w1 = scalar_load(plan_items + 2 * idx + 1);
+      tile = w1 & 0xFFFFF;
+      it.part = w1 >> 20;
+    } else {
+      const int rest = idx / units;
+      u = idx - rest * units;
+      tile = (int)gridDim.x / (units * smax) - 1 - rest / smax;
+      it.part = rest % smax;
+    }
     it.li = u / per_layer;
     const int rem = u - it.li * per_layer;
     it.kvh = rem / hblocks;
@@ -729,8 +750,9 @@ __global__ void __launch_bounds__(kWaves16 * 64, 2) prefill_attn16_kernel(const 
     if (it.window > 0 && it.wg_pos0 - it.window + 1 > 0) kb_lo = (it.wg_pos0 - it.window + 1) / kKeysPerBlock;
     const int nblk_tile = last_pos / kKeysPerBlock - kb_lo + 1;
     it.split = smax > 1 && nblk_tile > a.kchunk;
-    it.kb0 = kb_lo + (smax > 1 ? it.part * a.kchunk : 0);
-    it.nblk = smax > 1 ? min(a.kchunk, nblk_tile - it.part * a.kchunk) : nblk_tile;
+    const int chunk = it.split ? tile_chunk(nblk_tile, a.kchunk) : nblk_tile;
+    it.kb0 = kb_lo + it.part * chunk;
+    it.nblk = min(chunk, nblk_tile - it.part * chunk);  // (<= 0: a part that this tile does not have, direct launches only)
     it.head = it.kvh * a.group + hb * HPB + (wave % HPB);
     it.my_pos0 = it.wg_pos0 + (wave / HPB) * kStretch;  // first of the wave's 32 positions
     return it;
@@ -782,9 +804,10 @@ __global__ void __launch_bounds__(kWaves16 * 64, 2) prefill_attn16_kernel(const 
   // when those blocks belong to the next item, whose first blocks, and whose queries (loaded into the
   // registers the last scores have just freed), are therefore under way while this item's last P.V and
   // its store run. Nothing waits and no barrier stands between two items.
-  int idx = scalar_load(a.plan + blockIdx.x);
+  int idx = a.plan ? scalar_load(a.plan + blockIdx.x) : (int)blockIdx.x;
   if (idx >= item_end) return;
   Item it = item_at(idx);
+  if (it.nblk <= 0) return;  // (uniform over the workgroup, in front of everything that waits)
   int ks = 0;        // K stage of the block being worked on
   int kfs = 0;       // K stage the next block asked for goes to
   int vs = 0;        // V stage of the block being worked on
@@ -1055,14 +1078,21 @@ __global__ void __launch_bounds__(kWaves16 * 64, 2) prefill_attn16_kernel(const 
   }
 }
 
-// Combines the parts of split tiles: grid (query head, row, layer), one thread
-// per channel. Rows of tiles that were not split have been written by the
-// attention kernel itself.
+// Combines the parts of split tiles: a wave per (query row, head), four channels per lane, grid (rows x heads / 4,
+// layer). Rows of tiles that were not split have been written by the attention kernel itself. Bound: HBM / Infinity
+// Cache (parts x 1 KiB in, a row out), so the parts of up to eight-way splits - all that the rule makes - are asked for
+// at once, in front of the (max, sum) pairs' arithmetic. (2,047 rows x 8 heads in two parts: 20 us with a thread per
+// channel and a workgroup per row, 13 us now, both as the time it adds to the call.)
 template <int OUT, int D>
-__global__ void __launch_bounds__(D) prefill_merge_kernel(const PrefillArgs a, int rows_per_tile) {
+__global__ void __launch_bounds__(256) prefill_merge_kernel(const PrefillArgs a, int rows_per_tile) {
+  static_assert(D == 256, "a wave holds a row, four channels per lane");
   using elem_t = typename OutEl<OUT>::type;
-  const int head = blockIdx.x, row = blockIdx.y, li = blockIdx.z, d = threadIdx.x;
-  const int window = a.layer_window[a.layer_begin + li];
+  constexpr int kAtOnce = 8;
+  const int lane = threadIdx.x & 63, li = blockIdx.y;
+  const int pair = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
+  if (pair >= a.n * a.hq) return;
+  const int row = pair / a.hq;
+  const int window = scalar_load(a.layer_window + a.layer_begin + li);
   const int wg_pos0 = a.q_pos0 + (row / rows_per_tile) * rows_per_tile;
   const int last_pos = min(wg_pos0 + rows_per_tile, a.q_pos0 + a.n) - 1;
   int kb_lo = 0;
@@ -1070,17 +1100,38 @@ __global__ void __launch_bounds__(D) prefill_merge_kernel(const PrefillArgs a, i
   const int nblk = last_pos / kKeysPerBlock - kb_lo + 1;
   if (nblk <= a.kchunk) return;
   const int parts = (nblk + a.kchunk - 1) / a.kchunk;
-  const int64_t slot0 = (((int64_t)li * a.n + row) * a.hq + head) * a.smax;
+  const int64_t out_row = (int64_t)li * a.n * a.hq + pair;
+  const float2* const ml = reinterpret_cast<const float2*>(a.ws_ml) + out_row * a.smax;
+  const float* const acc = a.ws_acc + out_row * a.smax * D + 4 * lane;
+  // the first parts go out before the maxima are known (a part that does not exist: the last one once more)
+  f4 v[kAtOnce];
+#pragma unroll
+  for (int u = 0; u < kAtOnce; ++u) v[u] = *reinterpret_cast<const f4*>(acc + (int64_t)min(u, parts - 1) * D);
   float M = -INFINITY;
-  for (int p = 0; p < parts; ++p) M = fmaxf(M, a.ws_ml[(slot0 + p) * 2]);
-  float A = 0.f, L = 0.f;
-  for (int p = 0; p < parts; ++p) {
-    const float m = a.ws_ml[(slot0 + p) * 2];
-    const float wgt = m == -INFINITY ? 0.f : fast_exp2(m - M);  // (a part none of whose keys the row sees)
-    A += wgt * a.ws_acc[(slot0 + p) * D + d];
-    L += wgt * a.ws_ml[(slot0 + p) * 2 + 1];
+  for (int p = 0; p < parts; ++p) M = fmaxf(M, ml[p].x);
+  f4 A = {0.f, 0.f, 0.f, 0.f};
+  float L = 0.f;
+  for (int p0 = 0; p0 < parts; p0 += kAtOnce) {
+    if (p0 > 0) {
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) v[u] = *reinterpret_cast<const f4*>(acc + (int64_t)min(p0 + u, parts - 1) * D);
+    }
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) {
+      if (p0 + u < parts) {
+        const float2 w = ml[p0 + u];
+        const float wgt = w.x == -INFINITY ? 0.f : fast_exp2(w.x - M);  // (a part none of whose keys the row sees)
+        A += wgt * v[u];
+        L += wgt * w.y;
+      }
+    }
   }
-  reinterpret_cast<elem_t*>(a.out)[(((int64_t)li * a.n + row) * a.hq + head) * D + d] = (elem_t)(L > 0.f ? A / L : 0.f);
+  elem_t o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (elem_t)(L > 0.f ? A[e] / L : 0.f);
+  elem_t* const dst = reinterpret_cast<elem_t*>(a.out) + out_row * D + 4 * lane;
+  if constexpr (sizeof(elem_t) == 4) *reinterpret_cast<u4*>(dst) = *reinterpret_cast<const u4*>(o);
+  else *reinterpret_cast<u2*>(dst) = *reinterpret_cast<const u2*>(o);
 }
 
 // float32 queries rounded (to nearest even) to the element type of the cache, 8 per thread: what the
@@ -1237,7 +1288,8 @@ void build_prefill_plan(const PrefillArgs& a, int hpb, int wgs, int cus, std::ve
       const int nblk = tile_key_blocks(a, rows_per_tile, w, t);
       const int parts = a.kchunk > 0 ? (nblk + a.kchunk - 1) / a.kchunk : 1;
       for (int part = 0; part < parts; ++part) {
-        const int blocks = a.kchunk > 0 ? std::min(a.kchunk, nblk - part * a.kchunk) : nblk;
+        const int chunk = a.kchunk > 0 ? tile_chunk(nblk, a.kchunk) : nblk;
+        const int blocks = std::min(chunk, nblk - part * chunk);
         for (int r = 0; r < per_layer; ++r) items.push_back(It{li * per_layer + r, t | (part << 20), blocks});
       }
     }
@@ -1464,18 +1516,20 @@ hipError_t launch_typed(const PrefillArgs& a, PrefillPlans* plans, hipStream_t s
   // Which kernel: rows16 < 0 leaves it to this rule: the kernel on 16x16x32 MFMAs (two workgroups
   // per CU) when there are at least two work items per CU, else the one on 32x32x16 MFMAs, whose
   // single workgroup per CU gets through an item in half the time.
-  b.rows16 = a.rows16 < 0 ? (all_items >= 2L * cus ? 1 : 0) : a.rows16;
+  // A direct launch is on 16x16x32 MFMAs with a workgroup per item (plan_prefill_split decided that).
+  b.rows16 = a.direct ? 1 : (a.rows16 < 0 ? (all_items >= 2L * cus ? 1 : 0) : a.rows16);
   // (the planned kernel needs the host's copy of the windows, and a plan of bounded size)
-  if (b.rows16 == 1 && (!a.host_window || all_items > kPlanMaxItems)) b.rows16 = 0;
+  if (b.rows16 == 1 && !a.direct && (!a.host_window || all_items > kPlanMaxItems)) b.rows16 = 0;
   auto workgroups = [&]() {
     const int slots = b.rows16 == 1 ? 2 * cus : cus;
     int w = all_items < slots ? (int)all_items : slots;
     if (a.max_workgroups > 0 && a.max_workgroups < w) w = a.max_workgroups;
     return w;
   };
-  int wgs = workgroups();
+  int wgs = a.direct ? items * a.smax : workgroups();
   int plan_slot = -1;
-  if (b.rows16 == 1) {
+  b.plan = nullptr;
+  if (b.rows16 == 1 && !a.direct) {
     hipError_t pe = plan_for(a, hpb, wgs, cus, plans, stream, &plan_slot);
     if (pe != hipSuccess) return pe;
     if (plan_slot >= 0) {
@@ -1501,7 +1555,8 @@ hipError_t launch_typed(const PrefillArgs& a, PrefillPlans* plans, hipStream_t s
     else if (err == hipSuccess) plans->pinned[plan_slot] = true;
   }
   if (err != hipSuccess || a.kchunk <= 0) return err;
-  hipLaunchKernelGGL((prefill_merge_kernel<OUT, D>), dim3(a.hq, a.n, a.n_layers), dim3(D), 0, stream, b, kStretch * pt);
+  hipLaunchKernelGGL((prefill_merge_kernel<OUT, D>), dim3((unsigned)(((int64_t)a.n * a.hq + 3) / 4), a.n_layers), dim3(256), 0, stream,
+                     b, kStretch * pt);
   return hipGetLastError();
 }
 
@@ -1590,13 +1645,33 @@ PrefillSplit plan_prefill_split(const PrefillArgs& a, int option) {
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       return out;
     if (items * 4 >= (long)cus * 3) return out;
-    int want = (int)std::min<long>(8, (cus + items - 1) / items);
-    want = std::min(want, max_nblk / 4);  // at least 4 key blocks per item
-    if (want <= 1) return out;
+    // Into how many parts, and on which kernel: the times in microseconds that both were measured to take for one round
+    // of items over the chip (one layer of 1,024 rows behind 3,072 and of 2,047 behind 6,157, 8 heads on 2, float32
+    // parts at 4.7 TB/s each way). The kernel on 32x32x16 MFMAs with one item per compute unit needs 15 us and 0.95 us a
+    // key block, the one on 16x16x32 with two items per compute unit 9 us and 1.58 us a block of both: of the two
+    // shapes the second is 11 % faster in four parts than the first in two on the longer call, the first 3 % faster in
+    // four parts than the second in eight on the shorter one.
+    const double part_us = 2.0 * a.n_layers * a.n * a.hq * 1024 / 4.7e6;
+    double best = 0;
+    int want = 1;
+    for (int direct = 0; direct <= (a.max_workgroups == 0 && a.rows16 < 0 ? 1 : 0); ++direct)
+      for (int p = 1; p <= 8 && (p == 1 || max_nblk / p >= 4); ++p) {
+        const long slots = direct ? 2L * cus : cus;
+        const double chunk = (max_nblk + p - 1) / p;
+        const double t = (direct ? 9.0 + 1.58 * chunk * ((items * p + slots - 1) / slots)
+                                 : 15.0 + 0.95 * chunk * ((items * p + slots - 1) / slots)) +
+                         (p > 1 ? 4.0 + part_us * p : 0.0);
+        if ((p > 1 || !direct) && (best == 0 || t < best)) {
+          best = t;
+          want = p;
+          out.direct = direct != 0;
+        }
+      }
+    if (want <= 1) return PrefillSplit{};
     kchunk = (max_nblk + want - 1) / want;
   }
   const int smax = (max_nblk + kchunk - 1) / kchunk;
-  if (smax <= 1) return out;
+  if (smax <= 1) return PrefillSplit{};
   out.kchunk = kchunk;
   out.smax = smax;
   out.rows = (size_t)a.n_layers * a.n * a.hq * smax;
