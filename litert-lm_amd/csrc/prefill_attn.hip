@@ -1705,12 +1705,10 @@ bool prefill_supported(int kv_dtype, int io_dtype, int head_dim) {
 // K planes of such a call are staged as the int8 values themselves): half(q x scale), one thread per 8 channels of
 // a query row.
 template <int IO, int D>
-__global__ void __launch_bounds__(256) stage_queries_i8_kernel(const void* __restrict__ q, _Float16* __restrict__ dst,
-                                                               const float* __restrict__ scales, CacheGeom geom, int layer_begin,
-                                                               int seq, int n, int hq, int group, int64_t pieces) {
+__device__ __forceinline__ void stage_queries_i8(const void* __restrict__ q, _Float16* __restrict__ dst,
+                                                 const float* __restrict__ scales, const CacheGeom& geom, int layer_begin,
+                                                 int seq, int n, int hq, int group, int64_t i) {
   static_assert(IO == kF32 || IO == kBF16, "half queries are taken as they are");
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= pieces) return;
   constexpr int kPieces = D / 8;
   const int d0 = 8 * (int)(i % kPieces);
   const int64_t row = i / kPieces;  // (layer, token, head)
@@ -1734,20 +1732,18 @@ __global__ void __launch_bounds__(256) stage_queries_i8_kernel(const void* __res
   *reinterpret_cast<h8*>(dst + row * D + d0) = o;
 }
 
-// Grid (chunks of a plane's range / 256, planes of the call): one thread per 16-byte chunk of an int8 plane, which
-// becomes two 16-byte chunks of the half plane (attn_params.h has both layouts):
+// One thread per 16-byte chunk of an int8 plane, which becomes two 16-byte chunks of the half plane (attn_params.h has
+// both layouts):
 //   K: chunk c of token t (channels 16 c .. + 15) -> chunks 2 c and 2 c + 1 of the same token, tile and row;
 //   V: a chunk holds 16 tokens of one channel, slots 4 T + j of a 64-token block; slots 0..7 are the 8 slots of the
 //      same chunk position in half block 2 B, slots 8..15 those in half block 2 B + 1.
-// Blocks of 64 tokens that no query of the call sees (in front of a layer's window) are left alone.
-__global__ void __launch_bounds__(256) dequant_planes_kernel(const uint8_t* __restrict__ cache, const float* __restrict__ scales,
-                                                             CacheGeom src, uint8_t* __restrict__ staged, CacheGeom dst,
-                                                             const int32_t* __restrict__ layer_window, int layer_begin,
-                                                             int seq, int q_pos0, int64_t chunks, int scale_k) {
-  const int64_t ci = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ci >= chunks) return;
+// Blocks of 64 tokens that no query of the call sees (in front of a layer's window) are left alone. plane: (layer of the
+// call, KV head, K / V).
+__device__ __forceinline__ void dequant_chunk(const uint8_t* __restrict__ cache, const float* __restrict__ scales,
+                                              const CacheGeom& src, uint8_t* __restrict__ staged, const CacheGeom& dst,
+                                              const int32_t* __restrict__ layer_window, int layer_begin, int seq, int q_pos0,
+                                              int plane, int64_t ci, int scale_k) {
   const int D = src.head_dim;
-  const int plane = blockIdx.y;  // (layer of the call, KV head, K / V)
   const int is_v = plane & 1;
   const int kvh = (plane >> 1) % src.hkv;
   const int li = (plane >> 1) / src.hkv;
@@ -1790,6 +1786,40 @@ __global__ void __launch_bounds__(256) dequant_planes_kernel(const uint8_t* __re
   }
 }
 
+// What a prefill over an int8 cache stages, in one launch: the first plane_blocks workgroups of each of the call's planes
+// (blocks_per_plane each) turn int8 chunks into half chunks, the ones behind them (none for half activations) scale the
+// queries. (As two launches the two passes took 5.6 + 5.2 us in front of a call of 1,024 rows behind 3,072, most of it
+// the launches.)
+struct StageI8Args {
+  const uint8_t* cache;
+  const float* scales;
+  CacheGeom src, dst;
+  uint8_t* staged;
+  const int32_t* layer_window;
+  int32_t layer_begin, seq, q_pos0, scale_k;
+  int32_t plane_blocks, blocks_per_plane;
+  int64_t chunks;  // per plane
+  const void* q;
+  _Float16* q_stage;
+  int32_t n, hq, group;
+  int64_t pieces;
+};
+template <int IO, int D>
+__global__ void __launch_bounds__(256) stage_i8_kernel(const StageI8Args a) {
+  const int block = (int)blockIdx.x;
+  if (block < a.plane_blocks) {
+    const int plane = block / a.blocks_per_plane;
+    const int64_t ci = (int64_t)(block - plane * a.blocks_per_plane) * 256 + threadIdx.x;
+    if (ci < a.chunks)
+      dequant_chunk(a.cache, a.scales, a.src, a.staged, a.dst, a.layer_window, a.layer_begin, a.seq, a.q_pos0, plane, ci, a.scale_k);
+    return;
+  }
+  if constexpr (IO != kF16) {
+    const int64_t i = (int64_t)(block - a.plane_blocks) * 256 + threadIdx.x;
+    if (i < a.pieces) stage_queries_i8<IO, D>(a.q, a.q_stage, a.scales, a.src, a.layer_begin, a.seq, a.n, a.hq, a.group, i);
+  }
+}
+
 // Bytes of the staging area for `n_layers` layers of a call that ends at position `end` (exclusive).
 int64_t prefill_i8_stage_bytes(const CacheGeom& g, int n_layers, int end) {
   return (int64_t)n_layers * g.hkv * 2 * round_up64(end, kTokenAlign) * g.head_dim * 2;
@@ -1809,21 +1839,35 @@ hipError_t launch_i8(const PrefillArgs& a, PrefillPlans* plans, hipStream_t stre
   g.esize = 2;
   g.plane_bytes = (int64_t)g.cap * g.head_dim * 2;
   const int64_t chunks = (int64_t)(g.cap / 64) * 4 * D;
+  StageI8Args st{};
+  st.cache = a.cache;
+  st.scales = a.scales;
+  st.src = a.geom;
+  st.dst = g;
+  st.staged = reinterpret_cast<uint8_t*>(a.kv_stage);
+  st.layer_window = a.layer_window;
+  st.layer_begin = a.layer_begin;
+  st.seq = a.seq;
+  st.q_pos0 = a.q_pos0;
+  st.scale_k = OUT == kF16 ? 1 : 0;
+  st.chunks = chunks;
+  st.blocks_per_plane = (int32_t)((chunks + 255) / 256);
+  const int64_t plane_blocks = (int64_t)st.blocks_per_plane * a.n_layers * a.geom.hkv * 2;
+  st.q = a.q;
+  st.q_stage = reinterpret_cast<_Float16*>(a.q_stage);
+  st.n = a.n;
+  st.hq = a.hq;
+  st.group = a.group;
+  st.pieces = OUT != kF16 ? (int64_t)a.n_layers * a.n * a.hq * (D / 8) : 0;
+  const int64_t blocks = plane_blocks + (st.pieces + 255) / 256;
+  if (blocks > INT32_MAX) return hipErrorInvalidValue;
+  st.plane_blocks = (int32_t)plane_blocks;
   // (the first launch of the call carries the start event of a timed call, the attention kernel the stop event)
-  hipExtLaunchKernelGGL(dequant_planes_kernel, dim3((unsigned)((chunks + 255) / 256), a.n_layers * a.geom.hkv * 2), dim3(256),
-                        0, stream, ev0, nullptr, 0, a.cache, a.scales, a.geom, reinterpret_cast<uint8_t*>(a.kv_stage), g,
-                        a.layer_window, a.layer_begin, a.seq, a.q_pos0, chunks, OUT == kF16 ? 1 : 0);
-  hipError_t e = hipGetLastError();
+  hipExtLaunchKernelGGL((stage_i8_kernel<OUT, D>), dim3((unsigned)blocks), dim3(256), 0, stream, ev0, nullptr, 0, st);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   PrefillArgs b = a;
-  if constexpr (OUT != kF16) {
-    const int64_t pieces = (int64_t)a.n_layers * a.n * a.hq * (D / 8);
-    hipLaunchKernelGGL((stage_queries_i8_kernel<OUT, D>), dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, a.q,
-                       reinterpret_cast<_Float16*>(a.q_stage), a.scales, a.geom, a.layer_begin, a.seq, a.n, a.hq, a.group,
-                       pieces);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    b.q = a.q_stage;
-  }
+  if constexpr (OUT != kF16) b.q = a.q_stage;
   b.q_staged = 1;
   b.cache = reinterpret_cast<const uint8_t*>(a.kv_stage);
   b.geom = g;
