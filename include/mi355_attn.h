@@ -297,6 +297,22 @@ int mi355_attn_prefill_plan_probe(int32_t n_layers, int32_t n, int32_t q_pos0, i
                                   int32_t* items_off_home);
 
 /*
+ * Host only, no device needed (tests of the dispatch; no counterpart in the reference): the kernel that a prefill call of
+ * n rows at q_pos0 over n_layers layers takes with every option at its default on a part with `compute_units` compute
+ * units (MI355X: 256), room for an int8 cache's staging area given; *parts (may be NULL): work items that the longest
+ * tile's keys are cut into. < 0 on bad arguments.
+ */
+enum {
+  MI355_ATTN_ROUTE_ROWWISE = 0,   /* every row an item of the decode kernel */
+  MI355_ATTN_ROUTE_SHORT = 1,     /* the kernel for short calls */
+  MI355_ATTN_ROUTE_TILED32 = 2,   /* 32x32x16 MFMAs, one workgroup per compute unit */
+  MI355_ATTN_ROUTE_PLANNED16 = 3, /* 16x16x32 MFMAs, two workgroups per compute unit and a work plan */
+  MI355_ATTN_ROUTE_DIRECT16 = 4   /* the same kernel, a workgroup per part and no plan */
+};
+int mi355_attn_prefill_route_probe(int32_t kv_dtype, int32_t n_layers, int32_t n, int32_t q_pos0, int32_t num_q_heads,
+                                   int32_t num_kv_heads, const int32_t* layer_window, int32_t compute_units, int32_t* parts);
+
+/*
  * Measurement aid, no counterpart in the reference: streams `bytes` of the KV
  * cache, starting `offset` bytes into it, through `workgroups` workgroups of
  * `waves` waves with the decode kernel's load pattern (non-temporal 16-byte

@@ -94,6 +94,7 @@ def lib() -> ctypes.CDLL:
     L.mi355_attn_decode_step.argtypes = [vp, i32, i32p, i32p, i32, vp, vp, vp, vp, i32, errp]
     L.mi355_attn_decode_layers.argtypes = [vp, i32, i32, i32p, i32p, i32, vp, vp, i32, errp]
     L.mi355_attn_stream_probe.argtypes = [vp, ctypes.c_uint64, ctypes.c_uint64, i32, i32, errp]
+    L.mi355_attn_prefill_route_probe.argtypes = [i32] * 6 + [i32p, i32, i32p]
     L.mi355_attn_reset.argtypes = [vp, i32, errp]
     L.mi355_attn_sync.argtypes = [vp, errp]
     L.mi355_attn_stream.argtypes = [vp]
@@ -106,8 +107,8 @@ def lib() -> ctypes.CDLL:
     L.mi355_attn_cache_bytes.restype = ctypes.c_uint64
     L.mi355_attn_version.restype = ctypes.c_char_p
     for name in ("create", "kv_append", "kv_set_scales", "kv_read", "set_layer_transform", "pre_attention", "prefill",
-                 "prefill_layers", "decode", "decode_layers", "decode_step", "decode_noalloc", "prefill_plan_probe", "stream_probe",
-                 "reset", "sync", "set_timing", "set_option"):
+                 "prefill_layers", "decode", "decode_layers", "decode_step", "decode_noalloc", "prefill_plan_probe",
+                 "prefill_route_probe", "stream_probe", "reset", "sync", "set_timing", "set_option"):
         getattr(L, "mi355_attn_" + name).restype = c
     _lib = L
     return L
@@ -299,6 +300,17 @@ class Attn:
     @property
     def cache_bytes(self) -> int:
         return int(lib().mi355_attn_cache_bytes(self._h))
+
+
+ROUTE_ROWWISE, ROUTE_SHORT, ROUTE_TILED32, ROUTE_PLANNED16, ROUTE_DIRECT16 = range(5)
+
+
+def prefill_route(kv_dtype, q_heads, kv_heads, windows, q_pos0, n, compute_units=256):
+    """mi355_attn_prefill_route_probe: (route, parts) of a prefill call over len(windows) layers, all options default."""
+    parts = ctypes.c_int32()
+    route = lib().mi355_attn_prefill_route_probe(kv_dtype, len(windows), n, q_pos0, q_heads, kv_heads, _i32_array(windows),
+                                                 compute_units, ctypes.byref(parts))
+    return route, parts.value
 
 
 def version() -> str:

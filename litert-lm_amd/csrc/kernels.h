@@ -33,7 +33,21 @@ struct PrefillSplit {
   bool direct = false;  // on 16x16x32 MFMAs, a workgroup per item and no plan
   size_t rows = 0;  // rows of the workspace: n_layers * n * hq * smax
 };
-PrefillSplit plan_prefill_split(const PrefillArgs& args, int option);
+// (cus: compute units to plan for, 0 = those of the current device)
+PrefillSplit plan_prefill_split(const PrefillArgs& args, int option, int cus = 0);
+
+// What the split is made of, for the rule that weighs a tiled launch against another kernel (host only): the rows of a
+// tile, the most key blocks that a tile of the call sees, and the number of parts and the kernel chosen for `items` work
+// items of up to that many blocks.
+struct PrefillParts {
+  int parts = 1;
+  bool direct = false;
+};
+int prefill_tile_rows(int group);
+int prefill_most_key_blocks(const int32_t* window, int n_layers, int q_pos0, int n, int tile_rows);
+long prefill_work_items(const PrefillArgs& args);  // of the launch, its split decided
+bool prefill_takes_plan(const PrefillArgs& args, long items, int cus);  // (a launch that is not direct)
+PrefillParts choose_prefill_parts(long items, int most, int n_layers, int n, int hq, int cus, bool may_direct);
 
 // Work plans of the prefill kernel on 16x16x32 MFMAs, kept by the handle: which workgroup runs which work items
 // in which order, computed on the host (longest processing time first over the workgroups: an item's time is

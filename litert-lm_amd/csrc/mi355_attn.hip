@@ -79,6 +79,8 @@ __global__ void iota_items_kernel(int32_t* lens, int32_t* seq_ids, int n, int q_
 
 }  // namespace
 
+constexpr int kI8MinRows = 16;  // int8 cache: prefill calls of fewer rows take the row-wise path unless an option moves that
+
 struct mi355_attn {
   mi355_attn_config cfg{};
   CacheGeom geom{};
@@ -98,7 +100,7 @@ struct mi355_attn {
   size_t q_stage_bytes = 0;
   void* d_kv_stage = nullptr;  // prefill over an int8 cache: the half planes of the layers of a pass
   size_t kv_stage_bytes = 0;
-  int prefill_i8_min_rows = 16;  // int8 cache: calls of fewer rows take the row-wise path
+  int prefill_i8_min_rows = kI8MinRows;  // int8 cache: calls of fewer rows take the row-wise path
   int prefill_i8_stage_mib = 2048;  // int8 cache: limit of the staging area (a pass covers as many layers as fit, at least one)
   int prefill_short = -1;      // the kernel for short calls: 1 always, 0 never, < 0 by rule
   int prefill_key_split = -1;  // < 0 by rule, 0 off, > 0 key blocks per work item
@@ -442,10 +444,18 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   return stage_out_end(h, 1, out, io_bytes, error_msg);
 }
 
+// The key split of a tiled launch, its workspace bounded where the rule decides.
+constexpr size_t kSplitRowsMax = (size_t)256 << 10;  // 256 Ki rows = 258 MiB at head_dim 256
+PrefillSplit split_of(const PrefillArgs& a, int option, int cus = 0) {
+  const PrefillSplit split = plan_prefill_split(a, option, cus);
+  return option < 0 && split.rows > kSplitRowsMax ? PrefillSplit{} : split;
+}
+
 // Whether a prefill call runs on the kernel for short calls (prefill_short.hip): option prefill_short, or by rule where
 // no option asks for a particular one of the other kernels.
+bool short_prefill_takes(int n_layers, int n) { return n_layers <= kInlineLayers && n <= 65535; }
 bool takes_short_prefill(const mi355_attn* h, int layer_begin, int n_layers, int q_pos0, int n) {
-  if (n_layers > kInlineLayers || n > 65535 || h->prefill_short == 0) return false;
+  if (!short_prefill_takes(n_layers, n) || h->prefill_short == 0) return false;
   if (h->prefill_short == 1) return true;
   if (h->prefill_rows16 >= 0 || h->prefill_key_split >= 0 || h->prefill_workgroups > 0) return false;
   return prefill_short_wanted(h->cfg.kv_dtype, h->cfg.num_q_heads, h->cfg.num_kv_heads, h->window.data() + layer_begin,
@@ -565,9 +575,7 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
     }
     a.kv_stage = h->d_kv_stage;
     a.kv_stage_bytes = (int64_t)h->kv_stage_bytes;
-    PrefillSplit split = plan_prefill_split(a, h->prefill_key_split);
-    constexpr size_t kSplitRowsMax = (size_t)256 << 10;  // 256 Ki rows = 258 MiB at head_dim 256
-    if (split.kchunk > 0 && split.rows > kSplitRowsMax && h->prefill_key_split < 0) split = PrefillSplit{};
+    const PrefillSplit split = split_of(a, h->prefill_key_split);
     if (split.kchunk > 0) {
       if (split.rows > kSplitRowsMax)
         return fail(error_msg, MI355_ATTN_RESOURCE_EXHAUSTED, "prefill_key_split=%d needs %zu workspace rows (limit %zu)",
@@ -1018,6 +1026,34 @@ int mi355_attn_prefill_plan_probe(int32_t n_layers, int32_t n, int32_t q_pos0, i
                                   int32_t* items_per_wg, int32_t* blocks_per_wg, int32_t* items_off_home) {
   return mi355::prefill_plan_probe(n_layers, n, q_pos0, num_q_heads, num_kv_heads, layer_window, workgroups, compute_units,
                                    items_per_wg, blocks_per_wg, items_off_home);
+}
+
+int mi355_attn_prefill_route_probe(int32_t kv_dtype, int32_t n_layers, int32_t n, int32_t q_pos0, int32_t num_q_heads,
+                                   int32_t num_kv_heads, const int32_t* layer_window, int32_t compute_units, int32_t* parts) {
+  if (kv_dtype < MI355_ATTN_F32 || kv_dtype > MI355_ATTN_I8 || n_layers < 1 || n < 1 || q_pos0 < 0 || num_kv_heads < 1 ||
+      num_q_heads < num_kv_heads || num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > kMaxGroup || !layer_window ||
+      compute_units < 1)
+    return -1;
+  if (parts) *parts = 1;
+  if (kv_dtype == MI355_ATTN_I8 && n < kI8MinRows) return MI355_ATTN_ROUTE_ROWWISE;
+  if (short_prefill_takes(n_layers, n) &&
+      prefill_short_wanted(kv_dtype, num_q_heads, num_kv_heads, layer_window, n_layers, q_pos0, n))
+    return MI355_ATTN_ROUTE_SHORT;
+  if (kv_dtype == MI355_ATTN_F32) return MI355_ATTN_ROUTE_ROWWISE;
+  PrefillArgs a{};
+  a.n_layers = n_layers;
+  a.n = n;
+  a.q_pos0 = q_pos0;
+  a.hq = num_q_heads;
+  a.group = num_q_heads / num_kv_heads;
+  a.geom.hkv = num_kv_heads;
+  a.host_window = layer_window;
+  a.rows16 = -1;
+  const PrefillSplit split = split_of(a, -1, compute_units);
+  if (parts) *parts = split.smax;
+  if (split.direct) return MI355_ATTN_ROUTE_DIRECT16;
+  a.kchunk = split.kchunk;
+  return prefill_takes_plan(a, prefill_work_items(a), compute_units) ? MI355_ATTN_ROUTE_PLANNED16 : MI355_ATTN_ROUTE_TILED32;
 }
 
 int mi355_attn_decode_step(mi355_attn* h, int32_t layer, const int32_t* seq_ids, const int32_t* kv_lens, int32_t batch,

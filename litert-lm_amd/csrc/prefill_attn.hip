@@ -1496,30 +1496,9 @@ hipError_t launch_typed(const PrefillArgs& a, PrefillPlans* plans, hipStream_t s
     for (int u = 0; u < units; ++u) b.unit_order[u] = (uint16_t)order[u];
     b.use_order = 1;
   }
-  long all_items = items;
-  if (a.kchunk > 0 && a.host_window) {
-    // work items of a key split: the parts that hold at least one key block (the tickets also
-    // number the empty ones, which the drawing thread skips)
-    const int tiles = (a.n + kStretch * pt - 1) / (kStretch * pt);
-    all_items = 0;
-    for (int li = 0; li < a.n_layers; ++li) {
-      const int w = a.host_window[a.layer_begin + li];
-      for (int t = 0; t < tiles; ++t) {
-        const int p0 = a.q_pos0 + t * kStretch * pt;
-        const int last = std::min(p0 + kStretch * pt, a.q_pos0 + a.n) - 1;
-        const int lo = (w > 0 && p0 - w + 1 > 0) ? (p0 - w + 1) / kKeysPerBlock : 0;
-        const int nblk = last / kKeysPerBlock - lo + 1;
-        all_items += (long)((nblk + a.kchunk - 1) / a.kchunk) * a.geom.hkv * (G / hpb);
-      }
-    }
-  }
-  // Which kernel: rows16 < 0 leaves it to this rule: the kernel on 16x16x32 MFMAs (two workgroups
-  // per CU) when there are at least two work items per CU, else the one on 32x32x16 MFMAs, whose
-  // single workgroup per CU gets through an item in half the time.
+  const long all_items = prefill_work_items(a);
   // A direct launch is on 16x16x32 MFMAs with a workgroup per item (plan_prefill_split decided that).
-  b.rows16 = a.direct ? 1 : (a.rows16 < 0 ? (all_items >= 2L * cus ? 1 : 0) : a.rows16);
-  // (the planned kernel needs the host's copy of the windows, and a plan of bounded size)
-  if (b.rows16 == 1 && !a.direct && (!a.host_window || all_items > kPlanMaxItems)) b.rows16 = 0;
+  b.rows16 = a.direct || prefill_takes_plan(a, all_items, cus) ? 1 : 0;
   auto workgroups = [&]() {
     const int slots = b.rows16 == 1 ? 2 * cus : cus;
     int w = all_items < slots ? (int)all_items : slots;
@@ -1618,57 +1597,101 @@ int prefill_plan_probe(int n_layers, int n, int q_pos0, int hq, int hkv, const i
   return total;
 }
 
-PrefillSplit plan_prefill_split(const PrefillArgs& a, int option) {
-  PrefillSplit out;
-  if (option == 0 || !a.host_window) return out;
-  const int G = a.group;
-  const int hpb = (G % 4 == 0) ? 4 : ((G % 2 == 0) ? 2 : 1);
-  const int rows_per_tile = kStretch * (4 / hpb);
+int prefill_tile_rows(int group) { return kStretch * (4 / (group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1))); }
+
+int prefill_most_key_blocks(const int32_t* window, int n_layers, int q_pos0, int n, int tile_rows) {
+  const int tiles = (n + tile_rows - 1) / tile_rows;
+  int most = 1;
+  for (int li = 0; li < n_layers; ++li) {
+    const int w = window[li];
+    if (li > 0 && w == window[li - 1]) continue;
+    for (int t = 0; t < tiles; ++t) {
+      const int p0 = q_pos0 + t * tile_rows;
+      const int last = std::min(p0 + tile_rows, q_pos0 + n) - 1;
+      const int lo = (w > 0 && p0 - w + 1 > 0) ? (p0 - w + 1) / kKeysPerBlock : 0;
+      most = std::max(most, last / kKeysPerBlock - lo + 1);
+    }
+  }
+  return most;
+}
+
+// Work items of a launch: tiles, or the parts of a key split that hold at least one key block (the tickets also number
+// the empty ones, which the drawing thread skips).
+long prefill_work_items(const PrefillArgs& a) {
+  const int rows_per_tile = prefill_tile_rows(a.group);
   const int tiles = (a.n + rows_per_tile - 1) / rows_per_tile;
-  const long items = (long)a.n_layers * a.geom.hkv * (G / hpb) * tiles;
-  int max_nblk = 1;
+  const long per_tile = (long)a.geom.hkv * (a.group * rows_per_tile / (kStretch * 4));  // KV heads x head blocks
+  if (a.kchunk <= 0 || !a.host_window) return a.n_layers * per_tile * tiles;
+  long items = 0;
   for (int li = 0; li < a.n_layers; ++li) {
     const int w = a.host_window[a.layer_begin + li];
     for (int t = 0; t < tiles; ++t) {
       const int p0 = a.q_pos0 + t * rows_per_tile;
       const int last = std::min(p0 + rows_per_tile, a.q_pos0 + a.n) - 1;
       const int lo = (w > 0 && p0 - w + 1 > 0) ? (p0 - w + 1) / kKeysPerBlock : 0;
-      max_nblk = std::max(max_nblk, last / kKeysPerBlock - lo + 1);
+      const int nblk = last / kKeysPerBlock - lo + 1;
+      items += (nblk + a.kchunk - 1) / a.kchunk * per_tile;
     }
   }
+  return items;
+}
+
+// Which kernel: rows16 < 0 leaves it to this rule: the planned one on 16x16x32 MFMAs (two workgroups per CU) when there
+// are at least two work items per CU, else the one on 32x32x16 MFMAs, whose single workgroup per CU gets through an item
+// in half the time. (The planned kernel needs the host's copy of the windows, and a plan of bounded size.)
+bool prefill_takes_plan(const PrefillArgs& a, long items, int cus) {
+  return (a.rows16 < 0 ? items >= 2L * cus : a.rows16 == 1) && a.host_window && items <= kPlanMaxItems;
+}
+
+PrefillParts choose_prefill_parts(long items, int most, int n_layers, int n, int hq, int cus, bool may_direct) {
+  PrefillParts out;
+  if (items * 4 >= (long)cus * 3) return out;
+  // Into how many parts, and on which kernel: the times in microseconds that both were measured to take for one round
+  // of items over the chip (one layer of 1,024 rows behind 3,072 and of 2,047 behind 6,157, 8 heads on 2, float32
+  // parts at 4.7 TB/s each way). The kernel on 32x32x16 MFMAs with one item per compute unit needs 15 us and 0.95 us a
+  // key block, the one on 16x16x32 with two items per compute unit 9 us and 1.58 us a block of both: of the two
+  // shapes the second is 11 % faster in four parts than the first in two on the longer call, the first 3 % faster in
+  // four parts than the second in eight on the shorter one. (Launches that fill a small part of the chip take less than
+  // this: prefill_short_wanted has what the launches that come of it were measured to take.)
+  const double part_us = 2.0 * n_layers * n * hq * 1024 / 4.7e6;
+  double best = 0;
+  for (int direct = 0; direct <= (may_direct ? 1 : 0); ++direct)
+    for (int p = 1; p <= 8 && (p == 1 || most / p >= 4); ++p) {
+      const long slots = direct ? 2L * cus : cus;
+      const double chunk = (most + p - 1) / p;
+      const double t = (direct ? 9.0 + 1.58 * chunk * ((items * p + slots - 1) / slots)
+                               : 15.0 + 0.95 * chunk * ((items * p + slots - 1) / slots)) +
+                       (p > 1 ? 4.0 + part_us * p : 0.0);
+      if ((p > 1 || !direct) && (best == 0 || t < best)) {
+        best = t;
+        out.parts = p;
+        out.direct = direct != 0;
+      }
+    }
+  return out;
+}
+
+PrefillSplit plan_prefill_split(const PrefillArgs& a, int option, int cus) {
+  PrefillSplit out;
+  if (option == 0 || !a.host_window) return out;
+  const int G = a.group;
+  const int hpb = (G % 4 == 0) ? 4 : ((G % 2 == 0) ? 2 : 1);
+  const int rows_per_tile = prefill_tile_rows(G);
+  const int tiles = (a.n + rows_per_tile - 1) / rows_per_tile;
+  const long items = (long)a.n_layers * a.geom.hkv * (G / hpb) * tiles;
+  const int max_nblk = prefill_most_key_blocks(a.host_window + a.layer_begin, a.n_layers, a.q_pos0, a.n, rows_per_tile);
   int kchunk;
   if (option > 0) {
     kchunk = option;
   } else {
-    int cus = 0, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    int dev = 0;
+    if (cus <= 0 && (hipGetDevice(&dev) != hipSuccess ||
+                     hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess))
       return out;
-    if (items * 4 >= (long)cus * 3) return out;
-    // Into how many parts, and on which kernel: the times in microseconds that both were measured to take for one round
-    // of items over the chip (one layer of 1,024 rows behind 3,072 and of 2,047 behind 6,157, 8 heads on 2, float32
-    // parts at 4.7 TB/s each way). The kernel on 32x32x16 MFMAs with one item per compute unit needs 15 us and 0.95 us a
-    // key block, the one on 16x16x32 with two items per compute unit 9 us and 1.58 us a block of both: of the two
-    // shapes the second is 11 % faster in four parts than the first in two on the longer call, the first 3 % faster in
-    // four parts than the second in eight on the shorter one.
-    const double part_us = 2.0 * a.n_layers * a.n * a.hq * 1024 / 4.7e6;
-    double best = 0;
-    int want = 1;
-    for (int direct = 0; direct <= (a.max_workgroups == 0 && a.rows16 < 0 ? 1 : 0); ++direct)
-      for (int p = 1; p <= 8 && (p == 1 || max_nblk / p >= 4); ++p) {
-        const long slots = direct ? 2L * cus : cus;
-        const double chunk = (max_nblk + p - 1) / p;
-        const double t = (direct ? 9.0 + 1.58 * chunk * ((items * p + slots - 1) / slots)
-                                 : 15.0 + 0.95 * chunk * ((items * p + slots - 1) / slots)) +
-                         (p > 1 ? 4.0 + part_us * p : 0.0);
-        if ((p > 1 || !direct) && (best == 0 || t < best)) {
-          best = t;
-          want = p;
-          out.direct = direct != 0;
-        }
-      }
-    if (want <= 1) return PrefillSplit{};
-    kchunk = (max_nblk + want - 1) / want;
+    const PrefillParts c = choose_prefill_parts(items, max_nblk, a.n_layers, a.n, a.hq, cus, a.max_workgroups == 0 && a.rows16 < 0);
+    if (c.parts <= 1) return out;
+    out.direct = c.direct;
+    kchunk = (max_nblk + c.parts - 1) / c.parts;
   }
   const int smax = (max_nblk + kchunk - 1) / kchunk;
   if (smax <= 1) return PrefillSplit{};

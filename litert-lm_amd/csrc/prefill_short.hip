@@ -251,26 +251,37 @@ int prefill_short_rows_log2(int group) {
   return r;
 }
 
-// Whether the short kernel is expected to finish a call before the tiled kernels of prefill_attn.hip, by the times in
-// microseconds that both were measured to take (head_dim 256, MI355X, calls queued back to back, 64 to 2,048 rows behind
-// 0 to 4,096 cached ones, 1 to 40 layers; the two formulas are within some 15 % of the measured times, and the short
-// kernel has to come out ahead by as much). Examples, tiled / short, bfloat16, 4 query heads on 1 KV head: one layer of 64
-// rows 9.9 / 5.1 us, 256 rows 15.9 / 8.0, 1,024 rows 29.5 / 14.1, 2,048 rows 41.2 / 29.6; four layers of 1,024 rows with
-// a window of 512 41 / 27, eight 32 / 47, 26 of 256 rows 20 / 28; 64 rows behind 4,096 (8 heads on 2) 32 / 38. int8 cache,
-// 300 rows 24 / 10, 256 rows behind 3,072 47 / 31. A float32 cache always takes the short kernel: the alternative is
-// one decode item per row, which reads every key once per position instead of once per 16 columns (300 rows 36 / 17,
-// 300 behind 2,000 305 / 81).
+// Whether the short kernel is expected to finish a call before the tiled kernels of prefill_attn.hip: both sides by
+// formulas fitted to measured times (head_dim 256, MI355X, calls queued back to back, 770 shapes spread at random over
+// 16 to 4,096 rows behind 0 to 12,000 cached ones, 1 to 34 layers with and without windows, sixteen head counts). Nine
+// tenths of the times are within 15 % of the formulas, and what they choose takes 0.3 % longer than the better side in
+// the mean (on 600 other shapes 1.5 %, most of it the spread between two runs). Examples, tiled / short, us: bfloat16, 4
+// query heads on 1 KV head, one layer of 64 rows 9.9 / 5.1, 256 rows 15.9 / 8.0, 1,024 rows 25.7 / 13.6, 1,370
+// rows behind 1,338 35 / 38, 17 behind 1,207 19 / 14, 26 layers of 256 rows 20 / 28; 8 heads on 2, 2 layers of 1,768
+// behind 693 83 / 96. int8 cache, 300 rows 24 / 10, 256 rows behind 3,072 47 / 31. A float32 cache always takes the short
+// kernel: the alternative is one decode item per row, which reads every key once per position instead of once per 16
+// columns (300 rows 36 / 17, 300 behind 2,000 305 / 81).
+//
+// What decides for the short kernel beside the key blocks themselves is what one XCD has to do. Units (layer x KV head)
+// vary fastest over the workgroups, which go round the eight XCDs, so with a number of units that shares a factor f with 8
+// a unit's tiles all go to 8 / f of them: with 8 units the only global layer among windowed ones is the work of a single
+// XCD (8 layers of 1,686 rows behind 1,059, window 512: 204 us, tiled 92), and units whose planes do not fit its L2
+// (4 MiB) together are read from behind it again and again.
+//
 // The activation type is not part of the rule, so that calls that differ in nothing else run the same arithmetic.
 bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, int n_layers, int q_pos0, int n) {
-  constexpr int kCus = 256;  // (what the times were measured on; the launches themselves ask the device)
+  constexpr int kCus = 256, kXcds = 8;  // what the times were measured on
   if (kv_dtype == kF32) return true;
+  const bool i8 = kv_dtype == kI8;
   const int group = hq / hkv, rows_log2 = prefill_short_rows_log2(group);
-  const int vb = kv_dtype == kI8 ? 64 : 32;
-  const double wgs = (double)n_layers * hkv * short_tiles(q_pos0, n, rows_log2);
+  const int vb = i8 ? 64 : 32;
+  const int units = n_layers * hkv;
+  const double tiles = short_tiles(q_pos0, n, rows_log2), wgs = units * tiles;
   if (wgs > 16 * kCus) return false;
   const int hpb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
-  const int tile_rows = 32 * (4 / hpb), tiles = (n + tile_rows - 1) / tile_rows;
-  const double items = (double)n_layers * hkv * (group / hpb) * tiles;
+  const int tile_rows = prefill_tile_rows(group);
+  const long items = (long)n_layers * hkv * (group / hpb) * ((n + tile_rows - 1) / tile_rows);
+  const int classes = units % 8 == 0 ? 8 : (units % 4 == 0 ? 4 : (units % 2 == 0 ? 2 : 1));  // of units that share XCDs
   // key blocks of a stretch of `rows` positions: mean over the call (the count is linear in the position but for the
   // corner at the window, so a few samples do) and most
   auto blocks = [&](int w, int first, int rows, int block) {
@@ -279,45 +290,81 @@ bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, 
     return (double)(last / block - lo / block + 1);
   };
   constexpr int kSamples = 9;
-  double short_mean = 0, short_most = 0, tiled_mean = 0, tiled_most = 0;
-  for (int li = 0; li < n_layers; ++li)
-    for (int k = 0; k < kSamples; ++k) {
-      const int at = q_pos0 + (int)((int64_t)(n - 1) * k / (kSamples - 1));
-      const double bs = blocks(window[li], at >> rows_log2 << rows_log2, 1 << rows_log2, vb);
-      const double bt = blocks(window[li], at, n < tile_rows ? n : tile_rows, 32);
-      short_mean += bs;
-      tiled_mean += bt;
-      if (bs > short_most) short_most = bs;
-      if (bt > tiled_most) tiled_most = bt;
+  double short_mean = 0, short_most = 0, short_least = 1e9, tiled_mean = 0, tiled_most = 0, tiled_least = 1e9;
+  double load[kXcds] = {}, planes[kXcds] = {};  // of a class: key blocks per compute unit, MiB of K and V that it sees
+  double sum_s = 0, sum_t = 0;                  // of the layer (kept from the layer before where the window is the same)
+  int seen = 0;
+  for (int li = 0; li < n_layers; ++li) {
+    if (li == 0 || window[li] != window[li - 1]) {
+      sum_s = sum_t = 0;
+      for (int k = 0; k < kSamples; ++k) {
+        const int at = q_pos0 + (int)((int64_t)(n - 1) * k / (kSamples - 1));
+        const double bs = blocks(window[li], at >> rows_log2 << rows_log2, 1 << rows_log2, vb);
+        const double bt = blocks(window[li], at, n < tile_rows ? n : tile_rows, 32);
+        sum_s += bs;
+        sum_t += bt;
+        short_most = fmax(short_most, bs);
+        short_least = fmin(short_least, bs);
+        tiled_most = fmax(tiled_most, bt);
+        tiled_least = fmin(tiled_least, bt);
+      }
+      const int lo = window[li] > 0 && q_pos0 - window[li] + 1 > 0 ? q_pos0 - window[li] + 1 : 0;
+      seen = (q_pos0 + n - 1) / vb - lo / vb + 1;
     }
-  short_mean /= kSamples * n_layers;
-  tiled_mean /= kSamples * n_layers;
+    short_mean += sum_s / (kSamples * n_layers);
+    tiled_mean += sum_t / (kSamples * n_layers);
+    for (int h = 0; h < hkv; ++h) {
+      const int c = (li * hkv + h) % classes;
+      load[c] += sum_s / kSamples * tiles * classes / kCus;
+      planes[c] += seen / 32.0;  // (a block is 32 KiB of K and V)
+    }
+  }
+  // Up to two rounds over the compute units, longest first: the one that gets the longest of the second round as well.
+  auto two_rounds = [&](double count, double from, double to) { return to + from + (to - from) * (1 - kCus / count); };
 
-  const double per_block = kv_dtype == kI8 ? 1.75 : 1.0;  // (64 keys instead of 32, and a conversion)
+  double planes_mean = 0;
+  for (int c = 0; c < classes; ++c) planes_mean += planes[c] / classes;
   double t_short;
   if (wgs <= kWideWorkgroups) {
-    t_short = 4.5 + 0.28 * per_block * short_most;
+    t_short = i8 ? 7.2 + 0.44 * short_most + 0.6 * planes_mean : 5.8 + 0.21 * short_most + 0.54 * planes_mean;
   } else {
-    const double longest = 0.36 * per_block * short_most, rate = 0.32 * per_block * short_mean * wgs / kCus + 2.7 * wgs / (2 * kCus);
-    t_short = 5.0 + (longest > rate ? longest : rate);
+    // The compute units of the busiest XCD, in blocks each, with what an L2 too small costs (nothing while all workgroups
+    // run at once: those of a unit then walk its blocks together) ...
+    double busiest = 0;
+    const double rounds = wgs / (2 * kCus), apart = fmin(1.0, fmax(0.0, rounds - 1));
+    for (int c = 0; c < classes; ++c) {
+      const double slow = fmin(i8 ? 0.8 : 3.0, fmax(0.0, (i8 ? 0.8 : 0.08) * (planes[c] - 4)));
+      busiest = fmax(busiest, load[c] * (1 + slow * apart));
+    }
+    // ... and in rounds of two workgroups a compute unit, longest first: what is left for the last one is a round all the same
+    const double full = floor(rounds), rest = wgs - full * 2 * kCus;
+    if (rounds <= 1) busiest = fmax(busiest, two_rounds(wgs, short_least, short_most));
+    else busiest = fmax(busiest, 2 * full * short_mean + (rest > kCus ? 2 : (rest > 0 ? (i8 ? 0.65 : 1.26) : 0)) * short_least);
+    t_short = (i8 ? 5.2 : 3.5) + fmax(0.28 * short_most, (i8 ? 0.42 : 0.22) * busiest) + (i8 ? 5.6 : 4.5) * rounds +
+              (i8 ? 0.3 : 0.85) * planes_mean;
   }
+
+  const int most = prefill_most_key_blocks(window, n_layers, q_pos0, n, tile_rows);
+  const PrefillParts split = choose_prefill_parts(items, most, n_layers, n, hq, kCus, true);
   double t_tiled;
-  int want = items * 4 >= 3 * kCus ? 1 : (int)((kCus + items - 1) / items);
-  if (want > 8) want = 8;
-  if (want > tiled_most / 4) want = (int)(tiled_most / 4);
-  if (want > 1) {  // keys split over work items, parts merged by a second launch (plan_prefill_split)
-    const double chunk = tiled_most / want;
-    const double part_bytes = tiled_mean / chunk * n_layers * n * hq * 1024;
-    t_tiled = 9.0 + 1.5 * chunk + 2 * part_bytes / 4.7e6;
+  if (split.parts > 1) {
+    const long slots = split.direct ? 2 * kCus : kCus;
+    const double walked = (double)((most + split.parts - 1) / split.parts) * ((items * split.parts + slots - 1) / slots);
+    const double part_bytes = (double)split.parts * tiled_mean / most * n_layers * n * hq * 1024;
+    t_tiled = (split.direct ? 7.9 + 1.4 * walked : 10.5 + 0.89 * walked) + 2.8 + 1.17 * 2 * part_bytes / 4.7e6;
   } else if (items < 2 * kCus) {
-    const double rounds = (double)(((long)items + kCus - 1) / kCus) * (4.0 + 1.6 * tiled_mean), longest = 4.0 + 1.6 * tiled_most;
-    t_tiled = 4.0 + (rounds > longest ? rounds : longest);
+    double walked = fmax(tiled_mean * items / kCus, tiled_most);
+    if (items > kCus) walked = fmax(walked, two_rounds(items, tiled_least, tiled_most));
+    t_tiled = 6.8 + 0.85 * walked + 6.8 * items / kCus;
   } else {
-    const double rate = 1.25 * tiled_mean * items / kCus, longest = 1.75 * tiled_most;
-    t_tiled = 7.0 + (rate > longest ? rate : longest);
+    t_tiled = 14.2 + fmax(1.1 * tiled_mean * items / kCus, 1.2 * tiled_most);
   }
-  if (kv_dtype == kI8) t_tiled += 5.5;  // the staging pass
-  return t_short * 1.15 < t_tiled;
+  // (the staging pass of an int8 cache: planes read and written as halves, queries in 16 bits)
+  if (i8) t_tiled += 3.0 + 0.14e-6 * 256 * ((double)units * 2 * (q_pos0 + n) * 3 + (double)n_layers * n * hq * 4);
+  // (16-bit caches: 5 % for the pass that rounds float32 queries, which the times above are without. An int8 cache in
+  // launches of up to two workgroups a compute unit: the tiled times come out some 5 % too long around the tie of 1,024
+  // rows behind 3,072, 60 / 62 us)
+  return t_short < (i8 ? (wgs > kWideWorkgroups && wgs <= 2 * kCus ? 0.95 : 1.0) : 1.05) * t_tiled;
 }
 
 hipError_t launch_prefill_short(const PrefillShortArgs& a, int kv_dtype, int io_dtype, hipStream_t stream, hipEvent_t ev0,
