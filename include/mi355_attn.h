@@ -34,14 +34,15 @@
  * the output is written in io_dtype from those sums.
  * An int8 cache enters the matrix cores as IEEE half values. Decode converts in
  * registers (K scales folded into the queries, V scales applied to the sums). A
- * prefill call of 16 rows or more first turns the planes it reads into half
+ * prefill call too short to fill the chip does the same on the kernel for short
+ * calls (option "prefill_short"). A longer one first turns the planes it reads into half
  * planes in a staging area of the handle (2 bytes per cache byte of the layers of
  * a pass, grown on demand up to "prefill_i8_stage_mib"; the call runs in passes
  * over as many layers as fit), V as half(value x scale), K as the values
  * themselves with the scales folded into float32 / bfloat16 queries on their way
  * to half, or as half(value x scale) under half queries, which are read as they
- * are; smaller calls, and calls that would have to allocate while the stream is
- * being captured, run row by row through the decode kernel.
+ * are; calls under 16 rows, and longer ones that would have to allocate while the
+ * stream is being captured, run row by row through the decode kernel.
  * A bfloat16 cache keeps its K planes in bfloat16 and its V planes as IEEE half
  * values, so that the probabilities multiply V with 11 significant bits on the
  * fp16 matrix-core path: a bfloat16 value v is stored without loss for
@@ -356,12 +357,14 @@ float mi355_attn_last_kernel_ms(mi355_attn* handle);
  *                      from the number of workgroups of the launch
  *   "rowwise_prefill"  0/1 run prefill row by row through the decode kernel
  *   "prefill_short"    the prefill kernel for short calls, one 16-column tile of
- *                      positions x query heads per workgroup: 1 always, 0 never, -1
- *                      (default): by rule, where none of the options below asks for
- *                      another kernel (an fp32 cache, which the tiled kernels do not
- *                      take: always)
+ *                      positions x query heads per workgroup: 1 always (but for calls
+ *                      over more than 64 layers or 65,535 rows and under option
+ *                      rowwise_prefill), 0 never, -1 (default): by rule, where none of
+ *                      the options below asks for another kernel (an fp32 cache, which
+ *                      the tiled kernels do not take: always). It needs no room beside
+ *                      the cache, int8 included
  *   "prefill_i8_min_rows" int8 cache: prefill calls of fewer rows run row by row
- *                      (default 16)
+ *                      (default 16) unless prefill_short is 1
  *   "prefill_i8_stage_mib" int8 cache: limit of the staging area for half planes,
  *                      MiB (default 2048; one layer's planes are staged even when
  *                      they exceed it)

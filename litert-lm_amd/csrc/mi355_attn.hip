@@ -455,8 +455,9 @@ PrefillSplit split_of(const PrefillArgs& a, int option, int cus = 0) {
 // no option asks for a particular one of the other kernels.
 bool short_prefill_takes(int n_layers, int n) { return n_layers <= kInlineLayers && n <= 65535; }
 bool takes_short_prefill(const mi355_attn* h, int layer_begin, int n_layers, int q_pos0, int n) {
-  if (!short_prefill_takes(n_layers, n) || h->prefill_short == 0) return false;
+  if (h->rowwise_prefill || !short_prefill_takes(n_layers, n) || h->prefill_short == 0) return false;
   if (h->prefill_short == 1) return true;
+  if (h->cfg.kv_dtype == MI355_ATTN_I8 && n < h->prefill_i8_min_rows) return false;
   if (h->prefill_rows16 >= 0 || h->prefill_key_split >= 0 || h->prefill_workgroups > 0) return false;
   return prefill_short_wanted(h->cfg.kv_dtype, h->cfg.num_q_heads, h->cfg.num_kv_heads, h->window.data() + layer_begin,
                               n_layers, q_pos0, n);
@@ -484,6 +485,29 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
   if (int rc = stage_in(h, 0, q, io_bytes, &dq, error_msg)) return rc;
   if (int rc = stage_out_begin(h, 1, out, io_bytes, &dout, error_msg)) return rc;
   hipEvent_t e0 = h->timing ? h->ev0 : nullptr, e1 = h->timing ? h->ev1 : nullptr;
+  // The short kernel first: it reads the planes as they are and needs no room, neither now nor while a graph is recorded.
+  if (takes_short_prefill(h, layer_begin, n_layers, q_pos0, n)) {
+    PrefillShortArgs a{};
+    a.q = dq;
+    a.out = dout;
+    a.cache = h->cache;
+    a.scales = h->scales;
+    a.geom = h->geom;
+    a.hq = h->cfg.num_q_heads;
+    a.group = h->cfg.num_q_heads / h->cfg.num_kv_heads;
+    a.layer_begin = layer_begin;
+    a.n_layers = n_layers;
+    a.seq = seq;
+    a.q_pos0 = q_pos0;
+    a.n = n;
+    a.rows_log2 = prefill_short_rows_log2(a.group);
+    a.scale = h->cfg.scale;
+    a.softcap = h->cfg.softcap;
+    for (int i = 0; i < n_layers; ++i) a.window[i] = h->window[layer_begin + i];
+    HIP_OR_RETURN(launch_prefill_short(a, h->cfg.kv_dtype, h->cfg.io_dtype, h->stream, e0, e1));
+    h->timed = h->timing;
+    return stage_out_end(h, 1, out, io_bytes, error_msg);
+  }
   bool rowwise = !prefill_supported(h->cfg.kv_dtype, h->cfg.io_dtype, h->cfg.head_dim) || h->rowwise_prefill;
   // An int8 cache goes to the matrix cores through half planes staged per call (prefill_attn.hip): from a tile's
   // worth of rows on, in passes of as many layers as the staging area's limit holds.
@@ -512,30 +536,6 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
         }
       }
     }
-  }
-  // (An int8 call that has to take the row-wise path - few rows, or recorded without a staging area - still does. A
-  // float32 cache has no tiled kernel; there `rowwise` stands for the option alone.)
-  if (!(i8 ? rowwise : h->rowwise_prefill) && takes_short_prefill(h, layer_begin, n_layers, q_pos0, n)) {
-    PrefillShortArgs a{};
-    a.q = dq;
-    a.out = dout;
-    a.cache = h->cache;
-    a.scales = h->scales;
-    a.geom = h->geom;
-    a.hq = h->cfg.num_q_heads;
-    a.group = h->cfg.num_q_heads / h->cfg.num_kv_heads;
-    a.layer_begin = layer_begin;
-    a.n_layers = n_layers;
-    a.seq = seq;
-    a.q_pos0 = q_pos0;
-    a.n = n;
-    a.rows_log2 = prefill_short_rows_log2(a.group);
-    a.scale = h->cfg.scale;
-    a.softcap = h->cfg.softcap;
-    for (int i = 0; i < n_layers; ++i) a.window[i] = h->window[layer_begin + i];
-    HIP_OR_RETURN(launch_prefill_short(a, h->cfg.kv_dtype, h->cfg.io_dtype, h->stream, e0, e1));
-    h->timed = h->timing;
-    return stage_out_end(h, 1, out, io_bytes, error_msg);
   }
   const size_t layer_io_bytes = (size_t)n * h->cfg.num_q_heads * h->cfg.head_dim * io_size(h);
   for (int l0 = 0; !rowwise && l0 < n_layers; l0 += layers_per_pass) {

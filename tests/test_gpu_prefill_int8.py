@@ -205,6 +205,7 @@ def test_recorded_into_a_graph_without_room_it_takes_the_rowwise_path():
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
         with A.Attn(1, hq, hkv, D, L, 1, A.I8, A.F16, stream=side.cuda_stream) as at:
+            at.set_option("prefill_short", 0)  # (the kernel for short calls needs no room: the test below)
             kr, vr = fill_int8(at, 0, 0, gen(131, L, hkv, D), gen(132, L, hkv, D))
             qd, qr = queries(gen(133, n, hq, D), A.F16)
             out = torch.zeros_like(qd)
@@ -220,6 +221,37 @@ def test_recorded_into_a_graph_without_room_it_takes_the_rowwise_path():
                 assert plain_err(out.float().cpu().numpy(), ref) < TOL
             eager = prefill(at, 0, 0, 0, qd, rowwise=True)
             assert torch.equal(out, eager)
+            del g
+
+
+def test_short_calls_need_no_staging_area():
+    # a call that the kernel for short calls takes reads the int8 planes as they are: recorded into a graph by a handle
+    # that has staged nothing it is the same launch as run eagerly, and it allocates nothing (4 KV heads x 2 planes x
+    # 4,096 rows of halves would be 16 MiB)
+    L, hq, hkv, n = 4096, 8, 4, 121
+    assert A.prefill_route(A.I8, hq, hkv, [0], L - n, n)[0] == A.ROUTE_SHORT
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        with A.Attn(1, hq, hkv, D, L, 1, A.I8, A.F16, stream=side.cuda_stream) as at:
+            kr, vr = fill_int8(at, 0, 0, gen(135, L, hkv, D), gen(136, L, hkv, D))
+            qd, qr = queries(gen(137, n, hq, D), A.F16)
+            out, eager = torch.zeros_like(qd), torch.zeros_like(qd)
+            side.synchronize()
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=side):
+                at.prefill(0, 0, L - n, n, qd, out)
+            side.synchronize()
+            free = torch.cuda.mem_get_info()[0]
+            at.prefill(0, 0, L - n, n, qd, eager)
+            side.synchronize()
+            assert free - torch.cuda.mem_get_info()[0] < 8 << 20
+            ref = c_oracle.sdpa_f64(qr, kr, vr, D ** -0.5, q_pos0=L - n, kv_len=L)
+            assert plain_err(eager.float().cpu().numpy(), ref) < TOL
+            for _ in range(3):
+                out.zero_()
+                g.replay()
+                side.synchronize()
+                assert torch.equal(out, eager)
             del g
 
 
