@@ -452,13 +452,15 @@ PrefillSplit split_of(const PrefillArgs& a, int option, int cus = 0) {
 }
 
 // Whether a prefill call runs on the kernel for short calls (prefill_short.hip): option prefill_short, or by rule where
-// no option asks for a particular one of the other kernels.
+// no option asks for a particular one of the other kernels (a float32 cache has no other but the row-wise path, so the
+// options that choose among the tiled kernels say nothing there).
 bool short_prefill_takes(int n_layers, int n) { return n_layers <= kInlineLayers && n <= 65535; }
 bool takes_short_prefill(const mi355_attn* h, int layer_begin, int n_layers, int q_pos0, int n) {
   if (h->rowwise_prefill || !short_prefill_takes(n_layers, n) || h->prefill_short == 0) return false;
   if (h->prefill_short == 1) return true;
   if (h->cfg.kv_dtype == MI355_ATTN_I8 && n < h->prefill_i8_min_rows) return false;
-  if (h->prefill_rows16 >= 0 || h->prefill_key_split >= 0 || h->prefill_workgroups > 0) return false;
+  if (h->cfg.kv_dtype != MI355_ATTN_F32 && (h->prefill_rows16 >= 0 || h->prefill_key_split >= 0 || h->prefill_workgroups > 0))
+    return false;
   return prefill_short_wanted(h->cfg.kv_dtype, h->cfg.num_q_heads, h->cfg.num_kv_heads, h->window.data() + layer_begin,
                               n_layers, q_pos0, n);
 }
