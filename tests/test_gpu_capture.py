@@ -40,6 +40,9 @@ def test_prefill_shapes_first_seen_under_capture_and_more_captured_shapes_than_p
         with A.Attn(layers, hq, hkv, D, 1024, 1, A.F16, A.F16, layer_window=windows, stream=side.cuda_stream) as at:
             for layer in range(layers):
                 at.kv_append(layer, 0, 0, rnd(10 + layer, 1024, hkv, D), rnd(40 + layer, 1024, hkv, D))
+            # (calls of this size run on the short kernel or without a plan by rule)
+            at.set_option("prefill_short", 0)
+            at.set_option("prefill_rows16", 1)
             q = rnd(5, layers, n, hq, D)
             graphs = []
             # six chunk positions = six launch shapes: the first is new under capture, the others are run eagerly
@@ -65,6 +68,9 @@ def test_prefill_shapes_first_seen_under_capture_and_more_captured_shapes_than_p
                     assert torch.isfinite(out.float()).all(), pos0
                     err = float((out.float() - eager.float()).abs().max() / eager.float().abs().max())
                     assert err < 2e-3, (pos0, rep, err)
+                    # the first was captured without a plan and run eagerly with one: other kernels, other bits; the next
+                    # four are the same launch, and so is the last, which finds no free slot either way
+                    assert torch.equal(out, eager) == (pos0 > 0), (pos0, rep)
             # a new shape, eagerly, with every slot held by a graph
             eager = torch.full_like(q, float("nan"))
             at.prefill(0, 0, 448, n, q, eager, n_layers=layers)

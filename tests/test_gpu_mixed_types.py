@@ -249,17 +249,19 @@ def test_int8_cache_with_each_activation_type(io):
                 else:
                     err = orc.rel_err(got[b], ref)
                 assert err < TOL16, (io, ns, b, err)
-        # a prefill chunk over the int8 cache in this activation type
+        # a prefill chunk over the int8 cache in this activation type, on the kernel for short calls and staged
         n = 130
         qd, qr = rounded(gen(19, n, 8, D), io)
-        out = torch.empty_like(qd)
-        at.prefill(0, 0, 1000 - n, n, qd, out)
-        torch.cuda.synchronize()
         ref = c_oracle.sdpa_f64(qr, kvs[0][0], kvs[0][1], D ** -0.5, q_pos0=1000 - n, kv_len=1000)
-        got = out.float().cpu().numpy()
-        err = orc.rel_err_beyond_bf16_rounding(got, ref) if io == A.BF16 else orc.rel_err(got, ref)
-        say(f"int8 cache, activations {io}: prefill rel_err {err:.3e}")
-        assert err < TOL16
+        for short in (1, 0):
+            at.set_option("prefill_short", short)
+            out = torch.full_like(qd, float("nan"))
+            at.prefill(0, 0, 1000 - n, n, qd, out)
+            torch.cuda.synchronize()
+            got = out.float().cpu().numpy()
+            err = orc.rel_err_beyond_bf16_rounding(got, ref) if io == A.BF16 else orc.rel_err(got, ref)
+            say(f"int8 cache, activations {io}: prefill rel_err {err:.3e}")
+            assert err < TOL16
 
 
 # ------------------------------------------------------------------ the fused decode step with mixed types

@@ -567,6 +567,7 @@ def test_prefill_key_split_by_rule_softcap_and_limits():
     # by rule (the default): one 1024-token global layer of config 2 has 32 tiles for 256 compute units
     seed = orc.SEED_BASE + 1
     with make(1, 4, 1, 1024, 1, A.BF16, layer_window=[0]) as at:
+        at.set_option("prefill_short", 0)  # (by rule the kernel for short calls would take it)
         q = gen(seed + 1, 1024, 4, D)
         kr, vr = fill_seq(at, A.BF16, 0, 0, gen(seed + 11, 1024, 1, D), gen(seed + 21, 1024, 1, D))
         err, split = run_prefill(at, A.BF16, q, kr, vr, 0, 0)
@@ -650,6 +651,7 @@ def test_prefill_more_units_than_the_order_table_holds():
     nl, n, hq, hkv, dt = 40, 70, 8, 4, A.F16
     windows = [0 if l % 3 == 0 else 20 + l for l in range(nl)]
     with make(nl, hq, hkv, n, 1, dt, layer_window=windows) as at:
+        at.set_option("prefill_short", 0)
         qd, qr = dev(gen(111, nl, n, hq, D), dt)
         kd, kr = dev(gen(112, n, hkv, D), dt)
         vd, vr = dev(gen(113, n, hkv, D), dt)
@@ -672,7 +674,7 @@ def test_prefill_rowwise_fp32_and_int8():
     L = 200
     with make(1, 4, 1, 256, 1, A.F32, layer_window=[50]) as at:
         kr, vr = fill_seq(at, A.F32, 0, 0, gen(81, L, 1, D), gen(82, L, 1, D))
-        err, _ = run_prefill(at, A.F32, gen(83, 150, 4, D), kr, vr, 50, 50)
+        err, _ = run_prefill(at, A.F32, gen(83, 150, 4, D), kr, vr, 50, 50, rowwise=True)
         say(f"prefill fp32 rowwise: rel_err={err:.3e}")
         assert err < TOL[A.F32]
     with make(1, 8, 2, 256, 1, A.I8) as at:
@@ -682,7 +684,7 @@ def test_prefill_rowwise_fp32_and_int8():
         at.kv_append(0, 0, 0, torch.from_numpy(kq).to(DEV), torch.from_numpy(vq).to(DEV))
         at.kv_set_scales(0, 0, torch.from_numpy(ks).to(DEV), torch.from_numpy(vs).to(DEV))
         err, _ = run_prefill(at, A.F16, gen(86, L, 8, D), orc.dequantize_kv_int8(kq, ks),
-                             orc.dequantize_kv_int8(vq, vs), 0, 0)
+                             orc.dequantize_kv_int8(vq, vs), 0, 0, rowwise=True)
         say(f"prefill int8 rowwise: rel_err={err:.3e}")
         assert err < TOL[A.I8]
 

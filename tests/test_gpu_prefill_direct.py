@@ -1,6 +1,6 @@
-"""Prefill launches of few, long tiles: the keys of a tile are cut into parts of equal length and, where the measured
-times say so, run as a direct launch (a workgroup per item on 16x16x32 MFMAs, no work plan). Checked against the float64
-oracle where it can go wrong: tiles whose block counts leave parts empty or a block shorter than the others, ragged
+"""Prefill launches of few, long tiles: the keys of a tile are cut into as few parts as do, of the same length but for
+the last, and, where the measured times say so, run as a direct launch (a workgroup per item on 16x16x32 MFMAs, no work
+plan). Checked against the float64 oracle where it can go wrong: tiles whose block counts leave parts empty or a block shorter than the others, ragged
 ends, windows on some layers only (their tiles have fewer parts than the launch has room for), more parts than the
 merge asks for at once, float32 output, and an int8 cache through its staged planes.
 
@@ -39,13 +39,17 @@ def half(x):
 @pytest.mark.parametrize("kv", [A.F16, A.I8])
 @pytest.mark.parametrize("io", [A.F16, A.F32])
 @pytest.mark.parametrize("hq,hkv,start,n,windows,key_split", [
-    (8, 2, 4000, 2047, [0], -1),       # 128 items, four parts each: the direct launch, by rule
-    (8, 2, 3990, 1999, [0, 900], -1),  # two layers, one of them windowed
-    (6, 2, 5001, 1500, [0], -1),       # three heads a KV head: 128 positions a tile
+    (8, 2, 4000, 2047, [0], -1),          # 128 items, four parts each: the direct launch, by rule
+    (8, 2, 3990, 1400, [0, 900], -1),     # two layers, two parts; the windowed tiles are whole, their second part is empty
+    (8, 2, 6000, 1000, [0, 2500], -1),    # four parts; the windowed tiles have two of them
+    (6, 2, 5001, 1500, [0], -1),          # three heads a KV head: 128 positions a tile
     (4, 1, 1000, 333, [0, 200], 3),    # up to 14 parts: more than the merge asks for at once
 ])
 def test_split_tiles_against_the_oracle(kv, io, hq, hkv, start, n, windows, key_split):
     L, nl = start + n, len(windows)
+    if key_split < 0:
+        route, parts = A.prefill_route(kv, hq, hkv, windows, start, n)
+        assert route == A.ROUTE_DIRECT16 and parts > 1
     with A.Attn(nl, hq, hkv, D, L, 1, kv, io, layer_window=windows, stream=torch.cuda.current_stream().cuda_stream) as at:
         at.set_option("prefill_short", 0)
         at.set_option("prefill_key_split", key_split)
