@@ -633,9 +633,9 @@ def main():
                           "frac_of_mfma_peak": round(pre["flops"] / pre["sustained_sec_per_step"] / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4)},
             "single_global_layer_ms": round(pre["single_global_layer_ms"], 4),
             "layer_by_layer": None if args.no_pipeline else {
-                "what": "the same 26 layers as 26 launches in turn (how an executor calls it); key ranges of a "
-                        "launch this small are cut into parts that a second kernel merges (option "
-                        "prefill_key_split, default by rule), *_unsplit: with that switched off",
+                "what": "the same 26 layers as 26 launches in turn (how an executor calls it), on the kernel for short "
+                        "calls by rule (option prefill_short); *_unsplit: on the tiled kernel, its key ranges "
+                        "uncut (option prefill_key_split = 0)",
                 "ms": round(pre["layer_by_layer_ms"], 4), "TFLOPs": round(pre["flops"] / pre["layer_by_layer_ms"] / 1e9, 2),
                 "unsplit_ms": round(pre["layer_by_layer_unsplit_ms"], 4),
                 "single_global_layer_unsplit_ms": round(pre["single_global_layer_unsplit_ms"], 4)},

@@ -165,7 +165,7 @@ struct PrefillArgs {
   const int32_t* host_window;  // host copy of layer_window (for the ordering), may be null
   int32_t use_order;
   // Key split (launches with fewer work items than compute units): a work item covers at most kchunk
-  // key blocks of its tile, tiles with more blocks are cut into up to smax items of equal length whose unnormalised
+  // key blocks of its tile, tiles with more blocks are cut into up to smax items (tile_chunk) whose unnormalised
   // fp32 accumulators and (max, sum) pairs go to ws_acc / ws_ml, [layer][row][head][smax] x head_dim
   // and x 2 floats, and prefill_merge_kernel combines them. kchunk == 0: off.
   int32_t kchunk, smax;

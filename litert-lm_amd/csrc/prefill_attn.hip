@@ -66,9 +66,10 @@ struct El<kBF16> {
   static __device__ __forceinline__ f16v mfma(vec8 a, vec8 b, f16v c) { return mfma32_bf16(a, b, c); }
 };
 
-// Key blocks of one work item of a tile of nblk blocks, cut into as few parts of at most kchunk blocks as do, all of the
-// same length to a block (cut every kchunk blocks, the last part of a tile could be a single block, which costs an item
-// and a part of the merge like any other).
+// Key blocks of one work item of a tile of nblk blocks, cut into as few parts of at most kchunk blocks as do: the mean
+// length, rounded up, the last part what is left. Of a long tile the parts differ by a few blocks then (cut every kchunk
+// blocks, the last one could be a single block, which costs an item and a part of the merge like any other); of a short
+// one the last can still be small (13 blocks at kchunk 4: 4, 4, 4, 1).
 MI355_HD int tile_chunk(int nblk, int kchunk) {
   const int parts = (nblk + kchunk - 1) / kchunk;
   return (nblk + parts - 1) / parts;

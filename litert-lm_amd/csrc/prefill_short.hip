@@ -44,8 +44,9 @@ constexpr int lds_bytes() {
   return query_steps<KV, D>() * 1024 + NW * kCols * (D + kAccStride) * 4 + NW * kCols * 8;
 }
 
-// NW waves per workgroup; either way eight waves a compute unit, two per SIMD, which is all that 256 registers per
-// lane leave room for.
+// NW waves per workgroup, eight waves a compute unit either way, two per SIMD, which is all that 256 registers per lane
+// leave room for; but for a float32 cache in launches of four waves, whose 81.5 KiB of LDS let one workgroup run on a
+// compute unit instead of two.
 template <int KV, int IO, int D, int NW, bool CAP>
 __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const PrefillShortArgs a) {
   using io_t = typename IoT<IO>::type;
