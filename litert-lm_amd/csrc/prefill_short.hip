@@ -19,6 +19,8 @@
 #include <hip/hip_ext.h>
 #include <math.h>
 
+#include <algorithm>
+
 #include "attn_params.h"
 #include "kernels.h"
 #include "kv_blocks.h"
@@ -253,25 +255,25 @@ int prefill_short_rows_log2(int group) {
 }
 
 // Whether the short kernel is expected to finish a call before the tiled kernels of prefill_attn.hip: both sides by
-// formulas fitted to measured times (head_dim 256, MI355X, calls queued back to back, 770 shapes spread at random over
+// formulas fitted to measured times (head_dim 256, MI355X, calls queued back to back, 1,140 shapes spread at random over
 // 16 to 4,096 rows behind 0 to 12,000 cached ones, 1 to 34 layers with and without windows, sixteen head counts). Nine
 // tenths of the times are within 15 % of the formulas, and what they choose takes 0.3 % longer than the better side in
-// the mean (on 600 other shapes 1.5 %, most of it the spread between two runs). Examples, tiled / short, us: bfloat16, 4
-// query heads on 1 KV head, one layer of 64 rows 9.9 / 5.1, 256 rows 15.9 / 8.0, 1,024 rows 25.7 / 13.6, 1,370
-// rows behind 1,338 35 / 38, 17 behind 1,207 19 / 14, 26 layers of 256 rows 20 / 28; 8 heads on 2, 2 layers of 1,768
-// behind 693 83 / 96. int8 cache, 300 rows 24 / 10, 256 rows behind 3,072 47 / 31. A float32 cache always takes the short
-// kernel: the alternative is one decode item per row, which reads every key once per position instead of once per 16
-// columns (300 rows 36 / 17, 300 behind 2,000 305 / 81).
+// the mean (on 320 other shapes 0.4 %, five of them by 10 to 15 %). Examples, tiled / short, us: bfloat16, 4 query heads on 1 KV head, one layer of 64 rows 9.9 / 5.1, 256 rows
+// 15.9 / 8.0, 1,024 rows 25.7 / 13.6, 1,370 rows behind 1,338 35 / 38, 17 behind 1,207 19 / 14, 26 layers of 256 rows
+// 20 / 28; 8 heads on 2, 2 layers of 1,768 behind 693 83 / 96. int8 cache, 300 rows 24 / 10, 256 rows behind 3,072
+// 47 / 31. A float32 cache always takes the short kernel: the alternative is one decode item per row, which reads every
+// key once per position instead of once per 16 columns (300 rows 36 / 17, 300 behind 2,000 305 / 81).
 //
-// What decides for the short kernel beside the key blocks themselves is what one XCD has to do. Units (layer x KV head)
-// vary fastest over the workgroups, which go round the eight XCDs, so with a number of units that shares a factor f with 8
-// a unit's tiles all go to 8 / f of them: with 8 units the only global layer among windowed ones is the work of a single
-// XCD (8 layers of 1,686 rows behind 1,059, window 512: 204 us, tiled 92), and units whose planes do not fit its L2
-// (4 MiB) together are read from behind it again and again.
+// What decides for the short kernel beside the key blocks themselves is where its workgroups run. They go round the eight
+// XCDs and, within each, round its four engines of eight compute units, with the units (layer x KV head) varying fastest:
+// if the number of units shares a factor f with 32, all tiles of a unit are the work of 32 / f engines. With 8 units the
+// only global layer among windowed ones has a single XCD (8 layers of 1,686 rows behind 1,059, window 512: 204 us, tiled
+// 92), with 32 a single engine (16 layers of 108 rows behind 3,058, window 1,024: 103 us, tiled 63). And units whose
+// planes do not fit an XCD's L2 (4 MiB) together are read from behind it again and again.
 //
 // The activation type is not part of the rule, so that calls that differ in nothing else run the same arithmetic.
 bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, int n_layers, int q_pos0, int n) {
-  constexpr int kCus = 256, kXcds = 8;  // what the times were measured on
+  constexpr int kCus = 256, kXcds = 8, kEngines = 32;  // what the times were measured on
   if (kv_dtype == kF32) return true;
   const bool i8 = kv_dtype == kI8;
   const int group = hq / hkv, rows_log2 = prefill_short_rows_log2(group);
@@ -282,7 +284,8 @@ bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, 
   const int hpb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
   const int tile_rows = prefill_tile_rows(group);
   const long items = (long)n_layers * hkv * (group / hpb) * ((n + tile_rows - 1) / tile_rows);
-  const int classes = units % 8 == 0 ? 8 : (units % 4 == 0 ? 4 : (units % 2 == 0 ? 2 : 1));  // of units that share XCDs
+  const int classes = std::min(units & -units, kEngines);  // of units that share engines
+  const int xcd_classes = std::min(classes, kXcds);
   // key blocks of a stretch of `rows` positions: mean over the call (the count is linear in the position but for the
   // corner at the window, so a few samples do) and most
   auto blocks = [&](int w, int first, int rows, int block) {
@@ -292,11 +295,14 @@ bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, 
   };
   constexpr int kSamples = 9;
   double short_mean = 0, short_most = 0, short_least = 1e9, tiled_mean = 0, tiled_most = 0, tiled_least = 1e9;
-  double load[kXcds] = {}, planes[kXcds] = {};  // of a class: key blocks per compute unit, MiB of K and V that it sees
+  double load[kEngines] = {};  // of a class: key blocks per compute unit
+  double planes[kXcds] = {};   // MiB of K and V that an XCD sees
   double sum_s = 0, sum_t = 0;                  // of the layer (kept from the layer before where the window is the same)
   int seen = 0;
+  bool mixed = false;  // layers with different windows
   for (int li = 0; li < n_layers; ++li) {
     if (li == 0 || window[li] != window[li - 1]) {
+      mixed = li > 0;
       sum_s = sum_t = 0;
       for (int k = 0; k < kSamples; ++k) {
         const int at = q_pos0 + (int)((int64_t)(n - 1) * k / (kSamples - 1));
@@ -317,32 +323,34 @@ bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, 
     for (int h = 0; h < hkv; ++h) {
       const int c = (li * hkv + h) % classes;
       load[c] += sum_s / kSamples * tiles * classes / kCus;
-      planes[c] += seen / 32.0;  // (a block is 32 KiB of K and V)
+      planes[c % xcd_classes] += seen / 32.0;  // (a block is 32 KiB of K and V)
     }
   }
   // Up to two rounds over the compute units, longest first: the one that gets the longest of the second round as well.
   auto two_rounds = [&](double count, double from, double to) { return to + from + (to - from) * (1 - kCus / count); };
 
   double planes_mean = 0;
-  for (int c = 0; c < classes; ++c) planes_mean += planes[c] / classes;
+  for (int c = 0; c < xcd_classes; ++c) planes_mean += planes[c] / xcd_classes;
   double t_short;
   if (wgs <= kWideWorkgroups) {
     t_short = i8 ? 7.2 + 0.44 * short_most + 0.6 * planes_mean : 5.8 + 0.21 * short_most + 0.54 * planes_mean;
   } else {
-    // The compute units of the busiest XCD, in blocks each, with what an L2 too small costs (nothing while all workgroups
-    // run at once: those of a unit then walk its blocks together) ...
+    // The compute units of the busiest engine, in blocks each, with what an L2 too small costs (the workgroups of a unit
+    // walk its blocks together while all run at once, and less and less so in more rounds or beside shorter layers) ...
     double busiest = 0;
-    const double rounds = wgs / (2 * kCus), apart = fmin(1.0, fmax(0.0, rounds - 1));
+    const double rounds = wgs / (2 * kCus), apart = fmin(1.0, fmax(0.0, (rounds - 1) / (i8 ? 2.2 : 1.3)));
     for (int c = 0; c < classes; ++c) {
-      const double slow = fmin(i8 ? 0.8 : 3.0, fmax(0.0, (i8 ? 0.8 : 0.08) * (planes[c] - 4)));
-      busiest = fmax(busiest, load[c] * (1 + slow * apart));
+      const double over = fmax(0.0, planes[c % xcd_classes] - 4);
+      const double slow = mixed ? fmin(i8 ? 1.07 : 1.57, (i8 ? 0.16 : 0.117) * over)
+                                : apart * fmin(i8 ? 0.9 : 3.0, (i8 ? 0.027 : 0.064) * over);
+      busiest = fmax(busiest, load[c] * (1 + slow));
     }
     // ... and in rounds of two workgroups a compute unit, longest first: what is left for the last one is a round all the same
     const double full = floor(rounds), rest = wgs - full * 2 * kCus;
     if (rounds <= 1) busiest = fmax(busiest, two_rounds(wgs, short_least, short_most));
     else busiest = fmax(busiest, 2 * full * short_mean + (rest > kCus ? 2 : (rest > 0 ? (i8 ? 0.65 : 1.26) : 0)) * short_least);
-    t_short = (i8 ? 5.2 : 3.5) + fmax(0.28 * short_most, (i8 ? 0.42 : 0.22) * busiest) + (i8 ? 5.6 : 4.5) * rounds +
-              (i8 ? 0.3 : 0.85) * planes_mean;
+    t_short = (i8 ? 4.7 : 3.6) + fmax((i8 ? 0.45 : 0.28) * short_most, (i8 ? 0.42 : 0.212) * busiest) +
+              (i8 ? 5.6 : 4.4) * rounds + (i8 ? 0.65 : 0.95) * planes_mean;
   }
 
   const int most = prefill_most_key_blocks(window, n_layers, q_pos0, n, tile_rows);

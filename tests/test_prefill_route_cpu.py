@@ -24,6 +24,9 @@ MEASURED = [
     (A.BF16, 4, 1, 8, 512, 1059, 1686, 92.0, 203.6),
     (A.F16, 16, 2, 8, 512, 4227, 265, 172.0, 298.6),
     (A.F16, 4, 1, 8, 512, 1556, 639, 61.4, 79.4),
+    # ... or one engine of an XCD (a factor of 32)
+    (A.BF16, 8, 2, 16, 1024, 3058, 108, 62.8, 102.6),
+    (A.F16, 8, 4, 12, 512, 4822, 107, 67.8, 100.3),
     # more planes than an L2 holds, walked by few tiles each
     (A.F16, 2, 2, 26, 512, 79, 589, 33.6, 49.8),
     (A.BF16, 16, 2, 26, 0, 2068, 16, 51.1, 70.3),
