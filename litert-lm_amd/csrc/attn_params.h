@@ -84,7 +84,10 @@ MI355_HD int64_t v_elem_offset(int t, int d, int head_dim, int esize) {
          (int64_t)slot * esize;
 }
 
-// Arguments of the decode kernels (passed by value).
+// Arguments of the decode kernels, passed by value in blocks. A launch costs the host 2.3 us with 32 bytes of arguments, 2.9
+// with 256 and 3.5 to 4.1 from 384 to 1,600, and every compute unit fetches them before it can start, so a launch carries
+// what it needs: DecodeWork for as many sequences and layers as it has, DecodePre for the fused step, DecodeTables only where
+// sequences or windows do not fit a DecodeWork.
 struct DecodeArgs {
   const void* q;             // [n_layers][batch][hq][D] io dtype
   void* out;                 // same shape
@@ -92,53 +95,100 @@ struct DecodeArgs {
   const float* scales;       // int8 cache only
   float* ws_acc;             // [items][hq][num_splits][D] partial accumulators
   float* ws_ml;              // [items][hq][num_splits][2] partial (max, sum)
-  const int32_t* kv_lens;    // [batch] in dispatch order (unused when inline_items != 0)
-  const int32_t* seq_ids;    // [batch] or nullptr
-  const int32_t* rows;       // [batch] row in q / out of dispatch slot j (batches beyond kInlineItems), or nullptr
-  int32_t inline_items;      // != 0: batch <= kInlineItems and lens / sequence ids travel in the argument block,
-                             // in dispatch order (longest sequence first): entry j belongs to batch row inline_row[j]
-  int32_t inline_lens[kInlineItems];
-  int32_t inline_seq[kInlineItems];
-  int32_t inline_row[kInlineItems];
-  const int32_t* layer_window;  // [num_layers] (read only when n_layers > kInlineLayers)
-  int32_t inline_window[kInlineLayers];  // windows of layers layer_begin .. layer_begin + n_layers - 1
-  CacheGeom geom;
+  uint32_t* tickets;         // [items][hkv] visible keys whose partials are written, all zero between launches; nullptr:
+                             // the partials are merged by a launch of their own
+  int64_t plane_bytes;       // as in CacheGeom
+  int32_t hkv, max_seqs;
   int32_t hq, group;
-  int32_t layer_begin, n_layers, batch;
+  int32_t layer_begin, batch;
+  uint32_t hkv_inverse;      // 2^32 / hkv, rounded up; 0 for one KV head
   int32_t num_splits;
-  int32_t max_kv_len;        // max over kv_lens (host computed), sizes the partitions
-  int32_t min_kv_len;        // min over kv_lens (host computed; only the launch rules look at it)
-  int32_t rule_batch;        // sequences the launch rules count: batch, or those of the larger batch this launch is a part of
+  int32_t align;             // partitions start at, and hold, multiples of this many tokens (a power of two, whole blocks)
   float scale;               // softmax scale
   float softcap;
-  // The step before attention, run by the decode kernel itself for the one new token of every sequence
-  // (one layer, inline_items != 0): raw projections [batch][hq][D] / [batch][hkv][D] in the io dtype; the
-  // token's row is kv_len - 1. q is then unused. pre_q == nullptr: off. Flags and constants as in
-  // PreAttentionArgs.
-  const void* pre_q;
-  const void* pre_k;
-  const void* pre_v;
-  const float* pre_constants;
-  int32_t pre_rope, pre_norm_q, pre_norm_k, pre_norm_v, pre_q_scaled, pre_k_scaled;
-  float pre_eps, pre_weight_offset;
 };
+
+// A sequence of a launch: its cache slot, its length (below 2^23: a plane is under 2 GiB) and, above it, its row in q and
+// out (below kInlineItems). Sequences stand in dispatch order (longest first).
+struct DecodeItem { uint32_t row_len; int32_t seq; };
+constexpr int kDecodeLenBits = 24;
+constexpr int kFewItems = 8;  // launches of up to this many sequences carry so many
+// Windows of the launch's layers and their decode_partition_tokens: 2 bits a layer say which of up to four pairs.
+constexpr int kDecodeWindows = 4;
+template <int LAYERS>
+struct DecodeLayers {
+  uint32_t code[LAYERS / 16];
+  int32_t window[kDecodeWindows], per[kDecodeWindows];
+};
+template <>
+struct DecodeLayers<1> { int32_t window[1], per[1]; };
+template <int ITEMS, int LAYERS>
+struct DecodeWork {
+  DecodeLayers<LAYERS> layers;
+  DecodeItem item[ITEMS];
+};
+
+// Where a launch finds what does not fit a DecodeWork (of kInlineItems, kInlineLayers).
+struct DecodeTables {
+  const int32_t* layer_window;  // [num_layers], or nullptr: the DecodeWork has the windows
+  const int32_t* kv_lens;    // [batch] in dispatch order, or nullptr: the DecodeWork has the sequences
+  const int32_t* seq_ids;    // [batch] or nullptr
+  const int32_t* rows;       // [batch] row in q / out of dispatch slot j, or nullptr
+  int32_t max_kv_len;        // sizes the partitions
+};
+
+// The step before attention, run by the decode kernel itself for the one new token of every sequence (one layer, no
+// tables): raw projections [batch][hq][D] / [batch][hkv][D] in the io dtype; the token's row is kv_len - 1. DecodeArgs::q is
+// then unused. Flags and constants as in PreAttentionArgs.
+struct DecodePre {
+  const void* q;
+  const void* k;
+  const void* v;
+  const float* constants;
+  int32_t rope, norm_q, norm_k, norm_v, q_scaled, k_scaled;
+  float eps, weight_offset;
+};
+
+// What a launch is made from on the host.
+struct DecodeLaunch {
+  DecodeArgs args{};
+  DecodePre pre{};
+  bool fused = false;        // pre is filled in
+  DecodeWork<kInlineItems, kInlineLayers> work{};
+  DecodeTables tables{};
+  bool inline_items = false, inline_layers = false;  // work has the sequences / the windows
+  int32_t n_layers = 1;
+  int32_t esize = 0;         // of a cache element
+  int32_t max_kv_len = 0;    // max over kv_lens, sizes the partitions
+  int32_t min_kv_len = 0;    // min over kv_lens
+  int32_t widest_window = 0; // of the launch's layers, 0: a layer without one
+  int32_t rule_batch = 0;    // sequences the launch rules count: batch, or those of the larger batch this launch is a part of
+};
+// Launches of up to one workgroup a compute unit are bound by latency: they have waves for the rows of the fused step and
+// for the merge, and the workgroup that writes the last partial of a row merges it.
+constexpr int kLatencyWorkgroups = 256;
+constexpr int kDecodeTickets = kLatencyWorkgroups;  // entries of DecodeArgs::tickets
+inline bool decode_merges_itself(int n_layers, int rule_batch, int hkv, int num_splits) {
+  return num_splits > 1 && num_splits <= 64 && (int64_t)n_layers * rule_batch * hkv * num_splits <= kLatencyWorkgroups;
+}
 
 // Tokens per split-KV partition for a layer with the given window: the same
 // formula runs in the attention kernel and in the merge kernel.
-MI355_HD int decode_partition_tokens(int max_kv_len, int window, int num_splits) {
-  int span = max_kv_len;
-  if (window > 0 && window + (kTokenAlign - 1) < span) span = window + (kTokenAlign - 1);
-  int per = (span + num_splits - 1) / num_splits;
-  per = (per + kTokenAlign - 1) / kTokenAlign * kTokenAlign;
-  return per < kTokenAlign ? kTokenAlign : per;
+MI355_HD int decode_span(int max_kv_len, int window, int align) {
+  return window > 0 && window + (align - 1) < max_kv_len ? window + (align - 1) : max_kv_len;
 }
+MI355_HD int decode_partition_tokens(int max_kv_len, int window, int num_splits, int align) {
+  const int per = (decode_span(max_kv_len, window, align) + num_splits - 1) / num_splits;
+  return (per + align - 1) / align * align;
+}
+MI355_HD int decode_block_tokens(int esize) { return 64 / esize; }  // KvT::VB: what a wave loads at a time
 
-// First visible key and the 64-aligned row at which partition 0 starts.
-MI355_HD void decode_visible_range(int kv_len, int window, int* vlo, int* start) {
+// First visible key and the aligned row at which partition 0 starts.
+MI355_HD void decode_visible_range(int kv_len, int window, int align, int* vlo, int* start) {
   int lo = 0;
   if (window > 0 && kv_len > window) lo = kv_len - window;
   *vlo = lo;
-  *start = lo & ~(kTokenAlign - 1);
+  *start = lo & ~(align - 1);
 }
 
 struct PrefillArgs {

@@ -1,6 +1,6 @@
 // One-token decode attention over the KV cache (gfx950, wave64, MFMA).
 //
-// Grid: x = split-KV partition, y = KV head, z = (layer, sequence) item.
+// Grid: x = layer, y = sequence, z = split-KV partition x KV head.
 // A workgroup of NW waves streams the K and V rows of its partition exactly
 // once. Each wave owns every NW-th block of VB tokens and, per block, issues
 // 32 wave-wide 1 KiB streaming loads (16 of K, 16 of V at head_dim 256); the
@@ -10,14 +10,18 @@
 // head in the column dimension, so each lane keeps the running max / sum of
 // one query head; the probabilities leave the first MFMA already in the
 // operand layout of the second (O^T = V^T . P^T). Waves are merged through
-// LDS; partitions write (max, sum, accumulator) partials to a workspace that a
-// small second kernel merges by log-sum-exp.
+// LDS; partitions write (max, sum, accumulator) partials to a workspace, which
+// the workgroup that writes the last of a row (launches of up to one workgroup
+// a compute unit) or a small second kernel merges by log-sum-exp.
 //
 // Replaces the decode-time attention that the reference reaches through
 // compiled_model_.Run("decode", ...)
 // (runtime/executor/llm_litert_compiled_model_executor.cc:407,522).
 #include <hip/hip_runtime.h>
 #include <math.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "attn_params.h"
 #include "kernels.h"
@@ -37,17 +41,16 @@ namespace {
 // n >= group are zero columns. A lane only ever reads the entries it wrote
 // itself, so no barrier is needed; keeping Q out of the register file leaves
 // room for two waves per SIMD next to the 128 registers of K/V data in flight.
-// q_rows: the `group` query rows of this KV head, [group][D] (in HBM, or in LDS when the kernel has
-// produced them itself).
+// q_rows: the `group` query rows of this KV head, [group][D]; ks: its K scales (int8 cache only). (A kernel that has
+// produced the rows itself reads the operands from them as they lie in LDS, kRowsQ.)
 template <int KV, int D>
 constexpr int query_steps() { return KV == kF32 ? D / 16 : D / 32; }
 
 template <int KV, int IO, int D, int NQ>
-__device__ __forceinline__ void load_q(u4 (&w)[NQ], const DecodeArgs& a, const typename IoT<IO>::type* q_rows,
-                                       int kvh, int seq, int layer, int lane) {
+__device__ __forceinline__ void load_q(u4 (&w)[NQ], const typename IoT<IO>::type* q_rows, const float* ks, int group,
+                                       int lane) {
   const int n = lane & 15, g = lane >> 4;
-  const bool live = n < a.group;
-  const float* ks = KV == kI8 ? a.scales + a.geom.scale_offset(layer, seq, 0, kvh) : nullptr;
+  const bool live = n < group;
   const typename IoT<IO>::type* qrow = q_rows + (live ? n : 0) * D;
 #pragma unroll
   for (int step = 0; step < NQ; ++step) w[step] = q_operand<KV, IO, D>(qrow, ks, step, g);
@@ -66,7 +69,7 @@ __device__ __forceinline__ void store_q(u4* sm_q, const u4 (&w)[NQ], int group, 
 // tokens 4 g .. 4 g + 3 of every 16) and the unnormalised accumulators (channels
 // 16 * db + 4 * g .. + 3 of head n). Keys outside [vlo, p_hi) are masked.
 // The caller has requested block `first` into kreg / vreg (request_first_block) and left the Q
-// operands in sm_q while those loads were under way.
+// operands in sm_q while those loads were under way (QL: how they lie there, lane_q: byte offset of the lane's first).
 // patch_blk: a block one of whose rows is not in the cache yet (-1: none); patch(kreg, vreg) puts that
 // row into the block's registers once they are loaded.
 //
@@ -81,11 +84,11 @@ __device__ __forceinline__ void request_first_block(u4 (&kreg)[D / 16], u4 (&vre
   load_plane_block<D>(vreg, vrsrc, first * (64 * D), lane * 16);
 }
 
-template <int KV, int IO, int D, class Patch>
-__device__ __forceinline__ void stream_blocks(const DecodeArgs& a, __amdgpu_buffer_rsrc_t krsrc,
+template <int KV, int QL, int D, class Patch>
+__device__ __forceinline__ void stream_blocks(float sc, float softcap, __amdgpu_buffer_rsrc_t krsrc,
                                               __amdgpu_buffer_rsrc_t vrsrc, u4 (&kreg)[D / 16], u4 (&vreg)[D / 16],
-                                              int first, int blk_end, int step, int vlo, int p_hi, const u4* sm_q,
-                                              int patch_blk, Patch&& patch, int lane, float& m_run, float& l_run,
+                                              int first, int blk_end, int step, int vlo, int p_hi, const uint8_t* sm_q,
+                                              int lane_q, int patch_blk, Patch&& patch, int lane, float& m_run, float& l_run,
                                               f4 (&acc)[D / 16]) {
   constexpr int VB = KvT<KV>::VB, NT = VB / 16, NL = D / 16;
   constexpr int kBlockBytes = 64 * D;
@@ -100,16 +103,15 @@ __device__ __forceinline__ void stream_blocks(const DecodeArgs& a, __amdgpu_buff
   l_run = 0.f;
 #pragma unroll
   for (int i = 0; i < NL; ++i) acc[i] = f4{0.f, 0.f, 0.f, 0.f};
-  const float sc = a.scale, softcap = a.softcap;
 
   while (blk < blk_end) {
-    // The index is made opaque so the Q reads stay inside the loop: hoisted
+    // The offset is made opaque so the Q reads stay inside the loop: hoisted
     // they would occupy 32 to 64 registers for the whole kernel.
-    int qi = lane;
-    asm volatile("" : "+v"(qi));
+    int q_off = lane_q;
+    asm volatile("" : "+v"(q_off));
     if (blk == patch_blk) patch(kreg, vreg);
     f4 s[NT];
-    qk_block<KV, D>(kreg, sm_q, qi, s);
+    qk_block<KV, D, QL>(kreg, sm_q + q_off, s);
     const int nxt = blk + step;
     if (nxt < blk_end) load_plane_block<D>(kreg, krsrc, nxt * kBlockBytes, lane_off);
 
@@ -168,83 +170,149 @@ __device__ __forceinline__ void stream_blocks(const DecodeArgs& a, __amdgpu_buff
   // The four lanes (g = 0..3) of a head each summed their own tokens.
 }
 
-// Log-sum-exp merge of the split-KV partials: grid (query head, item), one
-// thread per channel. A separate launch because partials written by workgroups
-// on other XCDs are only guaranteed visible across a kernel boundary; an
-// in-kernel "last arrival merges" needs an L2 write-back and invalidate per
-// workgroup, which measured several times slower than this launch.
-// Grid (query head, sequence, layer). INL and the argument loads in front of the
-// first read of the partials: as in decode_attn_kernel.
-template <int KV, int IO, int D, bool INL>
-__global__ void __launch_bounds__(D) decode_merge_kernel(const DecodeArgs a) {
+// Log-sum-exp merge of the split-KV partials: grid (query head, sequence, layer), a wave for every 16 partitions (up to
+// four) that adds up their rows with four channels per lane. A launch of its own for decode launches of more workgroups than
+// compute units, where it takes 4 us and the workgroups of the attention have their slots for the next ones; smaller
+// launches merge themselves (decode_attn_kernel). What neither does is write back and invalidate an L2, the other way to
+// make partials visible to another XCD: a fence pair per workgroup made the launch several times slower.
+//
+// Bound: latency. A launch moves a few hundred KiB; its time is its trips to memory one behind the other, so there are
+// two, the arguments, then all (max, sum) pairs and rows at once, and the instructions of a single wave, so it is
+// straight-line code (rows that hold nothing are read as zeros through a resource that ends in front of them, and weigh 0).
+// INL and the argument loads in front of the first read of the partials: as in decode_attn_kernel.
+
+// What a workgroup works on: its sequence's slot, length and row in q / out, its layer's window and partition size.
+struct Place { int seq, kv_len, row, window, per; };
+template <int ITEMS, int LAYERS>
+__device__ __forceinline__ void item_of(const DecodeWork<ITEMS, LAYERS>& work, int j, Place& p) {
+  const DecodeItem it = work.item[j];
+  p.seq = it.seq;
+  p.kv_len = it.row_len & ((1u << kDecodeLenBits) - 1);
+  p.row = it.row_len >> kDecodeLenBits;
+}
+// Everything in the argument blocks, at addresses that depend on the block index only: one round of scalar loads.
+template <int ITEMS, int LAYERS>
+__device__ __forceinline__ Place inline_place(const DecodeWork<ITEMS, LAYERS>& work, int li, int j) {
+  Place p;
+  item_of(work, j, p);
+  const auto& t = work.layers;
+  if constexpr (LAYERS == 1) {
+    p.window = t.window[0];
+    p.per = t.per[0];
+  } else {
+    const int code = (t.code[li >> 4] >> (2 * (li & 15))) & 3;
+    p.window = code < 2 ? (code == 0 ? t.window[0] : t.window[1]) : (code == 2 ? t.window[2] : t.window[3]);
+    p.per = code < 2 ? (code == 0 ? t.per[0] : t.per[1]) : (code == 2 ? t.per[2] : t.per[3]);
+  }
+  return p;
+}
+__device__ __forceinline__ Place table_place(const DecodeArgs& a, const DecodeWork<kInlineItems, kInlineLayers>& work,
+                                             const DecodeTables& tab, int li, int j) {
+  Place p;
+  p.row = j;
+  if (!tab.kv_lens) {
+    item_of(work, j, p);
+  } else {
+    p.seq = tab.seq_ids ? tab.seq_ids[j] : j;
+    p.kv_len = tab.kv_lens[j];
+    if (tab.rows) p.row = tab.rows[j];
+  }
+  p.window = tab.layer_window ? tab.layer_window[a.layer_begin + li] : inline_place(work, li, 0).window;
+  p.row = __builtin_amdgcn_readfirstlane(p.row);
+  p.seq = __builtin_amdgcn_readfirstlane(p.seq);
+  p.kv_len = __builtin_amdgcn_readfirstlane(p.kv_len);
+  p.window = __builtin_amdgcn_readfirstlane(p.window);
+  p.per = decode_partition_tokens(tab.max_kv_len, p.window, a.num_splits, a.align);
+  return p;
+}
+// The blocks of a kernel's arguments behind DecodeArgs: DecodeTables where the DecodeWork does not hold everything (INL
+// false), DecodePre where the kernel runs the step before attention (PRE).
+struct NoBlock {};
+template <bool INL>
+using TableBlock = std::conditional_t<INL, NoBlock, DecodeTables>;
+template <int PRE>
+using PreBlock = std::conditional_t<PRE != 0, DecodePre, NoBlock>;
+
+constexpr int kMergeRows = 16;  // partitions of a wave at a time
+MI355_HD int merge_waves(int num_splits) { return num_splits >= 49 ? 4 : (num_splits + kMergeRows - 1) / kMergeRows; }
+
+template <int KV, int IO, int D, int ITEMS, int LAYERS, bool INL>
+__global__ void __launch_bounds__(256)
+decode_merge_kernel(const DecodeArgs a, const DecodeWork<ITEMS, LAYERS> work, const TableBlock<INL> tab) {
   using io_t = typename IoT<IO>::type;
-  __shared__ float sm_m[kMaxDecodeSplits], sm_l[kMaxDecodeSplits];
-  const int head = blockIdx.x, j = blockIdx.y, li = blockIdx.z, d = threadIdx.x;  // j: dispatch slot of the sequence
-  int batch = a.batch, layer_begin = a.layer_begin, num_splits = a.num_splits, max_kv_len = a.max_kv_len, hq = a.hq;
+  static_assert(D == 4 * 64, "four channels per lane");
+  __shared__ f4 sm_part[3][64];
+  const int head = blockIdx.x, j = blockIdx.y, li = blockIdx.z;  // j: dispatch slot of the sequence
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int batch = a.batch, layer_begin = a.layer_begin, num_splits = a.num_splits, align = a.align, hq = a.hq;
   const float* ws_ml = a.ws_ml;
   const float* ws_acc = a.ws_acc;
-  int kv_len = 0, window = 0, b = j;
-  if constexpr (INL) {
-    kv_len = a.inline_lens[j];
-    b = a.inline_row[j];
-    window = a.inline_window[li];
-  }
-  asm volatile("" : "+s"(batch), "+s"(layer_begin), "+s"(num_splits), "+s"(max_kv_len), "+s"(hq), "+s"(ws_ml),
-               "+s"(ws_acc), "+s"(kv_len), "+s"(window), "+s"(b));
-  if constexpr (!INL) {
-    if (a.inline_items) b = a.inline_row[j];
-    else if (a.rows) b = a.rows[j];
-    b = __builtin_amdgcn_readfirstlane(b);
-  }
-  const int item = li * batch + b;
+  void* out = a.out;
+  Place at{};
+  if constexpr (INL) at = inline_place(work, li, j);
+  asm volatile("" : "+s"(batch), "+s"(layer_begin), "+s"(num_splits), "+s"(align), "+s"(hq), "+s"(ws_ml), "+s"(ws_acc), "+s"(out),
+               "+s"(at.seq), "+s"(at.kv_len), "+s"(at.row), "+s"(at.window), "+s"(at.per));
+  if constexpr (!INL) at = table_place(a, work, tab, li, j);
+  const int kv_len = at.kv_len, per = at.per;
+  const int item = li * batch + at.row;
   const int layer = layer_begin + li;
-  if constexpr (!INL) {
-    kv_len = a.inline_items ? a.inline_lens[j] : a.kv_lens[j];
-    window = a.n_layers <= kInlineLayers ? a.inline_window[li] : a.layer_window[layer];
-    kv_len = __builtin_amdgcn_readfirstlane(kv_len);
-    window = __builtin_amdgcn_readfirstlane(window);
-  }
   int vlo, start;
-  decode_visible_range(kv_len, window, &vlo, &start);
-  const int per = decode_partition_tokens(max_kv_len, window, num_splits);
-  int nparts = (kv_len - start + per - 1) / per;
-  nparts = nparts < num_splits ? nparts : num_splits;
+  decode_visible_range(kv_len, at.window, align, &vlo, &start);
   const int64_t slot0 = ((int64_t)item * hq + head) * num_splits;
-  // one round trip for all (max, sum) pairs, then the weights come from LDS
-  for (int s = d; s < nparts; s += D) {
-    const float2 ml = *reinterpret_cast<const float2*>(ws_ml + (slot0 + s) * 2);
-    sm_m[s] = ml.x;
-    sm_l[s] = ml.y;
-  }
-  __syncthreads();
-  float M = -INFINITY;
-  for (int s = 0; s < nparts; ++s) M = fmaxf(M, sm_m[s]);
+  const float2* const mlp = reinterpret_cast<const float2*>(ws_ml) + slot0;
+  // Partitions s0 .. s0 + 63, lane u of this wave partition s0 + (u + 16 wave) % 64, so that its own are in lanes 0 to 15;
+  // a partition holds something if it starts in front of kv_len.
+  auto live = [&](int s) { return s < num_splits && start + s * per < kv_len; };
+  auto pairs = [&](int s0) {
+    const int s = s0 + ((lane + kMergeRows * wave) & 63);
+    return live(s) ? mlp[s] : float2{-INFINITY, 0.f};
+  };
+  f4 v[kMergeRows];
+  auto rows = [&](int s0) {
+    const int end = s0 + __popcll(__ballot(live(s0 + lane)));  // of these 64 partitions
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ws_acc + slot0 * D), 0, end * (D * 4), 0x00020000);
+#pragma unroll
+    for (int u = 0; u < kMergeRows; ++u)
+      v[u] = bit_cast<f4>(__builtin_amdgcn_raw_buffer_load_b128(rsrc, lane * 16 + (s0 + kMergeRows * wave + u) * (D * 4), 0, 0));
+  };
+  float2 ml = pairs(0);
+  rows(0);
+  f4 vscale = {1.f, 1.f, 1.f, 1.f};
+  if constexpr (KV == kI8)
+    vscale = *reinterpret_cast<const f4*>(a.scales + ((((int64_t)layer * a.max_seqs + at.seq) * 2 + 1) * a.hkv + head / a.group) * D + 4 * lane);
+  __builtin_amdgcn_sched_barrier(0);  // (everything is asked for before the pairs are waited for)
+  float M = wave_max(ml.x);
+  for (int s0 = 64; s0 < num_splits; s0 += 64) M = fmaxf(M, wave_max(pairs(s0).x));
   const float m_use = (M == -INFINITY) ? 0.f : M;
-  float A = 0.f, L = 0.f;
-  const float* accp = ws_acc + slot0 * D + d;
-  int s = 0;
-  for (; s + 8 <= nparts; s += 8) {
-    float v[8];
+  f4 A = {0.f, 0.f, 0.f, 0.f};
+  float L = 0.f;
+  for (int s0 = 0;;) {
+    const float wgt = fast_exp2(ml.x - m_use);
+    L += wave_sum(wgt * ml.y);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = accp[(int64_t)(s + u) * D];
+    for (int u = 0; u < kMergeRows; ++u) A += lane_value(wgt, u) * v[u];
+    s0 += 64;
+    if (s0 >= num_splits) break;
+    ml = pairs(s0);
+    rows(s0);
+  }
+  const int waves = merge_waves(num_splits);
+  if (waves > 1) {
+    if (wave > 0) sm_part[wave - 1][lane] = A;
+    __syncthreads();
+    if (wave > 0) return;
+    for (int w = 1; w < waves; ++w) A += sm_part[w - 1][lane];
+  }
+  io_t o[4];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const float wgt = fast_exp2(sm_m[s + u] - m_use);
-      A += wgt * v[u];
-      L += wgt * sm_l[s + u];
-    }
+  for (int e = 0; e < 4; ++e) {
+    float x = L > 0.f ? A[e] / L : 0.f;
+    if constexpr (KV == kI8) x *= vscale[e];
+    o[e] = (io_t)x;
   }
-  for (; s < nparts; ++s) {
-    const float wgt = fast_exp2(sm_m[s] - m_use);
-    A += wgt * accp[(int64_t)s * D];
-    L += wgt * sm_l[s];
-  }
-  float o = L > 0.f ? A / L : 0.f;
-  if constexpr (KV == kI8) {
-    const int seq = a.inline_items ? a.inline_seq[j] : (a.seq_ids ? a.seq_ids[j] : j);
-    o *= a.scales[a.geom.scale_offset(layer, seq, 1, head / a.group) + d];
-  }
-  reinterpret_cast<io_t*>(a.out)[((int64_t)item * hq + head) * D + d] = (io_t)o;
+  io_t* orow = reinterpret_cast<io_t*>(out) + ((int64_t)item * hq + head) * D + 4 * lane;
+  if constexpr (sizeof(io_t) == 4) *reinterpret_cast<u4*>(orow) = *reinterpret_cast<const u4*>(o);
+  else *reinterpret_cast<u2*>(orow) = *reinterpret_cast<const u2*>(o);
 }
 
 // INL: lengths, sequence ids and windows travel in the argument block (the host
@@ -264,19 +332,42 @@ __global__ void __launch_bounds__(D) decode_merge_kernel(const DecodeArgs a) {
 // delivered, so the results are the same bit for bit, and nothing waits for a store. No other
 // workgroup reads that block (partitions are whole blocks). Same arithmetic, lane for lane, as
 // pre_attention_kernel.
-// The rows are serial work for a wave (a norm with its cross-lane sums per row, two full-precision
-// sincosf per lane), so a PRE workgroup always has four waves to share them; those beyond NW leave
-// after the rows, and the attention itself runs on NW waves exactly as without PRE.
-template <int NW, bool PRE>
-constexpr int decode_wg_waves() { return PRE && NW < 4 ? 4 : NW; }
+// The rows are serial work for a wave (a norm with its cross-lane sums per row, two full-precision sincosf per lane). In a
+// launch of up to one workgroup a compute unit (kOwnWaves) four waves more have them, and the NW others request their first
+// block at once. (With the block behind the rows in the same waves, the compute unit's path to memory, 16 cycles for a load
+// of 1 KiB, 32 of them for each wave, brought the rows 1.2 us later.) Larger launches need the compute units' wave slots
+// for the attention (64 sequences of 1,000 tokens, 8 heads on 2: 40 us instead of 29): there four waves, or the NW, do both
+// (kSharedWaves), and those beyond NW leave after the rows.
+enum { kNoPre = 0, kOwnWaves = 1, kSharedWaves = 2 };
+constexpr int kRowWaves = 4;
+template <int NW, int PRE>
+constexpr int decode_wg_waves() { return PRE == kSharedWaves ? (NW < kRowWaves ? kRowWaves : NW) : NW + kRowWaves; }  // at most
 
-template <int KV, int IO, int D, int NW, bool INL, bool PRE>
-__global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_attn_kernel(const DecodeArgs a) {
+// Query rows of a PRE workgroup in LDS, as the matrix cores take them: half, bfloat16 or float32, 64 bytes of padding (the
+// operand reads of up to four rows then meet no bank conflict).
+template <int KV>
+constexpr int pre_row_bytes() { return kRowD * (KV == kF32 ? 4 : 2) + 64; }
+
+// One float of padding per four lanes: the accumulator rows of different heads start in different banks.
+constexpr int kAccStride = kRowD + 4;
+
+// What bounds this kernel in a launch of a few short partitions (a decode step of one sequence) is the way to the first
+// block: arguments, then the rows, the first K / V block and everything else that comes from memory in ONE further trip,
+// and as few instructions as can be in front of it (one wave issues an instruction every four or five cycles at best: a
+// hundred of them are a quarter of a microsecond). Measured on one layer's step at 1,152 tokens, from the first instruction:
+// rows there at 1.3 us, attention done at 5.2; with a wait for each row in front of its norm's weights, two further rounds of
+// arguments, two integer divisions and the rows in the attention's waves 2.9 and 7.0. What then ends such a launch is the
+// merge below: 2.3 us, against 3 for a launch of its own and its gap, and 3 us of the host's time saved (26 layers in turn,
+// 1,152 tokens: 252 us with two launches a layer, 222 with one).
+template <int KV, int IO, int D, int NW, int ITEMS, int LAYERS, bool INL, int PRE>
+__global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2)
+decode_attn_kernel(const DecodeArgs a, const DecodeWork<ITEMS, LAYERS> work, const TableBlock<INL> tab, const PreBlock<PRE> pre) {
   static_assert(!PRE || INL, "the fused step needs the items in the argument block");
-  constexpr int NWP = decode_wg_waves<NW, PRE>();  // waves of the workgroup; the first NW do the attention
+  constexpr int kFirstRowWave = PRE == kSharedWaves ? 0 : NW;
+  constexpr int kRowStep = PRE == kSharedWaves ? decode_wg_waves<NW, PRE>() : kRowWaves;
   constexpr int VB = KvT<KV>::VB, NL = D / 16;
   constexpr int NQ = query_steps<KV, D>();
-  extern __shared__ float smem[];
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: block addresses stay scalar
@@ -287,39 +378,46 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
   // index the host has put the longest sequences first (all their layers, then the
   // next sequence), so that the short ones fill the end of the launch.
   const int li = blockIdx.x, j = blockIdx.y;
-  // What the code in front of the first K/V loads needs from the argument block is
-  // read here in one go (left alone, the compiler sinks each scalar load behind the
-  // branch that needs it: four dependent round trips instead of one).
-  int hkv = a.geom.hkv, batch = a.batch, layer_begin = a.layer_begin, max_seqs = a.geom.max_seqs;
-  int num_splits = a.num_splits, max_kv_len = a.max_kv_len;
-  int64_t plane_bytes = a.geom.plane_bytes;
+  // What the kernel needs from the argument block is read here in one go (left alone, the compiler sinks each scalar load
+  // behind the branch that needs it: several dependent round trips instead of one).
+  int hkv = a.hkv, batch = a.batch, layer_begin = a.layer_begin, max_seqs = a.max_seqs, num_splits = a.num_splits, align = a.align;
+  uint32_t hkv_inverse = a.hkv_inverse;
+  int64_t plane_bytes = a.plane_bytes;
   const uint8_t* cache = a.cache;
-  int seq = 0, kv_len = 0, window = 0, b = j;
-  if constexpr (INL) {  // (addresses that depend on the block index only: the same round)
-    seq = a.inline_seq[j];
-    kv_len = a.inline_lens[j];
-    b = a.inline_row[j];
-    window = a.inline_window[li];
+  int hq = a.hq, G = a.group;
+  float* ws_acc = a.ws_acc;
+  float* ws_ml = a.ws_ml;
+  uint32_t* tickets = a.tickets;
+  void* out = a.out;
+  const float* scales = a.scales;
+  float sc = a.scale, softcap = a.softcap;
+  const void* q = a.q;
+  Place at{};
+  if constexpr (INL) at = inline_place(work, li, j);
+  const void *pre_q = nullptr, *pre_k = nullptr, *pre_v = nullptr;
+  const float* pre_constants = nullptr;
+  int pre_rope = 0, norm_q = 0, norm_k = 0, norm_v = 0, q_scaled = 0, k_scaled = 0;
+  float pre_eps = 0.f, pre_offset = 0.f;
+  asm volatile("" : "+s"(hkv), "+s"(batch), "+s"(layer_begin), "+s"(max_seqs), "+s"(num_splits), "+s"(align), "+s"(hkv_inverse),
+               "+s"(plane_bytes), "+s"(cache), "+s"(at.seq), "+s"(at.kv_len), "+s"(at.row), "+s"(at.window), "+s"(at.per));
+  if constexpr (PRE) {
+    pre_q = pre.q; pre_k = pre.k; pre_v = pre.v; pre_constants = pre.constants;
+    pre_rope = pre.rope; norm_q = pre.norm_q; norm_k = pre.norm_k; norm_v = pre.norm_v;
+    q_scaled = pre.q_scaled; k_scaled = pre.k_scaled;
+    pre_eps = pre.eps; pre_offset = pre.weight_offset;
+    if constexpr (PRE == kOwnWaves)
+      asm volatile("" : "+s"(pre_q), "+s"(pre_k), "+s"(pre_v), "+s"(pre_constants), "+s"(pre_rope), "+s"(norm_q),
+                 "+s"(norm_k), "+s"(norm_v), "+s"(q_scaled), "+s"(k_scaled), "+s"(pre_eps), "+s"(pre_offset), "+s"(hq),
+                 "+s"(G), "+s"(scales), "+s"(sc), "+s"(softcap), "+s"(ws_acc), "+s"(ws_ml), "+s"(tickets), "+s"(out));
   }
-  asm volatile("" : "+s"(hkv), "+s"(batch), "+s"(layer_begin), "+s"(max_seqs), "+s"(num_splits), "+s"(max_kv_len),
-               "+s"(plane_bytes), "+s"(cache), "+s"(seq), "+s"(kv_len), "+s"(window), "+s"(b));
-  const int split = blockIdx.z / hkv, kvh = blockIdx.z - split * hkv;
+  // blockIdx.z / hkv through the host's 2^32 / hkv, rounded up (0: one KV head), exact below 2^16 each
+  const int split = hkv_inverse ? (int)__umulhi(blockIdx.z, hkv_inverse) : (int)blockIdx.z, kvh = blockIdx.z - split * hkv;
   const int layer = layer_begin + li;
-  if constexpr (!INL) {
-    seq = a.inline_items ? a.inline_seq[j] : (a.seq_ids ? a.seq_ids[j] : j);
-    kv_len = a.inline_items ? a.inline_lens[j] : a.kv_lens[j];
-    if (a.inline_items) b = a.inline_row[j];
-    else if (a.rows) b = a.rows[j];
-    window = a.n_layers <= kInlineLayers ? a.inline_window[li] : a.layer_window[layer];
-  }
-  b = __builtin_amdgcn_readfirstlane(b);
+  if constexpr (!INL) at = table_place(a, work, tab, li, j);
+  const int seq = at.seq, kv_len = at.kv_len, window = at.window, per = at.per, b = at.row;
   const int item = li * batch + b;  // row of q, out and the partials
-  seq = __builtin_amdgcn_readfirstlane(seq);
-  kv_len = __builtin_amdgcn_readfirstlane(kv_len);
-  window = __builtin_amdgcn_readfirstlane(window);
   int vlo, start;
-  decode_visible_range(kv_len, window, &vlo, &start);
-  const int per = decode_partition_tokens(max_kv_len, window, num_splits);
+  decode_visible_range(kv_len, window, align, &vlo, &start);
   const int p_lo = start + split * per;
   const int p_hi = min(kv_len, p_lo + per);
   if (p_lo >= p_hi) return;  // empty partition: uniform over the workgroup
@@ -327,87 +425,119 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
   const uint8_t* kplane = cache + ((((int64_t)layer * max_seqs + seq) * hkv + kvh) * 2) * plane_bytes;  // geom.plane_offset
   const int blk_end = (p_hi + VB - 1) / VB;
   const int first_blk = __builtin_amdgcn_readfirstlane(p_lo / VB + wave);
-  const int64_t streamed = wave < NW && first_blk < blk_end ? plane_bytes : 0;  // (a helper wave of a PRE workgroup streams nothing)
+  const int64_t streamed = wave < NW && first_blk < blk_end ? plane_bytes : 0;
   const __amdgpu_buffer_rsrc_t krsrc = plane_resource(kplane, streamed);
   const __amdgpu_buffer_rsrc_t vrsrc = plane_resource(kplane + plane_bytes, streamed);
 
-  u4* sm_q = reinterpret_cast<u4*>(smem) + wave * (NQ * 64);
+  // LDS: the accumulators, maxima and sums of the waves (NW > 1), behind them the queries
+  float* sm_acc = reinterpret_cast<float*>(smem);
+  float2* sm_ml = reinterpret_cast<float2*>(sm_acc + (NW > 1 ? NW * G * kAccStride : 0));
+  uint8_t* const sm_q0 = reinterpret_cast<uint8_t*>(sm_ml + (NW > 1 ? (NW * G + 1) / 2 * 2 : 0));
   float m_run, l_run;
   f4 acc[NL];
   using io_t = typename IoT<IO>::type;
-  // What the queries are made from is asked for first, the first block right behind it: loads complete in the order
-  // they were issued, so the queries are normed, rotated and staged while the block is still on its way.
   u4 kreg[NL], vreg[NL];
   if constexpr (PRE) {
     static_assert(D == kRowD, "row helpers are written for head_dim 256");
     constexpr int ESZ = KV == kF32 ? 4 : (KV == kI8 ? 1 : 2);
     constexpr int NT = VB / 16, KPT = NL / NT;
-    const int G = a.group;
-    // behind the merge area: [G][D] query rows (io type), then the new key and value row as the planes hold them
-    io_t* sm_rows = reinterpret_cast<io_t*>(smem + NW * NQ * 64 * 4 + NW * G * (D + 2));
-    uint8_t* sm_krow = reinterpret_cast<uint8_t*>(sm_rows + G * D);
-    uint8_t* sm_vrow = sm_krow + D * ESZ;
+    constexpr int kRowBytes = pre_row_bytes<KV>();
+    // [G] query rows as matrix operands, then the new key and value row as the planes hold them
+    uint8_t* const sm_krow = sm_q0 + G * kRowBytes;
+    uint8_t* const sm_vrow = sm_krow + D * ESZ;
     const int t = kv_len - 1;
     const bool owns_row = p_hi == kv_len;  // exactly one partition per sequence and KV head
-    // The rows: one copy of the code, at kernel scope, run by every wave of the workgroup (attention waves
-    // and helper waves alike) and closed by the workgroup's one barrier, which all NWP waves reach exactly
-    // once.
-    {
+    if (wave < kFirstRowWave) {
+      request_first_block<D>(kreg, vreg, krsrc, vrsrc, first_blk, lane);
+    } else {
       const int nrows = G + (owns_row ? 2 : 0);  // G query rows, then the key and the value row
-      constexpr int kMaxRows = (kMaxGroup + 2 + NWP - 1) / NWP;
+      constexpr int kMaxRows = (kMaxGroup + 2 + kRowStep - 1) / kRowStep;
       const int d0 = 2 * lane, d1 = D / 2 + 2 * lane;
-      float xs[kMaxRows][4];
+      typename RawPair<IO>::type lo[kMaxRows], hi[kMaxRows];
       float2 w0[kMaxRows], w1[kMaxRows], freq = {0.f, 0.f};
-      // every row of this wave, its norm's weights and the frequencies in flight before the first is waited for
+      float2 ks0, ks1, vs0, vs1;  // int8 cache: scales of the lane's channels
+      ks0 = ks1 = vs0 = vs1 = float2{0.f, 0.f};
+      // every row of this wave, its norm's weights, the scales and the frequencies in flight before the first is waited for
 #pragma unroll
       for (int r = 0; r < kMaxRows; ++r) {
-        const int row = wave + r * NWP;
+        const int row = wave - kFirstRowWave + r * kRowStep;
+        w0[r] = w1[r] = float2{0.f, 0.f};
         if (row < nrows) {
-          const void* src = row < G ? a.pre_q : (row == G ? a.pre_k : a.pre_v);
-          const int64_t base = row < G ? ((int64_t)b * a.hq + kvh * G + row) * D : ((int64_t)b * hkv + kvh) * D;
-          load_pair<IO>(src, base + d0, xs[r][0], xs[r][1]);
-          load_pair<IO>(src, base + d1, xs[r][2], xs[r][3]);
-          const float* weights = row_weights(a.pre_constants, row < G ? 0 : (row == G ? 1 : 2), a.pre_q_scaled != 0, a.pre_k_scaled != 0);
-          w0[r] = w1[r] = float2{0.f, 0.f};
+          const void* src = row < G ? pre_q : (row == G ? pre_k : pre_v);
+          const int64_t base = (int64_t)(row < G ? b * hq + kvh * G + row : b * hkv + kvh) * D;
+          lo[r] = load_raw_pair<IO>(src, base + d0);
+          hi[r] = load_raw_pair<IO>(src, base + d1);
+          const float* weights = row_weights(pre_constants, row < G ? 0 : (row == G ? 1 : 2), q_scaled != 0, k_scaled != 0);
           if (weights) {
             w0[r] = *reinterpret_cast<const float2*>(weights + d0);
             w1[r] = *reinterpret_cast<const float2*>(weights + d1);
           }
         }
       }
-      if (a.pre_rope) freq = *reinterpret_cast<const float2*>(a.pre_constants + d0);
+      if (pre_rope) freq = *reinterpret_cast<const float2*>(pre_constants + d0);
+      if constexpr (KV == kI8) {
+        const float* ks = scales + (((int64_t)layer * max_seqs + seq) * 2 * hkv + kvh) * D;  // geom.scale_offset
+        ks0 = *reinterpret_cast<const float2*>(ks + d0);
+        ks1 = *reinterpret_cast<const float2*>(ks + d1);
+        vs0 = *reinterpret_cast<const float2*>(ks + hkv * D + d0);
+        vs1 = *reinterpret_cast<const float2*>(ks + hkv * D + d1);
+      }
       __builtin_amdgcn_sched_barrier(0);
-      request_first_block<D>(kreg, vreg, krsrc, vrsrc, first_blk, lane);
-      __builtin_amdgcn_sched_barrier(0);
-      const RowAngles ang = row_angles(a.pre_rope != 0, freq, t);
+      if constexpr (PRE == kSharedWaves) {
+        // The block behind the rows: a chip full of workgroups has the memory's queues full of blocks, and rows that wait in
+        // line with them keep the next workgroup's wave slots.
+#pragma unroll
+        for (int r = 0; r < kMaxRows; ++r)
+          asm volatile("" : "+v"(lo[r]), "+v"(hi[r]), "+v"(w0[r].x), "+v"(w0[r].y), "+v"(w1[r].x), "+v"(w1[r].y));
+        asm volatile("" : "+v"(freq.x), "+v"(freq.y));
+        if constexpr (KV == kI8)
+          asm volatile("" : "+v"(ks0.x), "+v"(ks0.y), "+v"(ks1.x), "+v"(ks1.y), "+v"(vs0.x), "+v"(vs0.y), "+v"(vs1.x), "+v"(vs1.y));
+        if (wave < NW) request_first_block<D>(kreg, vreg, krsrc, vrsrc, first_blk, lane);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const RowAngles ang = row_angles(pre_rope != 0, freq, t);
 #pragma unroll
       for (int r = 0; r < kMaxRows; ++r) {
-        const int row = wave + r * NWP;
+        const int row = wave - kFirstRowWave + r * kRowStep;
         if (row < nrows) {
           const int kind = row < G ? 0 : (row == G ? 1 : 2);
-          const bool norm = kind == 0 ? a.pre_norm_q != 0 : (kind == 1 ? a.pre_norm_k != 0 : a.pre_norm_v != 0);
-          const bool weighted = kind == 0 ? a.pre_q_scaled != 0 : (kind == 1 && a.pre_k_scaled != 0);
-          transform_row(xs[r], norm, weighted, w0[r], w1[r], a.pre_weight_offset, a.pre_eps, a.pre_rope != 0 && kind != 2, ang);
+          const bool norm = kind == 0 ? norm_q != 0 : (kind == 1 ? norm_k != 0 : norm_v != 0);
+          const bool weighted = kind == 0 ? q_scaled != 0 : (kind == 1 && k_scaled != 0);
+          float x[4];
+          unpack_pair<IO>(lo[r], x[0], x[1]);
+          unpack_pair<IO>(hi[r], x[2], x[3]);
+          transform_row(x, norm, weighted, w0[r], w1[r], pre_offset, pre_eps, pre_rope != 0 && kind != 2, ang);
           if (kind == 0) {
-            uint8_t* dst = reinterpret_cast<uint8_t*>(sm_rows + row * D);
-            store_pair<IO>(dst + d0 * sizeof(io_t), xs[r][0], xs[r][1]);
-            store_pair<IO>(dst + d1 * sizeof(io_t), xs[r][2], xs[r][3]);
+            // rounded to the io type, as a query that pre_attention_kernel has written out, then to the operand type
+            uint8_t* dst = sm_q0 + row * kRowBytes;
+            if constexpr (KV == kI8) {
+              float y[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) y[e] = (float)(io_t)x[e];
+              y[0] *= ks0.x; y[1] *= ks0.y; y[2] *= ks1.x; y[3] *= ks1.y;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(y[e]));  // (a product of its own, rounded once more to half, as in q_operand)
+              store_pair<kF16>(dst + d0 * 2, y[0], y[1]);
+              store_pair<kF16>(dst + d1 * 2, y[2], y[3]);
+            } else {
+              store_pair<KV>(dst + d0 * ESZ, x[0], x[1]);
+              store_pair<KV>(dst + d1 * ESZ, x[2], x[3]);
+            }
           } else {
             const int is_v = kind - 1;
             uint8_t* plane = const_cast<uint8_t*>(kplane) + is_v * plane_bytes;
-            const float* sc = KV == kI8 ? a.scales + a.geom.scale_offset(layer, seq, is_v, kvh) : nullptr;
-            store_cache_row<KV, false>(plane, sc, is_v, t, xs[r], lane);
-            store_cache_row<KV, true>(is_v ? sm_vrow : sm_krow, sc, is_v, t, xs[r], lane);
+            const float2 s0 = is_v ? vs0 : ks0, s1 = is_v ? vs1 : ks1;
+            store_cache_row<KV, false>(plane, s0, s1, is_v, t, x, lane);
+            store_cache_row<KV, true>(is_v ? sm_vrow : sm_krow, s0, s1, is_v, t, x, lane);
           }
         }
       }
     }
     // (a barrier for LDS alone: __syncthreads() would also wait for the block under way)
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (wave >= NW) return;  // a helper wave: its share of the rows, nothing else
-    u4 qw[NQ];
-    load_q<KV, IO, D>(qw, a, sm_rows, kvh, seq, layer, lane);
-    store_q(sm_q, qw, a.group, lane);
+    lds_barrier();
+    if (wave >= NW && !tickets) return;  // a row wave has done its share
+    // lane (n, g) reads row n as it lies (columns n >= G, which nobody looks at, get row 0)
+    const int lane_q = (n < G ? n : 0) * kRowBytes + g * (KV == kI8 ? 32 : 16);
     // Row t in the registers of its block. K: chunk c of the row is the 16 bytes of lane (t % 16, g) in load
     // (t % VB) / 16 * KPT + j with c = 4 j + g. V: element d of the row sits in lane (d % 16, (t % 16) / 4), load
     // d / 16, at element slot 4 * ((t % VB) / 16) + t % 4 of the lane's 16 bytes.
@@ -449,150 +579,264 @@ __global__ void __launch_bounds__((decode_wg_waves<NW, PRE>()) * 64, 2) decode_a
         vr[db] = (vr[db] & keep) | (ev & mask);
       }
     };
-    stream_blocks<KV, IO, D>(a, krsrc, vrsrc, kreg, vreg, first_blk, blk_end, NW, vlo, p_hi, sm_q, owns_row ? t / VB : -1,
-                             patch, lane, m_run, l_run, acc);
-  } else {
-    const io_t* q_rows = reinterpret_cast<const io_t*>(a.q) + ((int64_t)item * a.hq + kvh * a.group) * D;
+    if (wave < NW)
+      stream_blocks<KV, kRowsQ, D>(sc, softcap, krsrc, vrsrc, kreg, vreg, first_blk, blk_end, NW, vlo, p_hi, sm_q0, lane_q,
+                                   owns_row ? t / VB : -1, patch, lane, m_run, l_run, acc);
+  } else if (wave < NW) {
+    u4* const sm_q = reinterpret_cast<u4*>(sm_q0) + wave * (NQ * 64);
+    // The queries are asked for first, the first block right behind them: loads complete in the order they were issued, so
+    // the queries are staged while the block is still on its way.
+    const io_t* q_rows = reinterpret_cast<const io_t*>(q) + ((int64_t)item * hq + kvh * G) * D;
+    const float* ks = KV == kI8 ? scales + (((int64_t)layer * max_seqs + seq) * 2 * hkv + kvh) * D : nullptr;  // geom.scale_offset
     u4 qw[NQ];
     // (queries that are converted on the way would be waited for before the block is asked for: the block goes first)
-    if constexpr (KV == IO) load_q<KV, IO, D>(qw, a, q_rows, kvh, seq, layer, lane);
+    if constexpr (KV == IO) load_q<KV, IO, D>(qw, q_rows, ks, G, lane);
     __builtin_amdgcn_sched_barrier(0);
     request_first_block<D>(kreg, vreg, krsrc, vrsrc, first_blk, lane);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (KV != IO) load_q<KV, IO, D>(qw, a, q_rows, kvh, seq, layer, lane);
-    store_q(sm_q, qw, a.group, lane);
+    if constexpr (KV != IO) load_q<KV, IO, D>(qw, q_rows, ks, G, lane);
+    store_q(sm_q, qw, G, lane);
     auto patch = [](u4 (&)[NL], u4 (&)[NL]) {};
-    stream_blocks<KV, IO, D>(a, krsrc, vrsrc, kreg, vreg, first_blk, blk_end, NW, vlo, p_hi, sm_q, -1, patch, lane, m_run,
-                             l_run, acc);
+    stream_blocks<KV, kStagedQ, D>(sc, softcap, krsrc, vrsrc, kreg, vreg, first_blk, blk_end, NW, vlo, p_hi,
+                                   reinterpret_cast<const uint8_t*>(sm_q), lane * 16, -1, patch, lane, m_run, l_run, acc);
   }
-  float l_tot = wave_xor_add<16>(l_run);
-  l_tot = wave_xor_add<32>(l_tot);
-
-  const int G = a.group;
-  if constexpr (NW == 1) {
-    // One wave: nothing to merge. Lane (n, g) holds channels 16 * db + 4 * g .. + 3 of head n.
-    if (n < G) {
-      const int head = kvh * G + n;
-      if (a.num_splits == 1) {
-        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-        io_t* orow = reinterpret_cast<io_t*>(a.out) + ((int64_t)item * a.hq + head) * D + 4 * g;
-        const float* vs = nullptr;
-        if constexpr (KV == kI8) vs = a.scales + a.geom.scale_offset(layer, seq, 1, kvh) + 4 * g;
+  // Lane (n, g) holds channels 16 * db + 4 * g .. + 3 of head n; in rows of the output and of the partials:
+  const int64_t head0 = (int64_t)item * hq + kvh * G;
+  const float* vs = nullptr;
+  if constexpr (KV == kI8) vs = scales + ((((int64_t)layer * max_seqs + seq) * 2 + 1) * hkv + kvh) * D;  // geom.scale_offset
+  auto store_out = [&](int hn, f4 A, float L, f4 vscale) {  // a row, four channels per lane
+    io_t o[4];
 #pragma unroll
-        for (int db = 0; db < NL; ++db) {
-          io_t o[4];
+    for (int e = 0; e < 4; ++e) {
+      float x = L > 0.f ? A[e] / L : 0.f;
+      if constexpr (KV == kI8) x *= vscale[e];
+      o[e] = (io_t)x;
+    }
+    io_t* orow = reinterpret_cast<io_t*>(out) + (head0 + hn) * D + 4 * lane;
+    if constexpr (sizeof(io_t) == 4) *reinterpret_cast<u4*>(orow) = *reinterpret_cast<const u4*>(o);
+    else *reinterpret_cast<u2*>(orow) = *reinterpret_cast<const u2*>(o);
+  };
+  auto load_vscale = [&]() {
+    f4 r = {1.f, 1.f, 1.f, 1.f};
+    if constexpr (KV == kI8) r = *reinterpret_cast<const f4*>(vs + 4 * lane);
+    return r;
+  };
+  // The partials of this KV head, [G][num_splits] rows and pairs; written through to memory where another workgroup of the
+  // launch reads them.
+  const __amdgpu_buffer_rsrc_t acc_rsrc = __builtin_amdgcn_make_buffer_rsrc(ws_acc + head0 * num_splits * D, 0, G * num_splits * (D * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ml_rsrc = __builtin_amdgcn_make_buffer_rsrc(ws_ml + head0 * num_splits * 2, 0, G * num_splits * 8, 0x00020000);
+  auto store_part = [&](int hn, int d, f4 x) {
+    const int at_byte = ((hn * num_splits + split) * D + d) * 4;
+    if (tickets) __builtin_amdgcn_raw_buffer_store_b128(bit_cast<u4>(x), acc_rsrc, at_byte, 0, kDeviceScope);
+    else __builtin_amdgcn_raw_buffer_store_b128(bit_cast<u4>(x), acc_rsrc, at_byte, 0, 0);
+  };
+  auto store_pair_ml = [&](int hn, float m, float l) {
+    const u2 x = {__float_as_uint(m), __float_as_uint(l)};
+    const int at_byte = (hn * num_splits + split) * 8;
+    if (tickets) __builtin_amdgcn_raw_buffer_store_b64(x, ml_rsrc, at_byte, 0, kDeviceScope);
+    else __builtin_amdgcn_raw_buffer_store_b64(x, ml_rsrc, at_byte, 0, 0);
+  };
+  if (wave < NW) {
+    float l_tot = wave_xor_add<16>(l_run);
+    l_tot = wave_xor_add<32>(l_tot);
+    if constexpr (NW == 1) {
+      // One wave: nothing to merge.
+      if (n < G) {
+        if (num_splits == 1) {
+          const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+          io_t* orow = reinterpret_cast<io_t*>(out) + (head0 + n) * D + 4 * g;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float x = acc[db][e] * inv;
-            if constexpr (KV == kI8) x *= vs[16 * db + e];
-            o[e] = (io_t)x;
+          for (int db = 0; db < NL; ++db) {
+            io_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              float x = acc[db][e] * inv;
+              if constexpr (KV == kI8) x *= vs[16 * db + 4 * g + e];
+              o[e] = (io_t)x;
+            }
+            if constexpr (sizeof(io_t) == 4) *reinterpret_cast<u4*>(orow + 16 * db) = *reinterpret_cast<const u4*>(o);
+            else *reinterpret_cast<u2*>(orow + 16 * db) = *reinterpret_cast<const u2*>(o);
           }
-          if constexpr (sizeof(io_t) == 4) *reinterpret_cast<u4*>(orow + 16 * db) = *reinterpret_cast<const u4*>(o);
-          else *reinterpret_cast<u2*>(orow + 16 * db) = *reinterpret_cast<const u2*>(o);
+        } else {
+#pragma unroll
+          for (int db = 0; db < NL; ++db) store_part(n, 16 * db + 4 * g, acc[db]);
+          if (g == 0) store_pair_ml(n, m_run, l_tot);
         }
-      } else {
-        const int64_t slot = ((int64_t)item * a.hq + head) * a.num_splits + split;
-        float* prow = a.ws_acc + slot * D + 4 * g;
-#pragma unroll
-        for (int db = 0; db < NL; ++db) *reinterpret_cast<f4*>(prow + 16 * db) = acc[db];
-        if (g == 0) *reinterpret_cast<float2*>(a.ws_ml + slot * 2) = float2{m_run, l_tot};
       }
-    }
-    return;
-  }
-  // Merge the waves through LDS: [NW][group][D] accumulators, then max, sum.
-  float* sm_acc = smem + NW * NQ * 64 * 4;  // behind the waves' Q slices
-  float* sm_m = sm_acc + NW * G * D;
-  float* sm_l = sm_m + NW * G;
-  if (n < G) {
-    float* dst = sm_acc + (wave * G + n) * D + 4 * g;
-#pragma unroll
-    for (int db = 0; db < NL; ++db) *reinterpret_cast<f4*>(dst + 16 * db) = acc[db];
-    if (g == 0) {
-      sm_m[wave * G + n] = m_run;
-      sm_l[wave * G + n] = l_tot;
-    }
-  }
-  __syncthreads();
-
-  for (int e = threadIdx.x; e < G * D; e += NW * 64) {
-    const int hn = e / D, d = e - hn * D;
-    float M = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_m[w * G + hn]);
-    const float m_use = (M == -INFINITY) ? 0.f : M;
-    float A = 0.f, L = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float wgt = fast_exp2(sm_m[w * G + hn] - m_use);
-      A += wgt * sm_acc[(w * G + hn) * D + d];
-      L += wgt * sm_l[w * G + hn];
-    }
-    const int head = kvh * G + hn;
-    if (a.num_splits == 1) {
-      float o = L > 0.f ? A / L : 0.f;
-      if constexpr (KV == kI8) o *= a.scales[a.geom.scale_offset(layer, seq, 1, kvh) + d];
-      reinterpret_cast<io_t*>(a.out)[((int64_t)item * a.hq + head) * D + d] = (io_t)o;
     } else {
-      const int64_t slot = ((int64_t)item * a.hq + head) * a.num_splits + split;
-      a.ws_acc[slot * D + d] = A;
-      if (d == 0) {
-        a.ws_ml[slot * 2] = M;
-        a.ws_ml[slot * 2 + 1] = L;
+      // Merge the waves through LDS, then a wave per head and four channels per lane.
+      if (n < G) {
+        float* dst = sm_acc + (wave * G + n) * kAccStride + 4 * g;
+#pragma unroll
+        for (int db = 0; db < NL; ++db) *reinterpret_cast<f4*>(dst + 16 * db) = acc[db];
+        if (g == 0) sm_ml[wave * G + n] = float2{m_run, l_tot};
+      }
+      lds_barrier();
+      for (int hn = wave; hn < G; hn += NW) {
+        f4 v[NW];
+        float2 ml[NW];
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          ml[w] = sm_ml[w * G + hn];
+          v[w] = *reinterpret_cast<const f4*>(sm_acc + (w * G + hn) * kAccStride + 4 * lane);
+        }
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, ml[w].x);
+        const float m_use = (M == -INFINITY) ? 0.f : M;
+        f4 A = {0.f, 0.f, 0.f, 0.f};
+        float L = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          const float wgt = fast_exp2(ml[w].x - m_use);
+          A += wgt * v[w];
+          L += wgt * ml[w].y;
+        }
+        if (num_splits == 1) {
+          store_out(hn, A, L, load_vscale());
+        } else {
+          store_part(hn, 4 * lane, A);
+          if (lane == 0) store_pair_ml(hn, M, L);
+        }
       }
     }
+  } else if constexpr (NW > 1) {
+    lds_barrier();  // (a wave that is here for the merge of the partials)
+  }
+  if (!tickets) return;
+
+  // The merge of the partials by the workgroup that writes the last of them: every workgroup counts the keys of its
+  // partition once its stores have been acknowledged (device scope: they and the loads below go through to memory, the
+  // workgroups of a row sit on different XCDs, whose L2s are different ones; no cache is written back or invalidated).
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
+  uint32_t* const sm_last = reinterpret_cast<uint32_t*>(smem);
+  if (threadIdx.x == 0) {
+    uint32_t* ticket = tickets + item * hkv + kvh;
+    const uint32_t mine = p_hi - p_lo;
+    const uint32_t before = __hip_atomic_fetch_add(ticket, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool last = before + mine == (uint32_t)(kv_len - start);
+    if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+    *sm_last = last;
+  }
+  lds_barrier();
+  if (!__builtin_amdgcn_readfirstlane((int)*sm_last)) return;
+  const f4 vscale = load_vscale();
+  for (int hn = wave; hn < G; hn += NW + kRowWaves) {
+    // as in decode_merge_kernel, sum for sum, with up to two of its waves' rows under way together
+    const bool live = lane < num_splits && start + lane * per < kv_len;
+    const int nparts = __popcll(__ballot(live));
+    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(ws_acc + (head0 + hn) * num_splits * D, 0, nparts * (D * 4), 0x00020000);
+    const u2 pair = __builtin_amdgcn_raw_buffer_load_b64(ml_rsrc, (hn * num_splits + (live ? lane : 0)) * 8, 0, kDeviceScope);
+    f4 v[2 * kMergeRows];
+    auto load_rows = [&](int u0, int s0) {
+#pragma unroll
+      for (int u = 0; u < kMergeRows; ++u)
+        v[u0 + u] = bit_cast<f4>(__builtin_amdgcn_raw_buffer_load_b128(rows, lane * 16 + (s0 + u) * (D * 4), 0, kDeviceScope));
+    };
+    load_rows(0, 0);
+    load_rows(kMergeRows, kMergeRows);
+    __builtin_amdgcn_sched_barrier(0);
+    const float m = live ? __uint_as_float(pair[0]) : -INFINITY;
+    const float M = wave_max(m);
+    const float m_use = (M == -INFINITY) ? 0.f : M;
+    const float wgt = fast_exp2(m - m_use);
+    const float L = wave_sum(wgt * (live ? __uint_as_float(pair[1]) : 0.f));
+    f4 A = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < nparts; s0 += 2 * kMergeRows) {
+      if (s0 > 0) {
+        load_rows(0, s0);
+        load_rows(kMergeRows, s0 + kMergeRows);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        f4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < kMergeRows; ++u) sum += lane_value(wgt, s0 + h * kMergeRows + u) * v[h * kMergeRows + u];
+        A = s0 + h == 0 ? sum : A + sum;
+      }
+    }
+    store_out(hn, A, L, vscale);
   }
 }
 
-template <int KV, int IO, int D, int NW, bool INL, bool PRE = false>
-hipError_t launch_inl(const DecodeArgs& a, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
-  const dim3 grid(a.n_layers, a.batch, a.num_splits * a.geom.hkv);
+template <int KV, int IO, int D, int NW, int ITEMS, int LAYERS, bool INL, int PRE = kNoPre>
+hipError_t launch_inl(const DecodeLaunch& l, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+  const DecodeArgs& a = l.args;
+  const dim3 grid(l.n_layers, a.batch, a.num_splits * a.hkv);
   constexpr int NQ = query_steps<KV, D>();
-  const size_t lds = (size_t)NW * NQ * 64 * 16 + (size_t)NW * a.group * (D + 2) * sizeof(float) +
-                     (PRE ? (size_t)a.group * D * sizeof(typename IoT<IO>::type) + 2 * (size_t)D * a.geom.esize : 0);
+  const size_t merge = NW > 1 ? (size_t)NW * a.group * kAccStride * sizeof(float) + (size_t)(NW * a.group + 1) / 2 * 2 * sizeof(float2) : 0;
+  const size_t lds = merge + (PRE ? (size_t)a.group * pre_row_bytes<KV>() + 2 * (size_t)D * l.esize : (size_t)NW * NQ * 64 * 16);
+  DecodeWork<ITEMS, LAYERS> work;
+  std::copy(l.work.item, l.work.item + ITEMS, work.item);
+  if constexpr (LAYERS == 1) {
+    work.layers.window[0] = l.work.layers.window[0];
+    work.layers.per[0] = l.work.layers.per[0];
+  } else {
+    work.layers = l.work.layers;
+  }
+  TableBlock<INL> tab{};
+  if constexpr (!INL) {
+    tab = l.tables;
+    tab.max_kv_len = l.max_kv_len;
+    if (l.inline_layers) tab.layer_window = nullptr;
+    if (l.inline_items) tab.kv_lens = nullptr;
+  }
+  PreBlock<PRE> pre{};
+  if constexpr (PRE) pre = l.pre;
+  // (a launch that merges its own partials has waves that are there for that, as the fused step has for its rows)
+  const int waves = PRE || a.tickets ? decode_wg_waves<NW, PRE>() : NW;
   // ev0/ev1 are attached to the dispatch itself: they carry the kernel's own
   // begin and end timestamps, not the host-side launch latency around it.
-  hipExtLaunchKernelGGL((decode_attn_kernel<KV, IO, D, NW, INL, PRE>), grid, dim3(decode_wg_waves<NW, PRE>() * 64), lds,
-                        stream, ev0, ev1, 0, a);
+  hipExtLaunchKernelGGL((decode_attn_kernel<KV, IO, D, NW, ITEMS, LAYERS, INL, PRE>), grid, dim3(waves * 64), lds, stream, ev0,
+                        ev1, 0, a, work, tab, pre);
   hipError_t err = hipGetLastError();
-  if (err != hipSuccess || a.num_splits == 1) return err;
-  hipLaunchKernelGGL((decode_merge_kernel<KV, IO, D, INL>), dim3(a.hq, a.batch, a.n_layers), dim3(D), 0, stream, a);
+  if (err != hipSuccess || a.num_splits == 1 || a.tickets) return err;
+  hipLaunchKernelGGL((decode_merge_kernel<KV, IO, D, ITEMS, LAYERS, INL>), dim3(a.hq, a.batch, l.n_layers),
+                     dim3(64 * merge_waves(a.num_splits)), 0, stream, a, work, tab);
   return hipGetLastError();
 }
 
 template <int KV, int IO, int D, int NW>
-hipError_t launch_variant(const DecodeArgs& a, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
-  if (a.pre_q) {
-    if (!a.inline_items || a.n_layers != 1) return hipErrorInvalidValue;
-    return launch_inl<KV, IO, D, NW, true, true>(a, stream, ev0, ev1);
+hipError_t launch_variant(const DecodeLaunch& l, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+  const bool few = l.args.batch <= kFewItems;
+  if (l.fused) {
+    if (!l.inline_items || !l.inline_layers || l.n_layers != 1) return hipErrorInvalidValue;
+    if ((int64_t)l.rule_batch * l.args.hkv * l.args.num_splits > kLatencyWorkgroups)
+      return launch_inl<KV, IO, D, NW, kInlineItems, 1, true, kSharedWaves>(l, stream, ev0, ev1);
+    return few ? launch_inl<KV, IO, D, NW, kFewItems, 1, true, kOwnWaves>(l, stream, ev0, ev1)
+               : launch_inl<KV, IO, D, NW, kInlineItems, 1, true, kOwnWaves>(l, stream, ev0, ev1);
   }
-  if (a.inline_items && a.n_layers <= kInlineLayers) return launch_inl<KV, IO, D, NW, true>(a, stream, ev0, ev1);
-  return launch_inl<KV, IO, D, NW, false>(a, stream, ev0, ev1);
+  if (!l.inline_items || !l.inline_layers) return launch_inl<KV, IO, D, NW, kInlineItems, kInlineLayers, false>(l, stream, ev0, ev1);
+  return few ? launch_inl<KV, IO, D, NW, kFewItems, kInlineLayers, true>(l, stream, ev0, ev1)
+             : launch_inl<KV, IO, D, NW, kInlineItems, kInlineLayers, true>(l, stream, ev0, ev1);
 }
 
 template <int KV, int IO, int D>
-hipError_t launch_typed(const DecodeArgs& a, const DecodeTuning& t, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+hipError_t launch_typed(const DecodeLaunch& l, const DecodeTuning& t, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+  const DecodeArgs& a = l.args;
   int waves = t.waves;
   if (waves == 0) {
     // Measured on MI355X (head_dim 256, 4096-token context): with several
     // workgroups per CU one wave each is as fast or faster (fewer LDS merges),
-    // with less than one per CU more waves per workgroup hide the latency.
-    const int wgs = a.n_layers * (a.rule_batch > 0 ? a.rule_batch : a.batch) * a.geom.hkv * a.num_splits;
-    waves = wgs >= 768 ? 1 : wgs >= 256 ? 2 : 4;
-    // ... and one wave when a partition is one or two key blocks: more waves
-    // would only add to the merge (one layer of 1024 tokens in 64-token
-    // partitions: 7.7 us instead of 8.7 us per call).
+    // with less than one per CU more waves per workgroup hide the latency:
+    // one for every block of a partition, up to four (a step of one sequence of
+    // 1,152 tokens in partitions of two blocks: 8.8 us with two waves, 9.4 with
+    // one, 9.2 with four; of one block: 7.8, 8.1 with two).
     constexpr int VB = KvT<KV>::VB;
-    if (decode_partition_tokens(a.max_kv_len, 0, a.num_splits) <= 2 * VB) waves = 1;
+    const int wgs = l.n_layers * l.rule_batch * a.hkv * a.num_splits;
+    const int blocks = decode_partition_tokens(l.max_kv_len, l.widest_window, a.num_splits, a.align) / VB;
+    if (wgs <= kLatencyWorkgroups) waves = blocks >= 3 ? 4 : blocks;
+    else waves = wgs >= 768 || a.num_splits > 1 || blocks <= 2 ? 1 : 2;
     // ... and four waves for a big launch of whole sequences of unequal lengths: the wave slots of
     // the chip then hold a quarter of the workgroups at a time instead of all of them, and the short
     // sequences, dispatched last, fill in behind the long ones (16 layers x 64 sequences of 256 to
     // 4096 tokens: 6.5 instead of 6.1 TB/s; sequences of equal length lose 1 % and keep one wave).
-    if (a.num_splits == 1 && wgs >= 1024 && a.min_kv_len * 4 < a.max_kv_len * 3) waves = 4;
+    if (a.num_splits == 1 && wgs >= 1024 && l.min_kv_len * 4 < l.max_kv_len * 3) waves = 4;
   }
-  if (waves == 1) return launch_variant<KV, IO, D, 1>(a, s, e0, e1);
-  if (waves == 2) return launch_variant<KV, IO, D, 2>(a, s, e0, e1);
-  return launch_variant<KV, IO, D, 4>(a, s, e0, e1);
+  if (waves == 1) return launch_variant<KV, IO, D, 1>(l, s, e0, e1);
+  if (waves == 2) return launch_variant<KV, IO, D, 2>(l, s, e0, e1);
+  return launch_variant<KV, IO, D, 4>(l, s, e0, e1);
 }
 
 }  // namespace
@@ -604,17 +848,17 @@ bool decode_supported(int kv_dtype, int io_dtype, int head_dim) {
   return kv_dtype == io_dtype || (io_dtype == kF32 && (kv_dtype == kF16 || kv_dtype == kBF16));
 }
 
-hipError_t launch_decode(const DecodeArgs& a, int kv_dtype, int io_dtype, const DecodeTuning& tuning,
+hipError_t launch_decode(const DecodeLaunch& l, int kv_dtype, int io_dtype, const DecodeTuning& tuning,
                          hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
   switch (kv_dtype * 4 + io_dtype) {
-    case kF32 * 4 + kF32: return launch_typed<kF32, kF32, 256>(a, tuning, stream, ev0, ev1);
-    case kF16 * 4 + kF16: return launch_typed<kF16, kF16, 256>(a, tuning, stream, ev0, ev1);
-    case kF16 * 4 + kF32: return launch_typed<kF16, kF32, 256>(a, tuning, stream, ev0, ev1);
-    case kBF16 * 4 + kBF16: return launch_typed<kBF16, kBF16, 256>(a, tuning, stream, ev0, ev1);
-    case kBF16 * 4 + kF32: return launch_typed<kBF16, kF32, 256>(a, tuning, stream, ev0, ev1);
-    case kI8 * 4 + kF16: return launch_typed<kI8, kF16, 256>(a, tuning, stream, ev0, ev1);
-    case kI8 * 4 + kBF16: return launch_typed<kI8, kBF16, 256>(a, tuning, stream, ev0, ev1);
-    case kI8 * 4 + kF32: return launch_typed<kI8, kF32, 256>(a, tuning, stream, ev0, ev1);
+    case kF32 * 4 + kF32: return launch_typed<kF32, kF32, 256>(l, tuning, stream, ev0, ev1);
+    case kF16 * 4 + kF16: return launch_typed<kF16, kF16, 256>(l, tuning, stream, ev0, ev1);
+    case kF16 * 4 + kF32: return launch_typed<kF16, kF32, 256>(l, tuning, stream, ev0, ev1);
+    case kBF16 * 4 + kBF16: return launch_typed<kBF16, kBF16, 256>(l, tuning, stream, ev0, ev1);
+    case kBF16 * 4 + kF32: return launch_typed<kBF16, kF32, 256>(l, tuning, stream, ev0, ev1);
+    case kI8 * 4 + kF16: return launch_typed<kI8, kF16, 256>(l, tuning, stream, ev0, ev1);
+    case kI8 * 4 + kBF16: return launch_typed<kI8, kBF16, 256>(l, tuning, stream, ev0, ev1);
+    case kI8 * 4 + kF32: return launch_typed<kI8, kF32, 256>(l, tuning, stream, ev0, ev1);
   }
   return hipErrorInvalidValue;
 }

@@ -39,6 +39,10 @@ struct IoT<kBF16> { using type = __bf16; };
 // lane for all 32 loads) and are bounds-checked against the plane size.
 constexpr int kStreamingLoad = 2;  // "nt": the rows are read once per call
 constexpr int kCachedLoad = 0;     // the rows are read by several workgroups of a call
+constexpr int kDeviceScope = 16;   // "sc1": through to memory, for what workgroups of one launch hand to each other
+
+// Workgroup barrier that orders LDS traffic only (__syncthreads() would also wait for every load and store under way).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_resource(const uint8_t* plane, int64_t plane_bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(plane), 0, (int)plane_bytes, 0x00020000);
@@ -110,12 +114,23 @@ __device__ __forceinline__ u4 q_operand(const typename IoT<IO>::type* qrow, cons
   }
 }
 
+// Where a lane's Q operands of the steps lie in LDS, relative to the lane's first. Staged: [step][64 lanes] of 16 bytes.
+// Rows: whole query rows in the matrix cores' type, of which lane (n, g) reads chunk 4 * step + g (int8 cache: half
+// `step` % 2 of chunk 4 * (step / 2) + g) of row n.
+constexpr int kStagedQ = 0, kRowsQ = 1;
+template <int KV, int QL>
+__device__ __forceinline__ constexpr int q_step_bytes(int step) {
+  return QL == kStagedQ ? step * 1024 : (KV == kI8 ? (step >> 1) * 128 + (step & 1) * 16 : step * 64);
+}
+template <int KV, int QL>
+__device__ __forceinline__ u4 q_at(const uint8_t* lane_q, int step) {
+  return *reinterpret_cast<const u4*>(lane_q + q_step_bytes<KV, QL>(step));
+}
+
 // S^T tiles of one block: s[T][i] is the raw score of token 16*T + 4*g + i
-// against head n. sm_q[step * 64 + qi] is this lane's Q operand of a step; each
-// is read once and used for every tile of the block.
-template <int KV, int D>
-__device__ __forceinline__ void qk_block(const u4 (&kreg)[D / 16], const u4* sm_q, int qi,
-                                         f4 (&s)[KvT<KV>::VB / 16]) {
+// against head n. lane_q: this lane's Q operands in LDS; each is read once and used for every tile of the block.
+template <int KV, int D, int QL = kStagedQ>
+__device__ __forceinline__ void qk_block(const u4 (&kreg)[D / 16], const uint8_t* lane_q, f4 (&s)[KvT<KV>::VB / 16]) {
   constexpr int NT = KvT<KV>::VB / 16;
   constexpr int KPT = (D / 16) / NT;  // K loads per 16-token tile
 #pragma unroll
@@ -123,15 +138,15 @@ __device__ __forceinline__ void qk_block(const u4 (&kreg)[D / 16], const u4* sm_
 #pragma unroll
   for (int j = 0; j < KPT; ++j) {
     if constexpr (KV == kF16) {
-      const h8 qv = bit_cast<h8>(sm_q[j * 64 + qi]);
+      const h8 qv = bit_cast<h8>(q_at<KV, QL>(lane_q, j));
 #pragma unroll
       for (int T = 0; T < NT; ++T) s[T] = mfma16_f16(bit_cast<h8>(kreg[T * KPT + j]), qv, s[T]);
     } else if constexpr (KV == kBF16) {
-      const b8 qv = bit_cast<b8>(sm_q[j * 64 + qi]);
+      const b8 qv = bit_cast<b8>(q_at<KV, QL>(lane_q, j));
 #pragma unroll
       for (int T = 0; T < NT; ++T) s[T] = mfma16_bf16(bit_cast<b8>(kreg[T * KPT + j]), qv, s[T]);
     } else if constexpr (KV == kF32) {
-      const f4 qf = bit_cast<f4>(sm_q[j * 64 + qi]);
+      const f4 qf = bit_cast<f4>(q_at<KV, QL>(lane_q, j));
 #pragma unroll
       for (int T = 0; T < NT; ++T) {
         const f4 kf = bit_cast<f4>(kreg[T * KPT + j]);
@@ -139,7 +154,7 @@ __device__ __forceinline__ void qk_block(const u4 (&kreg)[D / 16], const u4* sm_
         for (int e = 0; e < 4; ++e) s[T] = mfma16_f32(kf[e], qf[e], s[T]);
       }
     } else {
-      const h8 q0 = bit_cast<h8>(sm_q[(2 * j) * 64 + qi]), q1 = bit_cast<h8>(sm_q[(2 * j + 1) * 64 + qi]);
+      const h8 q0 = bit_cast<h8>(q_at<KV, QL>(lane_q, 2 * j)), q1 = bit_cast<h8>(q_at<KV, QL>(lane_q, 2 * j + 1));
 #pragma unroll
       for (int T = 0; T < NT; ++T) {
         h8 lo, hi;

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace mi355 {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -128,6 +130,22 @@ __device__ __forceinline__ float wave_xor_add(float v) {
   static_assert(MASK == 16 || MASK == 32, "rows or halves of a wave");
   const float2 r = MASK == 16 ? wave_swap16(v) : wave_swap32(v);
   return r.x + r.y;
+}
+// The maximum over all lanes, in every lane.
+__device__ __forceinline__ float wave_max(float v) {
+  auto step = [](float x, auto ctrl) {
+    return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true)));
+  };
+  v = step(v, std::integral_constant<int, 0xB1>{});   // (the moves of wave_sum)
+  v = step(v, std::integral_constant<int, 0x4E>{});
+  v = step(v, std::integral_constant<int, 0x141>{});
+  v = step(v, std::integral_constant<int, 0x140>{});
+  v = wave_xor_max<16>(v);
+  return wave_xor_max<32>(v);
+}
+// The value of one lane, as a scalar.
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {

@@ -79,6 +79,8 @@ __global__ void iota_items_kernel(int32_t* lens, int32_t* seq_ids, int n, int q_
 
 }  // namespace
 
+constexpr int kSchedInts = 64;  // prefill queue counters and the stream probe's sink word, on a cache line of their own
+static_assert(kPrefillSchedInts + 1 <= kSchedInts, "the counters and the sink word");
 constexpr int kI8MinRows = 16;  // int8 cache: prefill calls of fewer rows take the row-wise path unless an option moves that
 
 struct mi355_attn {
@@ -92,6 +94,7 @@ struct mi355_attn {
   float* scales = nullptr;
   int32_t* d_window = nullptr;
   int32_t* d_sched = nullptr;  // prefill work-queue counters
+  uint32_t* d_tickets = nullptr;  // tickets of decode launches that merge their own partials (behind the counters)
   PrefillPlans pf_plans;       // prefill work plans by launch shape
   float* d_pf_acc = nullptr;   // prefill key split: parts of split tiles, allocated on first use
   float* d_pf_ml = nullptr;
@@ -242,22 +245,44 @@ int check_layers(const mi355_attn* h, int layer_begin, int n_layers, char** erro
   return 0;
 }
 
-void fill_decode_common(const mi355_attn* h, DecodeArgs* a) {
-  a->cache = h->cache;
-  a->scales = h->scales;
-  a->ws_acc = h->ws_acc;
-  a->ws_ml = h->ws_ml;
-  a->layer_window = h->d_window;
-  a->geom = h->geom;
-  a->hq = h->cfg.num_q_heads;
-  a->group = h->cfg.num_q_heads / h->cfg.num_kv_heads;
-  a->scale = h->cfg.scale;
-  a->softcap = h->cfg.softcap;
+void fill_decode_common(const mi355_attn* h, DecodeLaunch* l) {
+  DecodeArgs& a = l->args;
+  a.cache = h->cache;
+  a.scales = h->scales;
+  a.ws_acc = h->ws_acc;
+  a.ws_ml = h->ws_ml;
+  a.plane_bytes = h->geom.plane_bytes;
+  a.hkv = h->geom.hkv;
+  a.max_seqs = h->geom.max_seqs;
+  a.hq = h->cfg.num_q_heads;
+  a.group = h->cfg.num_q_heads / h->cfg.num_kv_heads;
+  a.hkv_inverse = h->geom.hkv > 1 ? (uint32_t)(((1ull << 32) + h->geom.hkv - 1) / h->geom.hkv) : 0;
+  a.scale = h->cfg.scale;
+  a.softcap = h->cfg.softcap;
+  l->esize = h->geom.esize;
+  l->tables.layer_window = h->d_window;
 }
 
-void fill_inline_windows(const mi355_attn* h, DecodeArgs* a) {
-  if (a->n_layers > kInlineLayers) return;
-  for (int i = 0; i < a->n_layers; ++i) a->inline_window[i] = h->window[a->layer_begin + i];
+// The windows of layers layer_begin .. layer_begin + n_layers - 1 and their partition sizes into the launch (reads
+// max_kv_len, num_splits and align), unless there are too many layers or different windows: then the kernels read the table in
+// memory.
+void fill_inline_windows(const mi355_attn* h, DecodeLaunch* l) {
+  if (l->n_layers > kInlineLayers) return;
+  auto& t = l->work.layers;
+  int windows = 0;
+  for (int i = 0; i < l->n_layers; ++i) {
+    const int window = h->window[l->args.layer_begin + i];
+    int w = 0;
+    while (w < windows && t.window[w] != window) ++w;
+    if (w == windows) {
+      if (windows == kDecodeWindows) return;
+      t.window[w] = window;
+      t.per[w] = decode_partition_tokens(l->max_kv_len, window, l->args.num_splits, l->args.align);
+      ++windows;
+    }
+    t.code[i >> 4] |= (uint32_t)w << (2 * (i & 15));
+  }
+  l->inline_layers = true;
 }
 
 // Raw projections of the one new token of every sequence (mi355_attn_decode_step): the decode kernel runs the
@@ -266,6 +291,38 @@ struct NewRows {
   const void* k;
   const void* v;
 };
+
+// The partitions of a decode launch by rule. `heads`: layers x sequences x KV heads; `block`: tokens a wave loads at a time.
+//
+// While every block of every sequence can have a wave of its own and every partition a compute unit, latency is all there
+// is: one partition of up to eight blocks (two for each of four waves; nothing to merge), else partitions of up to four
+// blocks (a wave each), so many that the merge still has its rows in one trip (32), or two blocks and up to 256 partitions
+// where the context needs more. One layer's step, 4 heads on 1, fp16, us, before this rule (64-token partitions, one up to
+// 512 tokens) / now: 300 tokens 11.3 / 8.1, 520 9.0 / 8.4, 1,152 10.6 / 8.8 (window 512: 9.2 / 7.8), 4,096 12.3 / 10.0,
+// 8,000 14.5 / 10.8; 8 sequences, one partition / a block each: 220 tokens 8.5 / 10.7, 380 11.3 / 10.9.
+//
+// Larger launches: about 512 workgroups, 1024 where sequences or layers see unequal lengths or the cache is float32 (16 layers x 64 sequences
+// are fastest without any split; one layer in 512 / 1024, us, decode and decode step: 64 sequences of 2,000, 8 heads on 2,
+// fp16 43.5 / 46.2 and 47.4 / 52.8, 40 of 3,000, 4 on 1, 23.1 / 24.5 and 24.1 / 26.5, 47 of 7,490, window 512, 13.9 / 14.5
+// and 15.5 / 17.1, 32 of 2,490, int8, 22.2 / 22.1 and 22.7 / 26.3, 61 ragged ones of up to 5,746 43.4 / 33.7, 11 of 3,874,
+// float32, 38.0 / 33.2; six layers x 4 sequences of 2,496, int8, five with a window of 512: 17.1 / 15.2), partitions of whole 64 tokens (4 layers x 15 float32 sequences of 3,170: 53 us in partitions of 176 tokens, 39 of 192), and one for
+// contexts of up to 512 tokens (64 sequences of 256 / 512 tokens, Hq8/Hkv2: 9.7 / 15.4 us against 11.0 / 16.1 split and
+// merged, 256 sequences 26.9 / 46.3 against 32.4 / 51.8).
+struct DecodeSplits { int count, align; };
+DecodeSplits choose_decode_splits(int max_len, int min_len, int widest, int narrowest, int heads, int block) {
+  const int blocks = (decode_span(max_len, widest, block) + block - 1) / block;
+  if (heads <= kLatencyWorkgroups) {
+    if (blocks <= 8) return {1, block};
+    const int few = std::min({32, blocks, kLatencyWorkgroups / heads});
+    if (blocks <= 4 * few) return {few, block};
+    const int many = std::min((blocks + 1) / 2, kLatencyWorkgroups / heads);
+    if (many > 32 && blocks <= 4 * many) return {many, block};
+  }
+  if (max_len <= 512) return {1, kTokenAlign};
+  const int most = decode_span(max_len, widest, 1), least = decode_span(min_len, narrowest, 1);
+  const int target = least * 4 < most * 3 || block == 16 ? 1024 : 512;
+  return {std::max(1, std::min({(target + heads - 1) / heads, (max_len + 63) / 64, 64})), kTokenAlign};
+}
 
 // no_alloc: the call may not allocate (mi355_attn_decode_noalloc): device pointers only, and the
 // partials go to this GPU's `scratch` instead of the handle's growable workspace.
@@ -331,20 +388,21 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
     max_len = whole->max_len;
     min_len = whole->min_len;
   }
-  if (num_splits == 0) {
-    // About 1024 workgroups (four waves per CU saturate HBM; measured: 30 layers x 2 KV heads at 4096 tokens
-    // run 8 % faster with 16-18 partitions than with 35, 16 layers x 64 sequences fastest without any split),
-    // partitions of >= 64 tokens.
-    const int rule_items = whole ? n_layers * whole->batch : items;
-    const int want = (1024 + rule_items * h->cfg.num_kv_heads - 1) / (rule_items * h->cfg.num_kv_heads);
-    num_splits = std::max(1, std::min({want, (max_len + 63) / 64, 64}));
-    // Contexts of up to 512 tokens: one partition, and with it no merge launch. Measured (one layer, fp16, Hq8/Hkv2,
-    // calls queued back to back): 1 sequence of 256 / 512 tokens 6.7 / 8.6 us against 9.9 / 9.8 us split and merged,
-    // 64 sequences 9.7 / 15.4 against 11.0 / 16.1 us, 256 sequences 26.9 / 46.3 against 32.4 / 51.8 us; from 640
-    // tokens on the split wins for small batches (1 sequence of 768 tokens: 10.9 against 9.8 us).
-    if (max_len <= 512) num_splits = 1;
+  int widest = h->window[layer_begin], narrowest = widest;  // windows of the layers (0: none, the widest of all)
+  for (int l = layer_begin + 1; l < layer_begin + n_layers; ++l) {
+    const int w = h->window[l];
+    if (w == 0 || (widest > 0 && w > widest)) widest = w;
+    if (w > 0 && (narrowest == 0 || w < narrowest)) narrowest = w;
   }
-  DecodeArgs a{};
+  int align = kTokenAlign;
+  if (num_splits == 0) {
+    const DecodeSplits splits = choose_decode_splits(max_len, min_len, widest, narrowest, n_layers * (whole ? whole->batch : batch) * h->cfg.num_kv_heads,
+                                                     decode_block_tokens(h->geom.esize));
+    num_splits = splits.count;
+    align = splits.align;
+  }
+  DecodeLaunch launch;
+  DecodeArgs& a = launch.args;
   const size_t slots = (size_t)items * h->cfg.num_q_heads * num_splits;
   if (no_alloc) {
     // the library's own choice of partitions is trimmed to the workspace; an explicit count is an error
@@ -362,7 +420,7 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   } else if (num_splits > 1) {
     if (int rc = ensure_workspace(h, slots, error_msg)) return rc;
   }
-  fill_decode_common(h, &a);
+  fill_decode_common(h, &launch);
   if (no_alloc) {
     float* const base = g_scratch_ptr[h->device];  // this GPU's copy of `scratch`
     a.ws_acc = base;
@@ -374,32 +432,31 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   if (int rc = stage_in(h, 0, q, io_bytes, &dq, error_msg)) return rc;
   if (new_rows) {
     const size_t kv_bytes = (size_t)batch * h->cfg.num_kv_heads * h->cfg.head_dim * io_size(h);
-    if (int rc = stage_in(h, 2, new_rows->k, kv_bytes, &a.pre_k, error_msg)) return rc;
-    if (int rc = stage_in(h, 3, new_rows->v, kv_bytes, &a.pre_v, error_msg)) return rc;
-    a.pre_q = dq;
+    if (int rc = stage_in(h, 2, new_rows->k, kv_bytes, &launch.pre.k, error_msg)) return rc;
+    if (int rc = stage_in(h, 3, new_rows->v, kv_bytes, &launch.pre.v, error_msg)) return rc;
+    launch.fused = true;
+    launch.pre.q = dq;
     const mi355_attn::LayerTransform& lt = h->transform[layer_begin];  // never set: a plain append
-    a.pre_constants = h->d_transform + (size_t)layer_begin * transform_floats(h->cfg.head_dim);
-    a.pre_rope = lt.rope;
-    a.pre_norm_q = lt.norm_q;
-    a.pre_norm_k = lt.norm_k;
-    a.pre_norm_v = lt.norm_v;
-    a.pre_q_scaled = lt.q_scaled;
-    a.pre_k_scaled = lt.k_scaled;
-    a.pre_eps = lt.eps;
-    a.pre_weight_offset = lt.weight_offset;
+    launch.pre.constants = h->d_transform + (size_t)layer_begin * transform_floats(h->cfg.head_dim);
+    launch.pre.rope = lt.rope;
+    launch.pre.norm_q = lt.norm_q;
+    launch.pre.norm_k = lt.norm_k;
+    launch.pre.norm_v = lt.norm_v;
+    launch.pre.q_scaled = lt.q_scaled;
+    launch.pre.k_scaled = lt.k_scaled;
+    launch.pre.eps = lt.eps;
+    launch.pre.weight_offset = lt.weight_offset;
   }
   if (int rc = stage_out_begin(h, 1, out, io_bytes, &dout, error_msg)) return rc;
   if (batch <= kInlineItems) {
-    a.inline_items = 1;
+    launch.inline_items = true;
     // dispatch order: longest sequence first (rows keep their places in q and out)
     int order[kInlineItems];
     for (int b = 0; b < batch; ++b) order[b] = b;
     std::stable_sort(order, order + batch, [&](int x, int y) { return kv_lens[x] > kv_lens[y]; });
     for (int j = 0; j < batch; ++j) {
       const int b = order[j];
-      a.inline_lens[j] = kv_lens[b];
-      a.inline_seq[j] = seq_ids ? seq_ids[b] : b;
-      a.inline_row[j] = b;
+      launch.work.item[j] = DecodeItem{(uint32_t)kv_lens[b] | (uint32_t)b << kDecodeLenBits, seq_ids ? seq_ids[b] : b};
     }
   } else {
     // lengths and slots of a larger batch go up through the pinned ring: a copy and, when the ring wraps, a wait
@@ -411,18 +468,31 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
                   "decode of %d sequences while the stream is being captured: more than %d sequences per call need "
                   "an upload that a capture cannot hold (capture calls of up to %d sequences)",
                   batch, kInlineItems, kInlineItems);
-    if (int rc = upload_items(h, seq_ids, kv_lens, batch, &a.kv_lens, &a.seq_ids, &a.rows, error_msg)) return rc;
+    if (int rc = upload_items(h, seq_ids, kv_lens, batch, &launch.tables.kv_lens, &launch.tables.seq_ids, &launch.tables.rows, error_msg)) return rc;
   }
   a.q = dq;
   a.out = dout;
   a.layer_begin = layer_begin;
-  a.n_layers = n_layers;
   a.batch = batch;
+  launch.n_layers = n_layers;
+  launch.max_kv_len = max_len;
+  launch.min_kv_len = min_len;
+  launch.widest_window = widest;
+  launch.rule_batch = whole ? whole->batch : batch;
+  // Partitions are rounded up, so fewer may cover the context than were asked for (4,096 tokens in 18: sixteen of 256): the
+  // launch has no workgroups for the others. (Their size stays what it is: any count in between gives the same.)
+  int used = 1;
+  for (int l = layer_begin; l < layer_begin + n_layers; ++l) {
+    const int window = h->window[l];
+    if (l > layer_begin && window == h->window[l - 1]) continue;
+    const int per = decode_partition_tokens(max_len, window, num_splits, align);
+    used = std::max(used, (decode_span(max_len, window, align) + per - 1) / per);
+  }
+  num_splits = used;
   a.num_splits = num_splits;
-  a.max_kv_len = max_len;
-  a.min_kv_len = min_len;
-  a.rule_batch = whole ? whole->batch : batch;
-  fill_inline_windows(h, &a);
+  a.align = align;
+  if (decode_merges_itself(n_layers, launch.rule_batch, a.hkv, num_splits)) a.tickets = h->d_tickets;
+  fill_inline_windows(h, &launch);
   bool scratch_fence = false;
   if (no_alloc && num_splits > 1) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -431,7 +501,7 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
     if (scratch_fence && g_scratch_used[h->device] && g_scratch_stream[h->device] != h->stream)
       HIP_OR_RETURN(hipStreamWaitEvent(h->stream, g_scratch_done[h->device], 0));
   }
-  HIP_OR_RETURN(launch_decode(a, h->cfg.kv_dtype, h->cfg.io_dtype, h->tuning, h->stream,
+  HIP_OR_RETURN(launch_decode(launch, h->cfg.kv_dtype, h->cfg.io_dtype, h->tuning, h->stream,
                               h->timing ? h->ev0 : nullptr, h->timing ? h->ev1 : nullptr));
   if (scratch_fence) {
     HIP_OR_RETURN(hipEventRecord(g_scratch_done[h->device], h->stream));
@@ -628,19 +698,22 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
     hipLaunchKernelGGL(iota_items_kernel, dim3((n + 255) / 256), dim3(256), 0, h->stream, lens, seqs, n, q_pos0,
                        seq);
     HIP_OR_RETURN(hipGetLastError());
-    DecodeArgs a{};
-    fill_decode_common(h, &a);
+    DecodeLaunch launch;
+    DecodeArgs& a = launch.args;
+    fill_decode_common(h, &launch);
     a.q = dq;
     a.out = dout;
-    a.kv_lens = lens;
-    a.seq_ids = seqs;
+    launch.tables.kv_lens = lens;
+    launch.tables.seq_ids = seqs;
     a.layer_begin = layer_begin;
-    a.n_layers = n_layers;
     a.batch = n;
     a.num_splits = 1;
-    a.max_kv_len = q_pos0 + n;
-    fill_inline_windows(h, &a);
-    HIP_OR_RETURN(launch_decode(a, h->cfg.kv_dtype, h->cfg.io_dtype, h->tuning, h->stream, e0, e1));
+    a.align = kTokenAlign;
+    launch.n_layers = n_layers;
+    launch.max_kv_len = q_pos0 + n;
+    launch.rule_batch = n;
+    fill_inline_windows(h, &launch);
+    HIP_OR_RETURN(launch_decode(launch, h->cfg.kv_dtype, h->cfg.io_dtype, h->tuning, h->stream, e0, e1));
   }
   h->timed = h->timing;
   return stage_out_end(h, 1, out, io_bytes, error_msg);
@@ -766,16 +839,17 @@ int mi355_attn_create(const mi355_attn_config* c, mi355_attn** out, char** error
   if ((e = hipMemcpyAsync(h->d_window, h->window.data(), sizeof(int32_t) * c->num_layers, hipMemcpyHostToDevice,
                           h->stream)) != hipSuccess)
     return bail(MI355_ATTN_INTERNAL, "window upload", e);
-  if ((e = hipMalloc(&h->d_sched, sizeof(int32_t) * (kPrefillSchedInts + 1))) != hipSuccess)  // (+ the stream probe's sink word)
-    return bail(MI355_ATTN_RESOURCE_EXHAUSTED, "prefill queue counters", e);
+  if ((e = hipMalloc(&h->d_sched, sizeof(int32_t) * (kSchedInts + kDecodeTickets))) != hipSuccess)
+    return bail(MI355_ATTN_RESOURCE_EXHAUSTED, "queue counters and tickets", e);
+  h->d_tickets = reinterpret_cast<uint32_t*>(h->d_sched + kSchedInts);
   h->transform.assign(c->num_layers, mi355_attn::LayerTransform{});
   const size_t transform_bytes = sizeof(float) * (size_t)c->num_layers * transform_floats(c->head_dim);
   if ((e = hipMalloc(&h->d_transform, transform_bytes)) != hipSuccess)
     return bail(MI355_ATTN_RESOURCE_EXHAUSTED, "layer transform constants", e);
   if ((e = hipMemsetAsync(h->d_transform, 0, transform_bytes, h->stream)) != hipSuccess)
     return bail(MI355_ATTN_INTERNAL, "layer transform clear", e);
-  if ((e = hipMemsetAsync(h->d_sched, 0, sizeof(int32_t) * kPrefillSchedInts, h->stream)) != hipSuccess)
-    return bail(MI355_ATTN_INTERNAL, "prefill queue clear", e);
+  if ((e = hipMemsetAsync(h->d_sched, 0, sizeof(int32_t) * (kSchedInts + kDecodeTickets), h->stream)) != hipSuccess)
+    return bail(MI355_ATTN_INTERNAL, "queue counters and tickets clear", e);
   if (c->kv_dtype == MI355_ATTN_I8 || c->kv_dtype == MI355_ATTN_F32) {
     // the row-wise prefill path's item list (these caches may take that path inside a captured graph, where nothing
     // can be allocated)

@@ -21,18 +21,31 @@ namespace mi355 {
 
 constexpr int kRowD = 256;
 
+// Two consecutive elements of type DT as they come from memory. Loads that stand behind a condition keep their values in
+// this form until all of them are on their way: a conversion behind the same condition would be a wait for its load.
 template <int DT>
-__device__ __forceinline__ void load_pair(const void* base, int64_t elem, float& a, float& b) {
+struct RawPair { using type = uint32_t; };
+template <>
+struct RawPair<kF32> { using type = u2; };
+template <int DT>
+__device__ __forceinline__ typename RawPair<DT>::type load_raw_pair(const void* base, int64_t elem) {
+  constexpr int ESZ = DT == kF32 ? 4 : 2;
+  return *reinterpret_cast<const typename RawPair<DT>::type*>(reinterpret_cast<const uint8_t*>(base) + elem * ESZ);
+}
+template <int DT>
+__device__ __forceinline__ void unpack_pair(typename RawPair<DT>::type x, float& a, float& b) {
   if constexpr (DT == kF32) {
-    const float2 x = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(base) + elem);
-    a = x.x; b = x.y;
+    a = __uint_as_float(x[0]); b = __uint_as_float(x[1]);
   } else if constexpr (DT == kF16) {
-    const h2 x = *reinterpret_cast<const h2*>(reinterpret_cast<const _Float16*>(base) + elem);
-    a = (float)x[0]; b = (float)x[1];
+    const h2 h = bit_cast<h2>(x);
+    a = (float)h[0]; b = (float)h[1];
   } else {
-    const uint32_t x = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(base) + elem);
     a = __uint_as_float(x << 16); b = __uint_as_float(x & 0xffff0000u);
   }
+}
+template <int DT>
+__device__ __forceinline__ void load_pair(const void* base, int64_t elem, float& a, float& b) {
+  unpack_pair<DT>(load_raw_pair<DT>(base, elem), a, b);
 }
 
 // Two consecutive elements of type DT at byte address p (4- or 8-byte aligned).
@@ -127,11 +140,11 @@ __device__ __forceinline__ const float* row_weights(const float* constants, int 
   return nullptr;
 }
 
-// The transformed key (is_v 0) or value (is_v 1) row of token t into its plane; `scales` = the plane's
-// [256] dequantisation scales (int8 cache only). LINEAR: `plane` is a buffer of 256 elements instead and
-// element d of the row goes to element d of the buffer, in the same element format.
+// The transformed key (is_v 0) or value (is_v 1) row of token t into its plane; s0, s1: the plane's
+// dequantisation scales of the lane's channels 2l, 2l+1 and 128+2l, 128+2l+1 (int8 cache only). LINEAR: `plane` is a
+// buffer of 256 elements instead and element d of the row goes to element d of the buffer, in the same element format.
 template <int KV, bool LINEAR = false>
-__device__ __forceinline__ void store_cache_row(uint8_t* plane, const float* scales, int is_v, int t,
+__device__ __forceinline__ void store_cache_row(uint8_t* plane, float2 s0, float2 s1, int is_v, int t,
                                                 const float (&x)[4], int lane) {
   constexpr int ESZ = KV == kF32 ? 4 : (KV == kI8 ? 1 : 2);
   constexpr int EPC = 16 / ESZ;
@@ -143,8 +156,6 @@ __device__ __forceinline__ void store_cache_row(uint8_t* plane, const float* sca
     return LINEAR ? (int64_t)d * ESZ : mi355::v_elem_offset(tt, d, kRowD, ESZ);
   };
   if constexpr (KV == kI8) {
-    const float2 s0 = *reinterpret_cast<const float2*>(scales + d0);
-    const float2 s1 = *reinterpret_cast<const float2*>(scales + d1);
     const int qv[4] = {quantise(x[0], s0.x), quantise(x[1], s0.y), quantise(x[2], s1.x), quantise(x[3], s1.y)};
     if (!is_v) {
       *reinterpret_cast<uint16_t*>(plane + k_chunk_offset(t, d0 / EPC, kRowD, ESZ) + d0 % EPC) =
@@ -168,6 +179,18 @@ __device__ __forceinline__ void store_cache_row(uint8_t* plane, const float* sca
       store_value<KV>(plane + v_elem_offset(t, d1 + 1, kRowD, ESZ), x[3]);
     }
   }
+}
+
+// The same with the scales where they lie (`scales`: the plane's [256]).
+template <int KV, bool LINEAR = false>
+__device__ __forceinline__ void store_cache_row(uint8_t* plane, const float* scales, int is_v, int t,
+                                                const float (&x)[4], int lane) {
+  float2 s0 = {0.f, 0.f}, s1 = {0.f, 0.f};
+  if constexpr (KV == kI8) {
+    s0 = *reinterpret_cast<const float2*>(scales + 2 * lane);
+    s1 = *reinterpret_cast<const float2*>(scales + kRowD / 2 + 2 * lane);
+  }
+  store_cache_row<KV, LINEAR>(plane, s0, s1, is_v, t, x, lane);
 }
 
 }  // namespace mi355

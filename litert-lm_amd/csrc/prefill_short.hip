@@ -123,10 +123,10 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
   for (int i = 0; i < NL; ++i) acc[i] = f4{0.f, 0.f, 0.f, 0.f};
   const float sc = a.scale, softcap = a.softcap;
   while (blk < blk_end) {
-    int qi = lane;  // opaque, so that the operand reads stay in the loop (hoisted they would fill the registers)
-    asm volatile("" : "+v"(qi));
+    int q_off = lane * 16;  // opaque, so that the operand reads stay in the loop (hoisted they would fill the registers)
+    asm volatile("" : "+v"(q_off));
     f4 s[NT];
-    qk_block<KV, D>(kreg, sm_q, qi, s);
+    qk_block<KV, D>(kreg, smem + q_off, s);
     const int nxt = blk + NW;
     if (nxt < blk_end) load_plane_block<D, kCachedLoad>(kreg, krsrc, nxt * kBlockBytes, lane * 16);
     if constexpr (CAP) {
