@@ -232,20 +232,32 @@ constexpr int kPrefillQueues = 2;                     // ticket queues; workgrou
 constexpr int kPrefillOrderUnits = 128;               // entries of PrefillArgs::unit_order
 constexpr int kPrefillSchedInts = kPrefillQueues + 1;  // + count of workgroups that are done
 
-// Arguments of prefill_short_kernel (passed by value).
+// Arguments of prefill_short_kernel (passed by value, with the windows of the call's layers behind them).
 struct PrefillShortArgs {
   const void* q;  // [n_layers][n][hq][D] io dtype
   void* out;
   const uint8_t* cache;
   const float* scales;  // int8 cache only
-  CacheGeom geom;
+  float* ws_acc;        // parts of split tiles: [unit][tile][part][16 columns] x D and x 2 floats, and a ticket per (unit, tile)
+  float* ws_ml;         // that counts key blocks, all zero between launches (used only where parts > 1)
+  uint32_t* tickets;
+  int64_t plane_bytes;  // as in CacheGeom
+  int32_t hkv, max_seqs;
   int32_t hq, group;
-  int32_t layer_begin, n_layers;
-  int32_t seq, q_pos0, n;
-  int32_t rows_log2;  // positions per workgroup (log2): prefill_short_rows_log2(group)
+  int32_t layer_begin, seq;
+  int32_t q_pos0, n;
+  int32_t rows_log2;    // positions per workgroup (log2): prefill_short_rows_log2(group)
+  uint32_t hkv_inverse; // 2^32 / hkv, rounded up; 0 for one KV head
+  int32_t tiles;        // of a unit (layer x KV head)
+  int32_t parts;        // workgroups that share the key blocks of a tile, at most
+  uint32_t parts_inverse;  // 2^32 / parts, rounded up; 0 for one
   float scale, softcap;
-  int32_t window[kInlineLayers];  // of layers layer_begin .. layer_begin + n_layers - 1
 };
+template <int LAYERS>
+struct PrefillWindows { int32_t of[LAYERS]; };  // of layers layer_begin .. layer_begin + n_layers - 1
+constexpr int kShortParts = 8;         // PrefillShortArgs::parts, at most
+constexpr int kShortPartSlots = 256;   // unit x tile x part of a call whose tiles are split, at most
+constexpr int kShortPartRows = 16;     // rows (columns of the tile) of a part
 
 struct KvCopyArgs {
   uint8_t* cache;

@@ -87,8 +87,11 @@ hipError_t launch_prefill(const PrefillArgs& args, int kv_dtype, int io_dtype, P
 int prefill_short_rows_log2(int group);  // log2 of the positions a workgroup takes
 // The rule: window[0 .. n_layers) are the windows of the call's layers. Host only.
 bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, int n_layers, int q_pos0, int n);
-hipError_t launch_prefill_short(const PrefillShortArgs& args, int kv_dtype, int io_dtype, hipStream_t stream,
-                                hipEvent_t ev0, hipEvent_t ev1);
+// (window: of the call's layers. Fills in what the launch decides: rows_log2, tiles, parts and the inverses.)
+hipError_t launch_prefill_short(PrefillShortArgs args, const int32_t* window, int n_layers, int kv_dtype, int io_dtype,
+                                hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
+// Parts that the tiles of a call are cut into: `wgs` tiles in all, the longest of `most` key blocks.
+int prefill_short_parts(int kv_dtype, long wgs, int most);
 
 // Scatter n boundary-layout rows into the cache planes / gather them back.
 hipError_t launch_kv_append(const KvCopyArgs& args, hipStream_t stream);

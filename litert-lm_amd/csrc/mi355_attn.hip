@@ -94,7 +94,7 @@ struct mi355_attn {
   float* scales = nullptr;
   int32_t* d_window = nullptr;
   int32_t* d_sched = nullptr;  // prefill work-queue counters
-  uint32_t* d_tickets = nullptr;  // tickets of decode launches that merge their own partials (behind the counters)
+  uint32_t* d_tickets = nullptr;  // tickets of launches that merge their own partials, all zero between launches (behind the counters)
   PrefillPlans pf_plans;       // prefill work plans by launch shape
   float* d_pf_acc = nullptr;   // prefill key split: parts of split tiles, allocated on first use
   float* d_pf_ml = nullptr;
@@ -117,6 +117,7 @@ struct mi355_attn {
   std::vector<LayerTransform> transform;
   std::vector<int32_t> window;
   std::vector<int32_t> filled;  // [layer][seq] rows written since the last reset
+  float* d_short_ws = nullptr;  // prefill of short calls: parts of split tiles
   // split-KV workspace
   float* ws_acc = nullptr;
   float* ws_ml = nullptr;
@@ -564,19 +565,21 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
     a.out = dout;
     a.cache = h->cache;
     a.scales = h->scales;
-    a.geom = h->geom;
+    a.ws_acc = h->d_short_ws;
+    a.ws_ml = h->d_short_ws + (size_t)kShortPartSlots * kShortPartRows * h->cfg.head_dim;
+    a.tickets = h->d_tickets;
+    a.plane_bytes = h->geom.plane_bytes;
+    a.hkv = h->geom.hkv;
+    a.max_seqs = h->geom.max_seqs;
     a.hq = h->cfg.num_q_heads;
     a.group = h->cfg.num_q_heads / h->cfg.num_kv_heads;
     a.layer_begin = layer_begin;
-    a.n_layers = n_layers;
     a.seq = seq;
     a.q_pos0 = q_pos0;
     a.n = n;
-    a.rows_log2 = prefill_short_rows_log2(a.group);
     a.scale = h->cfg.scale;
     a.softcap = h->cfg.softcap;
-    for (int i = 0; i < n_layers; ++i) a.window[i] = h->window[layer_begin + i];
-    HIP_OR_RETURN(launch_prefill_short(a, h->cfg.kv_dtype, h->cfg.io_dtype, h->stream, e0, e1));
+    HIP_OR_RETURN(launch_prefill_short(a, h->window.data() + layer_begin, n_layers, h->cfg.kv_dtype, h->cfg.io_dtype, h->stream, e0, e1));
     h->timed = h->timing;
     return stage_out_end(h, 1, out, io_bytes, error_msg);
   }
@@ -842,6 +845,10 @@ int mi355_attn_create(const mi355_attn_config* c, mi355_attn** out, char** error
   if ((e = hipMalloc(&h->d_sched, sizeof(int32_t) * (kSchedInts + kDecodeTickets))) != hipSuccess)
     return bail(MI355_ATTN_RESOURCE_EXHAUSTED, "queue counters and tickets", e);
   h->d_tickets = reinterpret_cast<uint32_t*>(h->d_sched + kSchedInts);
+  static_assert(kShortPartSlots <= kDecodeTickets, "short prefill calls and decode use the same tickets");
+  // (4 MiB, here and not on first use: a call that is recorded into a graph then runs as it does eagerly)
+  if ((e = hipMalloc(&h->d_short_ws, sizeof(float) * kShortPartSlots * kShortPartRows * (size_t)(c->head_dim + 2))) != hipSuccess)
+    return bail(MI355_ATTN_RESOURCE_EXHAUSTED, "parts of short prefill calls", e);
   h->transform.assign(c->num_layers, mi355_attn::LayerTransform{});
   const size_t transform_bytes = sizeof(float) * (size_t)c->num_layers * transform_floats(c->head_dim);
   if ((e = hipMalloc(&h->d_transform, transform_bytes)) != hipSuccess)
@@ -886,6 +893,7 @@ void mi355_attn_destroy(mi355_attn* h) {
   if (h->d_q_stage) (void)hipFree(h->d_q_stage);
   if (h->d_kv_stage) (void)hipFree(h->d_kv_stage);
   if (h->d_transform) (void)hipFree(h->d_transform);
+  if (h->d_short_ws) (void)hipFree(h->d_short_ws);
   if (h->ws_acc) (void)hipFree(h->ws_acc);
   if (h->ws_ml) (void)hipFree(h->ws_ml);
   if (h->d_ring) (void)hipFree(h->d_ring);

@@ -6,7 +6,8 @@
 // from the planes straight into registers (the decode kernel's loads and products, kv_blocks.h), and merge through
 // LDS at the end. Against the tiled kernels of prefill_attn.hip, where a workgroup takes 32 positions and a short
 // call is cut over the keys into work items whose float32 parts travel through HBM to a merge launch, this has 8
-// times as many workgroups of an eighth of the keys per wave, no parts in HBM and one launch.
+// times as many workgroups of an eighth of the keys per wave and one launch; a call that leaves half of the compute units
+// without a tile cuts its tiles over the keys too, into parts that the launch merges itself.
 //
 // Bound: a 16-column tile reads 32 KiB of K and V per 32 matrix instructions, so beyond one tile per compute unit
 // the path from the L2 (64 bytes per clock and compute unit) sets the time, and the tiled kernels, which feed 128
@@ -20,6 +21,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_params.h"
 #include "kernels.h"
@@ -35,6 +37,8 @@ constexpr int kAccStride = 4;  // floats of padding per accumulator row in LDS (
 // Launches of up to this many workgroups use eight waves each (one workgroup a compute unit), larger ones four.
 constexpr long kWideWorkgroups = 256;
 
+constexpr int kMinPartBlocks = 4;  // key blocks of a part of a split tile, at least
+
 int short_tiles(int q_pos0, int n, int rows_log2) { return ((q_pos0 + n - 1) >> rows_log2) - (q_pos0 >> rows_log2) + 1; }
 
 template <int KV, int D>
@@ -49,8 +53,12 @@ constexpr int lds_bytes() {
 // NW waves per workgroup, eight waves a compute unit either way, two per SIMD, which is all that 256 registers per lane
 // leave room for; but for a float32 cache in launches of four waves, whose 81.5 KiB of LDS let one workgroup run on a
 // compute unit instead of two.
-template <int KV, int IO, int D, int NW, bool CAP>
-__global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const PrefillShortArgs a) {
+//
+// A call of few tiles cuts each of them into up to `parts` stretches of its key blocks, a workgroup each (grid z). A part
+// leaves its unnormalised sums, maxima and totals in the workspace by device-scope stores, counts its blocks on the tile's
+// ticket, and the workgroup whose count completes the tile adds the parts up in order (as decode_attn_kernel does).
+template <int KV, int IO, int D, int NW, bool CAP, int LAYERS>
+__global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const PrefillShortArgs a, const PrefillWindows<LAYERS> windows) {
   using io_t = typename IoT<IO>::type;
   constexpr int VB = KvT<KV>::VB, NT = VB / 16, NL = D / 16;
   constexpr int NQ = query_steps<KV, D>();
@@ -63,45 +71,70 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;
-  // Grid (layer x KV head, tile): units vary fastest, so that tiles are dispatched from the longest key range down.
+  // Grid (layer x KV head, tile, part): units vary fastest, so that tiles are dispatched from the longest key range down.
+  // Everything in front of the first load comes in one round of scalar loads (left alone, each is sunk to its use).
   const int unit = blockIdx.x;
-  const int li = unit / a.geom.hkv, kvh = unit - li * a.geom.hkv;
-  const int layer = a.layer_begin + li;
-  const int window = a.window[li];
-  const int tile = (int)gridDim.y - 1 - (int)blockIdx.y;
-  const int rows_log2 = a.rows_log2, rows = 1 << rows_log2;
-  const int pos_end = a.q_pos0 + a.n;
-  const int tile_pos = ((a.q_pos0 >> rows_log2) + tile) << rows_log2;  // may lie in front of q_pos0, rows behind pos_end
-  const int first_pos = max(tile_pos, a.q_pos0), last_pos = min(tile_pos + rows, pos_end) - 1;
+  int hkv = a.hkv, max_seqs = a.max_seqs, hq = a.hq, group = a.group, layer_begin = a.layer_begin, seq = a.seq;
+  int q_pos0 = a.q_pos0, rows_n = a.n, rows_log2 = a.rows_log2, tiles = a.tiles;
+  uint32_t hkv_inverse = a.hkv_inverse, parts_inverse = a.parts_inverse;
+  int64_t plane_bytes = a.plane_bytes;
+  const uint8_t* cache = a.cache;
+  const float* scales = a.scales;
+  const void* q = a.q;
+  // (with one layer its window comes in the same round, else behind the unit's layer)
+  int window = LAYERS == 1 ? windows.of[0] : 0;
+  asm volatile("" : "+s"(hkv), "+s"(max_seqs), "+s"(hq), "+s"(group), "+s"(layer_begin), "+s"(seq), "+s"(q_pos0), "+s"(rows_n),
+               "+s"(rows_log2), "+s"(tiles), "+s"(hkv_inverse), "+s"(parts_inverse), "+s"(plane_bytes), "+s"(cache), "+s"(scales),
+               "+s"(q), "+s"(window));
+  const int li = LAYERS == 1 ? 0 : (hkv_inverse ? (int)__umulhi(unit, hkv_inverse) : unit), kvh = unit - li * hkv;
+  if constexpr (LAYERS > 1) window = windows.of[li];
+  const int layer = layer_begin + li;
+  const int tile = tiles - 1 - (int)blockIdx.y;
+  const int rows = 1 << rows_log2;
+  const int pos_end = q_pos0 + rows_n;
+  const int tile_pos = ((q_pos0 >> rows_log2) + tile) << rows_log2;  // may lie in front of q_pos0, rows behind pos_end
+  const int first_pos = max(tile_pos, q_pos0), last_pos = min(tile_pos + rows, pos_end) - 1;
   const int lo_first = window > 0 ? max(0, first_pos - window + 1) : 0;
   const int lo_last = window > 0 ? max(0, last_pos - window + 1) : 0;
-  const int blk0 = lo_first / VB, blk_end = last_pos / VB + 1;
+  int blk0 = lo_first / VB, blk_end = last_pos / VB + 1;
+  // this part of the tile's blocks
+  const int tile_blocks = blk_end - blk0;
+  int per_part = tile_blocks;
+  if (parts_inverse) {
+    // (ceil(blocks / parts) through the host's inverse, exact for what a plane holds)
+    per_part = max(kMinPartBlocks, (int)__umulhi(tile_blocks + a.parts - 1, parts_inverse));
+    blk0 += (int)blockIdx.z * per_part;
+    blk_end = min(blk_end, blk0 + per_part);
+    if (blk0 >= blk_end) return;  // (uniform over the workgroup)
+  }
 
   // this lane's column: head and position (columns without a row of the call hold zero queries and are not stored)
   const int head = c >> rows_log2;  // column = head * rows + row, so that a row's heads need no division
   const int pos = tile_pos + (c & (rows - 1));
-  const bool live = head < a.group && pos >= first_pos && pos <= last_pos;
+  const bool live = head < group && pos >= first_pos && pos <= last_pos;
   const int vlo = window > 0 ? max(0, pos - window + 1) : 0;
-  const int64_t row = live ? pos - a.q_pos0 : 0;
-  const int64_t q_elem = (((int64_t)li * a.n + row) * a.hq + kvh * a.group + (live ? head : 0)) * D;
+  const int64_t row = live ? pos - q_pos0 : 0;
+  const int64_t q_elem = (((int64_t)li * rows_n + row) * hq + kvh * group + (live ? head : 0)) * D;
 
-  const uint8_t* kplane = a.cache + a.geom.plane_offset(layer, a.seq, kvh, 0);
+  const uint8_t* kplane = cache + ((((int64_t)layer * max_seqs + seq) * hkv + kvh) * 2) * plane_bytes;  // geom.plane_offset
+  const float* ks = KV == kI8 ? scales + (((int64_t)layer * max_seqs + seq) * 2 * hkv + kvh) * D : nullptr;  // geom.scale_offset
   int blk = blk0 + wave;
   // (a wave without a block has a resource of no bytes: its first loads return zeros without a trip to memory; behind a
   // branch, the wait for the queries would have to be a wait for everything)
-  const int64_t streamed = blk < blk_end ? a.geom.plane_bytes : 0;
+  const int64_t streamed = blk < blk_end ? plane_bytes : 0;
   const __amdgpu_buffer_rsrc_t krsrc = plane_resource(kplane, streamed);
-  const __amdgpu_buffer_rsrc_t vrsrc = plane_resource(kplane + a.geom.plane_bytes, streamed);
+  const __amdgpu_buffer_rsrc_t vrsrc = plane_resource(kplane + plane_bytes, streamed);
 
-  // This wave's share of the query operands goes first, then its first K and V blocks: the wait for the former leaves
-  // the latter under way. (Queries that are converted on the way would be waited for before the blocks are asked for:
-  // then the blocks go first.)
+  // This wave's share of the query operands goes first, then its first K block: the wait for the former leaves the latter
+  // under way. (Queries that are converted on the way would be waited for before the block is asked for: then the block goes
+  // first.) The V block is requested behind the barrier that the queries need: the compute unit takes 16 cycles for a load
+  // of 1 KiB, so the V blocks of eight waves are a microsecond in which no wave could reach the barrier (26 layers of 1,024
+  // rows in turn: 410 us with both blocks in front of it, 390 so).
   static_assert(NQ % NW == 0, "every wave stages the same number of operands");
   constexpr int kQPerWave = NQ / NW;
   u4 qw[kQPerWave];
   auto load_queries = [&]() {
-    const float* ks = KV == kI8 ? a.scales + a.geom.scale_offset(layer, a.seq, 0, kvh) : nullptr;
-    const io_t* qrow = reinterpret_cast<const io_t*>(a.q) + q_elem;
+    const io_t* qrow = reinterpret_cast<const io_t*>(q) + q_elem;
 #pragma unroll
     for (int s = 0; s < kQPerWave; ++s) qw[s] = q_operand<KV, IO, D>(qrow, ks, wave * kQPerWave + s, g);
   };
@@ -109,13 +142,13 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
   __builtin_amdgcn_sched_barrier(0);
   u4 kreg[NL], vreg[NL];
   load_plane_block<D, kCachedLoad>(kreg, krsrc, blk * kBlockBytes, lane * 16);
-  load_plane_block<D, kCachedLoad>(vreg, vrsrc, blk * kBlockBytes, lane * 16);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (KV != IO) load_queries();
 #pragma unroll
   for (int s = 0; s < kQPerWave; ++s) sm_q[(wave * kQPerWave + s) * 64 + lane] = live ? qw[s] : u4{0, 0, 0, 0};
-  // (a barrier for LDS alone: __syncthreads() would also wait for the blocks under way)
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  lds_barrier();  // (__syncthreads() would also wait for the blocks under way)
+  load_plane_block<D, kCachedLoad>(vreg, vrsrc, blk * kBlockBytes, lane * 16);
+  __builtin_amdgcn_sched_barrier(0);
 
   float m_run = -INFINITY, l_run = 0.f;
   f4 acc[NL];
@@ -181,8 +214,9 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
   float l_tot = wave_xor_add<16>(l_run);
   l_tot = wave_xor_add<32>(l_tot);
 
-  // Merge the waves that had a block: accumulators and (max, sum) through LDS, then a wave per column and 4 channels
-  // per lane, so that whole rows leave.
+  // Merge the waves that had a block: accumulators and (max, sum) through LDS, then kCols / NW columns a wave with 4 channels
+  // per lane, so that whole rows leave. All LDS reads of a column go out together: one after the other, wave by wave, they
+  // were 2 us of a 10 us launch.
   const int nw = min(NW, blk_end - blk0);
   if (wave < nw) {
     float* dst = sm_acc + (wave * kCols + c) * (D + kAccStride) + 4 * g;
@@ -190,60 +224,156 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
     for (int db = 0; db < NL; ++db) *reinterpret_cast<f4*>(dst + 16 * db) = acc[db];
     if (g == 0) sm_ml[wave * kCols + c] = float2{m_run, l_tot};
   }
-  __syncthreads();
+  f4 vscale = {1.f, 1.f, 1.f, 1.f};
+  if constexpr (KV == kI8) vscale = *reinterpret_cast<const f4*>(ks + hkv * D + 4 * lane);
+  lds_barrier();
+  constexpr int kColsPerWave = kCols / NW;
+  f4 A[kColsPerWave];
+  float M[kColsPerWave], L[kColsPerWave];
+  // (all: every wave had a block. Conditions around the reads, or idle waves that bring zeros, would cost the others more)
+  auto merge_column = [&](int k, auto all) {
+    constexpr bool kAll = decltype(all)::value;
+    const int col = k * NW + wave;
+    const float2* mlp = sm_ml + col;
+    const float* accp = sm_acc + col * (D + kAccStride) + 4 * lane;
+    float2 ml[NW];
+    f4 v[NW];
+    if constexpr (kAll) {
 #pragma unroll
-  for (int k = 0; k < kCols / NW; ++k) {
+      for (int w = 0; w < NW; ++w) {
+        ml[w] = mlp[w * kCols];
+        v[w] = *reinterpret_cast<const f4*>(accp + w * kCols * (D + kAccStride));
+      }
+    }
+    M[k] = -INFINITY;
+#pragma unroll kAll ? NW : 1
+    for (int w = 0; w < (kAll ? NW : nw); ++w) M[k] = fmaxf(M[k], kAll ? ml[w].x : mlp[w * kCols].x);
+    const float m_use = (M[k] == -INFINITY) ? 0.f : M[k];
+    A[k] = f4{0.f, 0.f, 0.f, 0.f};
+    L[k] = 0.f;
+#pragma unroll kAll ? NW : 1
+    for (int w = 0; w < (kAll ? NW : nw); ++w) {
+      const float2 x = kAll ? ml[w] : mlp[w * kCols];
+      const f4 y = kAll ? v[w] : *reinterpret_cast<const f4*>(accp + w * kCols * (D + kAccStride));
+      const float wgt = fast_exp2(x.x - m_use);
+      A[k] += wgt * y;
+      L[k] += wgt * x.y;
+    }
+  };
+  if (nw == NW) {
+#pragma unroll
+    for (int k = 0; k < kColsPerWave; ++k) merge_column(k, std::true_type{});
+  } else {
+#pragma unroll
+    for (int k = 0; k < kColsPerWave; ++k) merge_column(k, std::false_type{});
+  }
+  if (per_part < tile_blocks) {
+    // a part: its columns to the workspace, and the last part of the tile adds them up
+    const int64_t slot0 = ((int64_t)unit * tiles + tile) * a.parts;
+    const __amdgpu_buffer_rsrc_t acc_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(a.ws_acc + slot0 * (kCols * D), 0, a.parts * (kCols * D * 4), 0x00020000);
+    const __amdgpu_buffer_rsrc_t ml_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(a.ws_ml + slot0 * (kCols * 2), 0, a.parts * (kCols * 8), 0x00020000);
+#pragma unroll
+    for (int k = 0; k < kColsPerWave; ++k) {
+      const int at = (int)blockIdx.z * kCols + k * NW + wave;
+      __builtin_amdgcn_raw_buffer_store_b128(bit_cast<u4>(A[k]), acc_rsrc, at * (D * 4) + lane * 16, 0, kDeviceScope);
+      if (lane == 0) __builtin_amdgcn_raw_buffer_store_b64(u2{__float_as_uint(M[k]), __float_as_uint(L[k])}, ml_rsrc, at * 8, 0, kDeviceScope);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    uint32_t* const sm_last = reinterpret_cast<uint32_t*>(smem);
+    if (threadIdx.x == 0) {
+      uint32_t* ticket = a.tickets + unit * tiles + tile;
+      const uint32_t mine = blk_end - blk0;
+      const uint32_t before = __hip_atomic_fetch_add(ticket, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const bool last = before + mine == (uint32_t)tile_blocks;
+      if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+      *sm_last = last;
+    }
+    lds_barrier();
+    if (!__builtin_amdgcn_readfirstlane((int)*sm_last)) return;
+    f4 v[kColsPerWave][kShortParts];
+    u2 ml[kColsPerWave][kShortParts];
+#pragma unroll
+    for (int k = 0; k < kColsPerWave; ++k)
+#pragma unroll
+      for (int p = 0; p < kShortParts; ++p) {
+        // (a part that does not exist is read as zeros behind the resource's end, and weighs 0)
+        const int at = p * per_part < tile_blocks ? p * kCols + k * NW + wave : kShortParts * kCols;
+        ml[k][p] = __builtin_amdgcn_raw_buffer_load_b64(ml_rsrc, at * 8, 0, kDeviceScope);
+        v[k][p] = bit_cast<f4>(__builtin_amdgcn_raw_buffer_load_b128(acc_rsrc, at * (D * 4) + lane * 16, 0, kDeviceScope));
+      }
+#pragma unroll
+    for (int k = 0; k < kColsPerWave; ++k) {
+      float m[kShortParts];
+      M[k] = -INFINITY;
+#pragma unroll
+      for (int p = 0; p < kShortParts; ++p) {
+        m[p] = p * per_part < tile_blocks ? __uint_as_float(ml[k][p][0]) : -INFINITY;
+        M[k] = fmaxf(M[k], m[p]);
+      }
+      const float m_use = (M[k] == -INFINITY) ? 0.f : M[k];
+      A[k] = f4{0.f, 0.f, 0.f, 0.f};
+      L[k] = 0.f;
+#pragma unroll
+      for (int p = 0; p < kShortParts; ++p) {
+        const float wgt = fast_exp2(m[p] - m_use);
+        A[k] += wgt * v[k][p];
+        L[k] += wgt * __uint_as_float(ml[k][p][1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kColsPerWave; ++k) {
     const int col = k * NW + wave;
     const int h = col >> rows_log2, p = tile_pos + (col & (rows - 1));
-    if (h >= a.group || p < first_pos || p > last_pos) continue;  // (uniform over the wave)
-    float M = -INFINITY;
-    for (int w = 0; w < nw; ++w) M = fmaxf(M, sm_ml[w * kCols + col].x);
-    const float m_use = (M == -INFINITY) ? 0.f : M;
-    f4 A = {0.f, 0.f, 0.f, 0.f};
-    float L = 0.f;
-    for (int w = 0; w < nw; ++w) {
-      const float2 ml = sm_ml[w * kCols + col];
-      const float wgt = fast_exp2(ml.x - m_use);
-      A += wgt * *reinterpret_cast<const f4*>(sm_acc + (w * kCols + col) * (D + kAccStride) + 4 * lane);
-      L += wgt * ml.y;
-    }
+    if (h >= group || p < first_pos || p > last_pos) continue;  // (uniform over the wave)
     f4 o;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = L > 0.f ? A[e] / L : 0.f;
-    if constexpr (KV == kI8)
-      o *= *reinterpret_cast<const f4*>(a.scales + a.geom.scale_offset(layer, a.seq, 1, kvh) + 4 * lane);
-    io_t* orow = reinterpret_cast<io_t*>(a.out) + (((int64_t)li * a.n + (p - a.q_pos0)) * a.hq + kvh * a.group + h) * D + 4 * lane;
+    for (int e = 0; e < 4; ++e) o[e] = L[k] > 0.f ? A[k][e] / L[k] : 0.f;
+    if constexpr (KV == kI8) o *= vscale;
+    io_t* orow = reinterpret_cast<io_t*>(a.out) + (((int64_t)li * rows_n + (p - q_pos0)) * hq + kvh * group + h) * D + 4 * lane;
     io_t w4[4] = {(io_t)o[0], (io_t)o[1], (io_t)o[2], (io_t)o[3]};
     if constexpr (sizeof(io_t) == 4) *reinterpret_cast<u4*>(orow) = *reinterpret_cast<const u4*>(w4);
     else *reinterpret_cast<u2*>(orow) = *reinterpret_cast<const u2*>(w4);
   }
 }
 
-template <int KV, int IO, int D, int NW, bool CAP>
-hipError_t launch_variant(const PrefillShortArgs& a, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+template <int KV, int IO, int D, int NW, bool CAP, int LAYERS>
+hipError_t launch_variant(const PrefillShortArgs& a, const int32_t* window, int n_layers, hipStream_t stream, hipEvent_t ev0,
+                          hipEvent_t ev1) {
   constexpr int kLds = lds_bytes<KV, D, NW>();
   // more than 64 KiB of LDS has to be requested once per kernel (idempotent: callers on several threads may both ask)
   static std::atomic<bool> configured{false};
   if (!configured.load(std::memory_order_acquire)) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_short_kernel<KV, IO, D, NW, CAP>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_short_kernel<KV, IO, D, NW, CAP, LAYERS>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (e != hipSuccess) return e;
     configured.store(true, std::memory_order_release);
   }
-  const int tiles = short_tiles(a.q_pos0, a.n, a.rows_log2);
-  hipExtLaunchKernelGGL((prefill_short_kernel<KV, IO, D, NW, CAP>), dim3(a.n_layers * a.geom.hkv, tiles), dim3(NW * 64), kLds,
-                        stream, ev0, ev1, 0, a);
+  PrefillWindows<LAYERS> windows{};
+  std::copy(window, window + n_layers, windows.of);
+  hipExtLaunchKernelGGL((prefill_short_kernel<KV, IO, D, NW, CAP, LAYERS>), dim3(n_layers * a.hkv, a.tiles, a.parts), dim3(NW * 64),
+                        kLds, stream, ev0, ev1, 0, a, windows);
   return hipGetLastError();
 }
 
+template <int KV, int IO, int NW, bool CAP>
+hipError_t launch_layers(const PrefillShortArgs& a, const int32_t* window, int n_layers, hipStream_t stream, hipEvent_t ev0,
+                         hipEvent_t ev1) {
+  return n_layers == 1 ? launch_variant<KV, IO, 256, NW, CAP, 1>(a, window, 1, stream, ev0, ev1)
+                       : launch_variant<KV, IO, 256, NW, CAP, kInlineLayers>(a, window, n_layers, stream, ev0, ev1);
+}
+
 template <int KV, int IO>
-hipError_t launch_typed(const PrefillShortArgs& a, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
-  const int tiles = short_tiles(a.q_pos0, a.n, a.rows_log2);
-  if ((long)tiles * a.n_layers * a.geom.hkv > kWideWorkgroups)
-    return a.softcap > 0.f ? launch_variant<KV, IO, 256, 4, true>(a, stream, ev0, ev1)
-                           : launch_variant<KV, IO, 256, 4, false>(a, stream, ev0, ev1);
-  return a.softcap > 0.f ? launch_variant<KV, IO, 256, 8, true>(a, stream, ev0, ev1)
-                         : launch_variant<KV, IO, 256, 8, false>(a, stream, ev0, ev1);
+hipError_t launch_typed(const PrefillShortArgs& a, const int32_t* window, int n_layers, hipStream_t stream, hipEvent_t ev0,
+                        hipEvent_t ev1) {
+  if ((long)a.tiles * n_layers * a.hkv > kWideWorkgroups)
+    return a.softcap > 0.f ? launch_layers<KV, IO, 4, true>(a, window, n_layers, stream, ev0, ev1)
+                           : launch_layers<KV, IO, 4, false>(a, window, n_layers, stream, ev0, ev1);
+  return a.softcap > 0.f ? launch_layers<KV, IO, 8, true>(a, window, n_layers, stream, ev0, ev1)
+                         : launch_layers<KV, IO, 8, false>(a, window, n_layers, stream, ev0, ev1);
 }
 
 }  // namespace
@@ -252,6 +382,26 @@ int prefill_short_rows_log2(int group) {
   int r = 0;
   while ((2 << r) * group <= kCols) ++r;
   return r;
+}
+
+// Parts of the tiles of a call of `wgs` tiles, the longest of `most` key blocks: as few as end the launch first by the
+// times measured (us: a key block of a workgroup 0.72 over a float32 cache, 0.40 over an int8 one, 0.184 otherwise; the parts'
+// way through the workspace 3), a workgroup a compute unit. 300 rows over a float32 cache, 4 heads on 1: three parts, 17.6 us
+// before, 12 now; 100 rows behind 1,000: eight, 45.6 and 19.5 with the step before; 64 behind 3,000, int8, 8 on 2: 31.4 and
+// 18.3; 26 behind 6,843, fp16, 8 on 1: 17.2 against 38.4 on the tiled kernels.
+int prefill_short_parts(int kv_dtype, long wgs, int most) {
+  if (wgs > kShortPartSlots / 2) return 1;
+  const double block = kv_dtype == kF32 ? 0.72 : (kv_dtype == kI8 ? 0.40 : 0.184), merge = 3.0;
+  int best = 1;
+  double t = block * most;
+  for (int p = 2; p <= kShortParts && p * wgs <= kShortPartSlots; ++p) {
+    const double tp = block * std::max((most + p - 1) / p, kMinPartBlocks) + merge;
+    if (tp < t - 0.2) {
+      best = p;
+      t = tp;
+    }
+  }
+  return best;
 }
 
 // Whether the short kernel is expected to finish a call before the tiled kernels of prefill_attn.hip: both sides by
@@ -333,7 +483,10 @@ bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, 
   for (int c = 0; c < xcd_classes; ++c) planes_mean += planes[c] / xcd_classes;
   double t_short;
   if (wgs <= kWideWorkgroups) {
-    t_short = i8 ? 7.2 + 0.44 * short_most + 0.6 * planes_mean : 5.8 + 0.21 * short_most + 0.54 * planes_mean;
+    const int parts = prefill_short_parts(kv_dtype, (long)wgs, (int)short_most);
+    const double walked = parts > 1 ? fmax(ceil(short_most / parts), kMinPartBlocks) : short_most;
+    t_short = i8 ? 6.4 + 0.40 * walked + 0.66 * planes_mean + (parts > 1 ? 3.3 : 0)
+                 : 5.4 + 0.184 * walked + 0.68 * planes_mean + (parts > 1 ? 3.0 : 0);
   } else {
     // The compute units of the busiest engine, in blocks each, with what an L2 too small costs (the workgroups of a unit
     // walk its blocks together while all run at once, and less and less so in more rounds or beside shorter layers) ...
@@ -376,21 +529,32 @@ bool prefill_short_wanted(int kv_dtype, int hq, int hkv, const int32_t* window, 
   return t_short < (i8 ? (wgs > kWideWorkgroups && wgs <= 2 * kCus ? 0.95 : 1.0) : 1.05) * t_tiled;
 }
 
-hipError_t launch_prefill_short(const PrefillShortArgs& a, int kv_dtype, int io_dtype, hipStream_t stream, hipEvent_t ev0,
-                                hipEvent_t ev1) {
-  if (a.n_layers < 1 || a.n_layers > kInlineLayers || a.group < 1 || a.group > kCols || a.n < 1 || a.geom.head_dim != 256)
-    return hipErrorInvalidValue;
-  const int tiles = short_tiles(a.q_pos0, a.n, a.rows_log2);
-  if (tiles > 65535) return hipErrorInvalidValue;
+hipError_t launch_prefill_short(PrefillShortArgs a, const int32_t* window, int n_layers, int kv_dtype, int io_dtype,
+                                hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+  if (n_layers < 1 || n_layers > kInlineLayers || a.group < 1 || a.group > kCols || a.n < 1) return hipErrorInvalidValue;
+  a.rows_log2 = prefill_short_rows_log2(a.group);
+  a.tiles = short_tiles(a.q_pos0, a.n, a.rows_log2);
+  if (a.tiles > 65535) return hipErrorInvalidValue;
+  const int vb = kv_dtype == kF32 ? 16 : (kv_dtype == kI8 ? 64 : 32);
+  int most = 0;
+  for (int l = 0; l < n_layers; ++l) {
+    // (a tile at the end of the call sees the most blocks, but where the window cuts them all alike)
+    const int last = a.q_pos0 + a.n - 1, lo = window[l] > 0 ? std::max(0, (last >> a.rows_log2 << a.rows_log2) - window[l] + 1) : 0;
+    most = std::max(most, last / vb - lo / vb + 1);
+  }
+  a.parts = prefill_short_parts(kv_dtype, (long)a.tiles * n_layers * a.hkv, most);
+  auto inverse = [](int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
+  a.parts_inverse = inverse(a.parts);
+  a.hkv_inverse = inverse(a.hkv);
   switch (kv_dtype * 4 + io_dtype) {
-    case kF32 * 4 + kF32: return launch_typed<kF32, kF32>(a, stream, ev0, ev1);
-    case kF16 * 4 + kF16: return launch_typed<kF16, kF16>(a, stream, ev0, ev1);
-    case kF16 * 4 + kF32: return launch_typed<kF16, kF32>(a, stream, ev0, ev1);
-    case kBF16 * 4 + kBF16: return launch_typed<kBF16, kBF16>(a, stream, ev0, ev1);
-    case kBF16 * 4 + kF32: return launch_typed<kBF16, kF32>(a, stream, ev0, ev1);
-    case kI8 * 4 + kF16: return launch_typed<kI8, kF16>(a, stream, ev0, ev1);
-    case kI8 * 4 + kBF16: return launch_typed<kI8, kBF16>(a, stream, ev0, ev1);
-    case kI8 * 4 + kF32: return launch_typed<kI8, kF32>(a, stream, ev0, ev1);
+    case kF32 * 4 + kF32: return launch_typed<kF32, kF32>(a, window, n_layers, stream, ev0, ev1);
+    case kF16 * 4 + kF16: return launch_typed<kF16, kF16>(a, window, n_layers, stream, ev0, ev1);
+    case kF16 * 4 + kF32: return launch_typed<kF16, kF32>(a, window, n_layers, stream, ev0, ev1);
+    case kBF16 * 4 + kBF16: return launch_typed<kBF16, kBF16>(a, window, n_layers, stream, ev0, ev1);
+    case kBF16 * 4 + kF32: return launch_typed<kBF16, kF32>(a, window, n_layers, stream, ev0, ev1);
+    case kI8 * 4 + kF16: return launch_typed<kI8, kF16>(a, window, n_layers, stream, ev0, ev1);
+    case kI8 * 4 + kBF16: return launch_typed<kI8, kBF16>(a, window, n_layers, stream, ev0, ev1);
+    case kI8 * 4 + kF32: return launch_typed<kI8, kF32>(a, window, n_layers, stream, ev0, ev1);
   }
   return hipErrorInvalidValue;
 }
