@@ -300,28 +300,39 @@ struct NewRows {
 // blocks (a wave each), so many that the merge still has its rows in one trip (32), or two blocks and up to 256 partitions
 // where the context needs more. One layer's step, 4 heads on 1, fp16, us, before this rule (64-token partitions, one up to
 // 512 tokens) / now: 300 tokens 11.3 / 8.1, 520 9.0 / 8.4, 1,152 10.6 / 8.8 (window 512: 9.2 / 7.8), 4,096 12.3 / 10.0,
-// 8,000 14.5 / 10.8; 8 sequences, one partition / a block each: 220 tokens 8.5 / 10.7, 380 11.3 / 10.9.
+// 8,000 14.5 / 10.8; 8 sequences, one partition / a block each: 220 tokens 8.5 / 10.7, 380 11.3 / 10.9. Five blocks a
+// partition of a 16-bit cache are still better than more workgroups where there are three to eight partitions (16 sequences
+// of 1,200, 8 on 2: 11.6 against 12.4, 40 of 900, 4 on 1, 11.2 against 11.9; with 16 partitions 12.7 against 12.3).
 //
-// Larger launches: about 512 workgroups, 1024 where sequences or layers see unequal lengths or the cache is float32 (16 layers x 64 sequences
-// are fastest without any split; one layer in 512 / 1024, us, decode and decode step: 64 sequences of 2,000, 8 heads on 2,
-// fp16 43.5 / 46.2 and 47.4 / 52.8, 40 of 3,000, 4 on 1, 23.1 / 24.5 and 24.1 / 26.5, 47 of 7,490, window 512, 13.9 / 14.5
-// and 15.5 / 17.1, 32 of 2,490, int8, 22.2 / 22.1 and 22.7 / 26.3, 61 ragged ones of up to 5,746 43.4 / 33.7, 11 of 3,874,
-// float32, 38.0 / 33.2; six layers x 4 sequences of 2,496, int8, five with a window of 512: 17.1 / 15.2), partitions of whole 64 tokens (4 layers x 15 float32 sequences of 3,170: 53 us in partitions of 176 tokens, 39 of 192), and one for
-// contexts of up to 512 tokens (64 sequences of 256 / 512 tokens, Hq8/Hkv2: 9.7 / 15.4 us against 11.0 / 16.1 split and
-// merged, 256 sequences 26.9 / 46.3 against 32.4 / 51.8).
+// Larger launches: about 512 workgroups, 1024 where sequences or layers see unequal lengths (16 layers x 64 sequences are
+// fastest without any split; one layer in 512 / 1024, us, decode and decode step: 64 sequences of 2,000, 8 heads on 2, fp16
+// 43.5 / 46.2 and 47.4 / 52.8, 40 of 3,000, 4 on 1, 23.1 / 24.5 and 24.1 / 26.5, 47 of 7,490, window 512, 13.9 / 14.5 and
+// 15.5 / 17.1, 32 of 2,490, int8, 22.2 / 22.1 and 22.7 / 26.3, 61 ragged ones of up to 5,746 43.4 / 33.7; six layers x 4
+// sequences of 2,496, int8, five with a window of 512: 17.1 / 15.2), partitions of whole 64 tokens (4 layers x 15 float32
+// sequences of 3,170: 53 us in partitions of 176 tokens, 39 of 192), and one for contexts of up to 512 tokens (64 sequences
+// of 256 / 512 tokens, Hq8/Hkv2: 9.7 / 15.4 us against 11.0 / 16.1 split and merged, 256 sequences 26.9 / 46.3 against 32.4 /
+// 51.8).
+//
+// Over a float32 cache a block's 128 matrix instructions of 32 cycles bound a wave: up to one workgroup a compute unit, of
+// four waves, where that still cuts every sequence in two (in 1024 single waves / so, decode and decode step: 20 of 3,000,
+// 4 on 1, 26.0 / 24.9 and 35.6 / 27.4, 40 of up to 1,120, 8 on 2, 28.1 / 26.6 and 41.2 / 30.5, 9 of up to 5,000, 4 on 1, 16.9 /
+// 13.9 and 21.8 / 16.4). Several layers of unequal lengths in one call are better in 1024 (4 layers x 15 of up to 3,170: 39
+// against 43.6).
 struct DecodeSplits { int count, align; };
-DecodeSplits choose_decode_splits(int max_len, int min_len, int widest, int narrowest, int heads, int block) {
+DecodeSplits choose_decode_splits(int max_len, int min_len, int widest, int narrowest, int n_layers, int heads, int block) {
   const int blocks = (decode_span(max_len, widest, block) + block - 1) / block;
   if (heads <= kLatencyWorkgroups) {
     if (blocks <= 8) return {1, block};
     const int few = std::min({32, blocks, kLatencyWorkgroups / heads});
-    if (blocks <= 4 * few) return {few, block};
+    if (blocks <= (block == 32 && few >= 3 && few <= 8 ? 5 : 4) * few) return {few, block};
     const int many = std::min((blocks + 1) / 2, kLatencyWorkgroups / heads);
     if (many > 32 && blocks <= 4 * many) return {many, block};
   }
   if (max_len <= 512) return {1, kTokenAlign};
   const int most = decode_span(max_len, widest, 1), least = decode_span(min_len, narrowest, 1);
-  const int target = least * 4 < most * 3 || block == 16 ? 1024 : 512;
+  const bool unequal = least * 4 < most * 3;
+  if (block == 16 && heads <= kLatencyWorkgroups / 2 && !(unequal && n_layers > 1)) return {kLatencyWorkgroups / heads, kTokenAlign};
+  const int target = unequal || block == 16 ? 1024 : 512;
   return {std::max(1, std::min({(target + heads - 1) / heads, (max_len + 63) / 64, 64})), kTokenAlign};
 }
 
@@ -397,7 +408,7 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   }
   int align = kTokenAlign;
   if (num_splits == 0) {
-    const DecodeSplits splits = choose_decode_splits(max_len, min_len, widest, narrowest, n_layers * (whole ? whole->batch : batch) * h->cfg.num_kv_heads,
+    const DecodeSplits splits = choose_decode_splits(max_len, min_len, widest, narrowest, n_layers, n_layers * (whole ? whole->batch : batch) * h->cfg.num_kv_heads,
                                                      decode_block_tokens(h->geom.esize));
     num_splits = splits.count;
     align = splits.align;
