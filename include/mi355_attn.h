@@ -262,14 +262,16 @@ int mi355_attn_decode_step(mi355_attn* handle, int32_t layer, const int32_t* seq
  * mi355_attn_decode for callers that cannot allocate: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc. It has no
  * counterpart in the reference. Same arguments, same kernels and bit-identical
- * results, but the split-KV partials go to a fixed workspace that is part of the
- * library image (8 MiB per GPU, held until the process ends) instead of the
- * handle's growable one, and the call makes no hipMalloc / hipFree.
+ * results, but the call makes no hipMalloc / hipFree: up to 4,096 partial results
+ * of the key range's partitions go to room that the handle holds from its creation
+ * (as those of mi355_attn_decode and mi355_attn_decode_step do), more to a fixed
+ * workspace that is part of the library image (8 MiB per GPU, held until the
+ * process ends) instead of the handle's growable one.
  * Limits: the handle must use device pointers (host_io = 0, else
  * kFailedPrecondition); batch x num_q_heads x num_splits <= 8192 partial results
  * (an explicit num_splits beyond that is kResourceExhausted; with num_splits = 0
  * the library chooses within the limit). All calls on one GPU share the
- * workspace. Calls queued on one stream never overlap. Eager calls on different
+ * library's workspace. Calls queued on one stream never overlap. Eager calls on different
  * streams are ordered by the library (each waits, on its stream, for the event
  * the previous one left), so they do not overlap either. Calls recorded into HIP
  * graphs are not ordered against anything outside their graph: replays of two
@@ -279,10 +281,25 @@ int mi355_attn_decode_step(mi355_attn* handle, int32_t layer, const int32_t* seq
  * alike): up to 64 sequences per call (more need an upload that a capture cannot
  * hold: kFailedPrecondition); kv_lens and seq_ids are baked into the recorded
  * launch, so a replay attends exactly the rows of the captured call - one graph
- * per position - and does not advance the handle's count of appended rows.
+ * per position - and does not advance the handle's count of appended rows. A call
+ * of more than 4,096 partial results other than this one needs the handle's growable
+ * workspace: kFailedPrecondition unless such a call has been made before the capture.
+ * What a recorded call writes to stays with the handle until it is destroyed, whatever
+ * is called in between.
  */
 int mi355_attn_decode_noalloc(mi355_attn* handle, int32_t layer, const int32_t* seq_ids, const int32_t* kv_lens,
                               int32_t batch, const void* q, void* out, int32_t num_splits, char** error_msg);
+
+/*
+ * Host only, no device needed (tests of the launch rules; no counterpart in the reference): the partitions of the key
+ * range that a decode call of `batch` sequences of min_len to max_len rows over n_layers layers runs with (num_splits: 0
+ * by rule, else what the caller asks for; partitions that would hold nothing are not counted). Out, may be NULL:
+ * *merged_in_launch (the attention launch merges the partitions itself, else a second launch does), *rows (partial
+ * results that the call leaves), *fixed_rows (how many a handle has room for from its creation on). < 0 on bad arguments.
+ */
+int mi355_attn_decode_plan_probe(int32_t kv_dtype, int32_t n_layers, int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
+                                 const int32_t* layer_window, int32_t max_len, int32_t min_len, int32_t num_splits,
+                                 int32_t* merged_in_launch, int32_t* rows, int32_t* fixed_rows);
 
 /*
  * Host only, no device needed (tests of the planner; no counterpart in the reference): the work plan that a

@@ -95,6 +95,7 @@ def lib() -> ctypes.CDLL:
     L.mi355_attn_decode_layers.argtypes = [vp, i32, i32, i32p, i32p, i32, vp, vp, i32, errp]
     L.mi355_attn_stream_probe.argtypes = [vp, ctypes.c_uint64, ctypes.c_uint64, i32, i32, errp]
     L.mi355_attn_prefill_route_probe.argtypes = [i32] * 6 + [i32p, i32, i32p]
+    L.mi355_attn_decode_plan_probe.argtypes = [i32] * 5 + [i32p] + [i32] * 3 + [i32p] * 3
     L.mi355_attn_reset.argtypes = [vp, i32, errp]
     L.mi355_attn_sync.argtypes = [vp, errp]
     L.mi355_attn_stream.argtypes = [vp]
@@ -108,7 +109,7 @@ def lib() -> ctypes.CDLL:
     L.mi355_attn_version.restype = ctypes.c_char_p
     for name in ("create", "kv_append", "kv_set_scales", "kv_read", "set_layer_transform", "pre_attention", "prefill",
                  "prefill_layers", "decode", "decode_layers", "decode_step", "decode_noalloc", "prefill_plan_probe",
-                 "prefill_route_probe", "stream_probe", "reset", "sync", "set_timing", "set_option"):
+                 "prefill_route_probe", "decode_plan_probe", "stream_probe", "reset", "sync", "set_timing", "set_option"):
         getattr(L, "mi355_attn_" + name).restype = c
     _lib = L
     return L
@@ -311,6 +312,15 @@ def prefill_route(kv_dtype, q_heads, kv_heads, windows, q_pos0, n, compute_units
     route = lib().mi355_attn_prefill_route_probe(kv_dtype, len(windows), n, q_pos0, q_heads, kv_heads, _i32_array(windows),
                                                  compute_units, ctypes.byref(parts))
     return route, parts.value
+
+
+def decode_plan(kv_dtype, q_heads, kv_heads, windows, lens, num_splits=0):
+    """mi355_attn_decode_plan_probe: (partitions, merged in the launch, partial results, results a handle has room for) of
+    a decode call of len(lens) sequences over len(windows) layers."""
+    merged, rows, fixed = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
+    n = lib().mi355_attn_decode_plan_probe(kv_dtype, len(windows), len(lens), q_heads, kv_heads, _i32_array(windows), max(lens), min(lens),
+                                           num_splits, ctypes.byref(merged), ctypes.byref(rows), ctypes.byref(fixed))
+    return n, bool(merged.value), rows.value, fixed.value
 
 
 def version() -> str:

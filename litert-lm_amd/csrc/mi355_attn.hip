@@ -117,11 +117,14 @@ struct mi355_attn {
   std::vector<LayerTransform> transform;
   std::vector<int32_t> window;
   std::vector<int32_t> filled;  // [layer][seq] rows written since the last reset
-  float* d_short_ws = nullptr;  // prefill of short calls: parts of split tiles (behind the cache, in its allocation)
-  // split-KV workspace
-  float* ws_acc = nullptr;
-  float* ws_ml = nullptr;
-  size_t ws_slots = 0;
+  // Partials of kFixedRows rows, behind the cache in its allocation and there from creation on: the parts of short prefill
+  // calls and the partitions of decode calls of so many partial results, one after the other on the handle's stream.
+  float* d_parts = nullptr;
+  // partials of larger decode calls, allocated on first use
+  float* ws = nullptr;
+  size_t ws_rows = 0;
+  bool ws_recorded = false;      // a recorded call writes to `ws`
+  std::vector<float*> ws_kept;   // earlier ones that recorded calls write to
 
   // ring of (kv_lens, seq_ids) uploads
   int32_t* h_ring = nullptr;
@@ -191,16 +194,52 @@ int stage_out_end(mi355_attn* h, int which, void* p, size_t bytes, char** error_
   return 0;
 }
 
-int ensure_workspace(mi355_attn* h, size_t slots, char** error_msg) {
-  if (h->ws_slots >= slots) return 0;
+// A room for `rows` partial results: accumulator rows, then (max, sum) pairs.
+constexpr size_t kFixedRows = (size_t)kShortPartSlots * kShortPartRows;
+float* partials_ml(const mi355_attn* h, float* acc, size_t rows) { return acc + rows * h->cfg.head_dim; }
+size_t partials_bytes(const mi355_attn* h, size_t rows) { return rows * (h->cfg.head_dim + 2) * sizeof(float); }
+
+// What the rule of plan_decode asks for, at most: below 2,048 workgroups of a KV head's query heads.
+size_t rule_rows(const mi355_attn* h) { return (size_t)2048 * (h->cfg.num_q_heads / h->cfg.num_kv_heads); }
+
+// Room for calls of more than kFixedRows partial results. It is made for whatever the rule may ask for, so that no later
+// length or batch allocates again; only counts of partitions that a caller gives can outgrow it. A recorded call goes on
+// writing to the room that it was recorded with, so that one is kept until the handle goes.
+int ensure_workspace(mi355_attn* h, size_t rows, char** error_msg) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  HIP_OR_RETURN(hipStreamIsCapturing(h->stream, &capturing));
+  const bool recording = capturing != hipStreamCaptureStatusNone;
+  if (h->ws_rows >= rows) {
+    h->ws_recorded |= recording;
+    return 0;
+  }
+  if (recording)
+    return fail(error_msg, MI355_ATTN_FAILED_PRECONDITION,
+                "decode with %zu partial results while the stream is being captured: more than %zu need a workspace that the "
+                "handle allocates on first use (make such a call before the capture)",
+                rows, std::max(h->ws_rows, kFixedRows));
   HIP_OR_RETURN(hipStreamSynchronize(h->stream));
-  if (h->ws_acc) HIP_OR_RETURN(hipFree(h->ws_acc));
-  if (h->ws_ml) HIP_OR_RETURN(hipFree(h->ws_ml));
-  h->ws_acc = h->ws_ml = nullptr;
-  h->ws_slots = 0;
-  HIP_OR_RETURN(hipMalloc(&h->ws_acc, slots * h->cfg.head_dim * sizeof(float)));
-  HIP_OR_RETURN(hipMalloc(&h->ws_ml, slots * 2 * sizeof(float)));
-  h->ws_slots = slots;
+  if (h->ws_recorded) {
+    try {
+      h->ws_kept.push_back(h->ws);
+    } catch (const std::bad_alloc&) {
+      return fail(error_msg, MI355_ATTN_RESOURCE_EXHAUSTED, "out of host memory");
+    }
+  } else if (h->ws) {
+    HIP_OR_RETURN(hipFree(h->ws));
+  }
+  h->ws = nullptr;
+  h->ws_rows = 0;
+  h->ws_recorded = false;
+  size_t room = std::max(rows, rule_rows(h));
+  hipError_t e = hipMalloc(&h->ws, partials_bytes(h, room));
+  if (e == hipErrorOutOfMemory && room > rows) {
+    (void)hipGetLastError();
+    room = rows;
+    e = hipMalloc(&h->ws, partials_bytes(h, room));
+  }
+  HIP_OR_RETURN(e);
+  h->ws_rows = room;
   return 0;
 }
 
@@ -250,8 +289,6 @@ void fill_decode_common(const mi355_attn* h, DecodeLaunch* l) {
   DecodeArgs& a = l->args;
   a.cache = h->cache;
   a.scales = h->scales;
-  a.ws_acc = h->ws_acc;
-  a.ws_ml = h->ws_ml;
   a.plane_bytes = h->geom.plane_bytes;
   a.hkv = h->geom.hkv;
   a.max_seqs = h->geom.max_seqs;
@@ -336,8 +373,52 @@ DecodeSplits choose_decode_splits(int max_len, int min_len, int widest, int narr
   return {std::max(1, std::min({(target + heads - 1) / heads, (max_len + 63) / 64, 64})), kTokenAlign};
 }
 
-// no_alloc: the call may not allocate (mi355_attn_decode_noalloc): device pointers only, and the
-// partials go to this GPU's `scratch` instead of the handle's growable workspace.
+// What a decode launch looks like: its partitions, those of them that hold anything, and the partial results they leave.
+struct DecodeShape {
+  const int32_t* window;  // of its layers
+  int n_layers, batch;
+  int rule_batch;         // as in DecodeLaunch
+  int hq, hkv, esize;
+  int max_len, min_len;
+};
+struct DecodePlan {
+  int num_splits, align;
+  int widest;             // window of its layers, 0: a layer without one
+  size_t rows;            // partial results (0: one partition)
+  bool merges_itself;
+};
+// num_splits: 0 by rule, then so many that `most_rows` hold their results (at least one).
+DecodePlan plan_decode(const DecodeShape& s, int num_splits, size_t most_rows) {
+  DecodePlan p{num_splits, kTokenAlign, s.window[0], 0, false};
+  int narrowest = p.widest;
+  for (int l = 1; l < s.n_layers; ++l) {
+    const int w = s.window[l];
+    if (w == 0 || (p.widest > 0 && w > p.widest)) p.widest = w;
+    if (w > 0 && (narrowest == 0 || w < narrowest)) narrowest = w;
+  }
+  const size_t heads = (size_t)s.n_layers * s.batch * s.hq;
+  if (num_splits == 0) {
+    const DecodeSplits splits = choose_decode_splits(s.max_len, s.min_len, p.widest, narrowest, s.n_layers,
+                                                     s.n_layers * s.rule_batch * s.hkv, decode_block_tokens(s.esize));
+    p.align = splits.align;
+    p.num_splits = std::max(1, (int)std::min((size_t)splits.count, most_rows / heads));
+  }
+  // Partitions are rounded up, so fewer may cover the context than were asked for (4,096 tokens in 18: sixteen of 256): the
+  // launch has no workgroups for the others. (Their size stays what it is: any count in between gives the same.)
+  int used = 1;
+  for (int l = 0; l < s.n_layers; ++l) {
+    if (l > 0 && s.window[l] == s.window[l - 1]) continue;
+    const int per = decode_partition_tokens(s.max_len, s.window[l], p.num_splits, p.align);
+    used = std::max(used, (decode_span(s.max_len, s.window[l], p.align) + per - 1) / per);
+  }
+  p.num_splits = used;
+  p.rows = used > 1 ? heads * used : 0;
+  p.merges_itself = decode_merges_itself(s.n_layers, s.rule_batch, s.hkv, used);
+  return p;
+}
+
+// no_alloc: the call may not allocate (mi355_attn_decode_noalloc): device pointers only, and partials
+// that do not fit the handle's fixed room go to this GPU's `scratch` instead of the handle's workspace.
 // new_rows: q holds raw query projections and the new token's key / value rows come with the call
 // (its row, kv_lens[b] - 1, need not have been appended).
 // The batch a launch is a part of (mi355_attn_decode_step cuts large batches into several launches): the launch rules
@@ -395,48 +476,39 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   }
   HIP_OR_RETURN(hipSetDevice(h->device));
   const int items = n_layers * batch;
-  const bool splits_chosen = num_splits == 0;
   if (whole) {
     max_len = whole->max_len;
     min_len = whole->min_len;
   }
-  int widest = h->window[layer_begin], narrowest = widest;  // windows of the layers (0: none, the widest of all)
-  for (int l = layer_begin + 1; l < layer_begin + n_layers; ++l) {
-    const int w = h->window[l];
-    if (w == 0 || (widest > 0 && w > widest)) widest = w;
-    if (w > 0 && (narrowest == 0 || w < narrowest)) narrowest = w;
-  }
-  int align = kTokenAlign;
-  if (num_splits == 0) {
-    const DecodeSplits splits = choose_decode_splits(max_len, min_len, widest, narrowest, n_layers, n_layers * (whole ? whole->batch : batch) * h->cfg.num_kv_heads,
-                                                     decode_block_tokens(h->geom.esize));
-    num_splits = splits.count;
-    align = splits.align;
-  }
+  // no_alloc: the library's own choice of partitions is trimmed to the workspace; an explicit count is an error
+  const size_t asked = (size_t)items * h->cfg.num_q_heads * num_splits;
+  if (no_alloc && num_splits > 1 && asked > kNoAllocSlots)
+    return fail(error_msg, MI355_ATTN_RESOURCE_EXHAUSTED,
+                "mi355_attn_decode_noalloc: %d layers x %d sequences x %d query heads x %d partitions = %zu partial "
+                "results, the fixed workspace holds %zu (pass fewer partitions, or 0 to let the library choose)",
+                n_layers, batch, h->cfg.num_q_heads, num_splits, asked, kNoAllocSlots);
+  const DecodeShape shape{h->window.data() + layer_begin, n_layers, batch, whole ? whole->batch : batch, h->cfg.num_q_heads,
+                          h->cfg.num_kv_heads, h->geom.esize, max_len, min_len};
+  const DecodePlan plan = plan_decode(shape, num_splits, no_alloc ? kNoAllocSlots : SIZE_MAX);
+  num_splits = plan.num_splits;
+  // The partials: in the handle's fixed room where they fit it, so that a call of up to a workgroup a compute unit neither
+  // allocates nor depends on an earlier call, recorded or not; larger ones in the workspace of the handle, or (no_alloc) in
+  // this GPU's `scratch`.
+  const bool in_scratch = no_alloc && plan.rows > kFixedRows;
+  if (!no_alloc && plan.rows > kFixedRows)
+    if (int rc = ensure_workspace(h, plan.rows, error_msg)) return rc;
   DecodeLaunch launch;
   DecodeArgs& a = launch.args;
-  const size_t slots = (size_t)items * h->cfg.num_q_heads * num_splits;
-  if (no_alloc) {
-    // the library's own choice of partitions is trimmed to the workspace; an explicit count is an error
-    if (num_splits > 1 && slots > kNoAllocSlots) {
-      if (splits_chosen) {
-        num_splits = (int)(kNoAllocSlots / ((size_t)items * h->cfg.num_q_heads));
-      } else {
-        return fail(error_msg, MI355_ATTN_RESOURCE_EXHAUSTED,
-                    "mi355_attn_decode_noalloc: %d layers x %d sequences x %d query heads x %d partitions = %zu partial "
-                    "results, the fixed workspace holds %zu (pass fewer partitions, or 0 to let the library choose)",
-                    n_layers, batch, h->cfg.num_q_heads, num_splits, slots, kNoAllocSlots);
-      }
-      if (num_splits < 1) num_splits = 1;
-    }
-  } else if (num_splits > 1) {
-    if (int rc = ensure_workspace(h, slots, error_msg)) return rc;
-  }
   fill_decode_common(h, &launch);
-  if (no_alloc) {
-    float* const base = g_scratch_ptr[h->device];  // this GPU's copy of `scratch`
-    a.ws_acc = base;
-    a.ws_ml = base + kNoAllocSlots * kNoAllocHeadDim;
+  if (plan.rows <= kFixedRows) {
+    a.ws_acc = h->d_parts;
+    a.ws_ml = partials_ml(h, a.ws_acc, kFixedRows);
+  } else if (in_scratch) {
+    a.ws_acc = g_scratch_ptr[h->device];
+    a.ws_ml = a.ws_acc + kNoAllocSlots * kNoAllocHeadDim;
+  } else {
+    a.ws_acc = h->ws;
+    a.ws_ml = partials_ml(h, h->ws, h->ws_rows);
   }
   const size_t io_bytes = (size_t)items * h->cfg.num_q_heads * h->cfg.head_dim * io_size(h);
   const void* dq = nullptr;
@@ -489,24 +561,14 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   launch.n_layers = n_layers;
   launch.max_kv_len = max_len;
   launch.min_kv_len = min_len;
-  launch.widest_window = widest;
-  launch.rule_batch = whole ? whole->batch : batch;
-  // Partitions are rounded up, so fewer may cover the context than were asked for (4,096 tokens in 18: sixteen of 256): the
-  // launch has no workgroups for the others. (Their size stays what it is: any count in between gives the same.)
-  int used = 1;
-  for (int l = layer_begin; l < layer_begin + n_layers; ++l) {
-    const int window = h->window[l];
-    if (l > layer_begin && window == h->window[l - 1]) continue;
-    const int per = decode_partition_tokens(max_len, window, num_splits, align);
-    used = std::max(used, (decode_span(max_len, window, align) + per - 1) / per);
-  }
-  num_splits = used;
+  launch.widest_window = plan.widest;
+  launch.rule_batch = shape.rule_batch;
   a.num_splits = num_splits;
-  a.align = align;
-  if (decode_merges_itself(n_layers, launch.rule_batch, a.hkv, num_splits)) a.tickets = h->d_tickets;
+  a.align = plan.align;
+  if (plan.merges_itself) a.tickets = h->d_tickets;
   fill_inline_windows(h, &launch);
   bool scratch_fence = false;
-  if (no_alloc && num_splits > 1) {
+  if (in_scratch) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     HIP_OR_RETURN(hipStreamIsCapturing(h->stream, &capturing));
     scratch_fence = capturing == hipStreamCaptureStatusNone;
@@ -576,8 +638,8 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
     a.out = dout;
     a.cache = h->cache;
     a.scales = h->scales;
-    a.ws_acc = h->d_short_ws;
-    a.ws_ml = h->d_short_ws + (size_t)kShortPartSlots * kShortPartRows * h->cfg.head_dim;
+    a.ws_acc = h->d_parts;
+    a.ws_ml = partials_ml(h, a.ws_acc, kFixedRows);
     a.tickets = h->d_tickets;
     a.plane_bytes = h->geom.plane_bytes;
     a.hkv = h->geom.hkv;
@@ -835,12 +897,12 @@ int mi355_attn_create(const mi355_attn_config* c, mi355_attn** out, char** error
   } else {
     h->stream = static_cast<hipStream_t>(c->stream);  // nullptr is the HIP default stream
   }
-  // Behind the cache, in one allocation (another of its own took creating and freeing a handle 0.35 ms longer): the parts of
-  // short prefill calls, 4 MiB. Here and not on first use: a call that is recorded into a graph then runs as it does eagerly.
+  // Behind the cache, in one allocation (another of its own took creating and freeing a handle 0.35 ms longer): the fixed room
+  // for partials, 4 MiB. Here and not on first use: a call that is recorded into a graph then runs as it does eagerly.
   const uint64_t parts_at = (h->cache_bytes + 255) / 256 * 256;
-  if ((e = hipMalloc(&h->cache, parts_at + sizeof(float) * kShortPartSlots * kShortPartRows * (size_t)(c->head_dim + 2))) != hipSuccess)
+  if ((e = hipMalloc(&h->cache, parts_at + partials_bytes(h, kFixedRows))) != hipSuccess)
     return bail(MI355_ATTN_RESOURCE_EXHAUSTED, "KV cache allocation", e);
-  h->d_short_ws = reinterpret_cast<float*>(h->cache + parts_at);
+  h->d_parts = reinterpret_cast<float*>(h->cache + parts_at);
   // Rows that were never written must read as finite numbers: a masked key
   // still enters P.V with probability 0, and 0 * NaN would poison the output.
   if ((e = hipMemsetAsync(h->cache, 0, h->cache_bytes, h->stream)) != hipSuccess)
@@ -905,8 +967,8 @@ void mi355_attn_destroy(mi355_attn* h) {
   if (h->d_q_stage) (void)hipFree(h->d_q_stage);
   if (h->d_kv_stage) (void)hipFree(h->d_kv_stage);
   if (h->d_transform) (void)hipFree(h->d_transform);
-  if (h->ws_acc) (void)hipFree(h->ws_acc);
-  if (h->ws_ml) (void)hipFree(h->ws_ml);
+  if (h->ws) (void)hipFree(h->ws);
+  for (float* ws : h->ws_kept) (void)hipFree(ws);
   if (h->d_ring) (void)hipFree(h->d_ring);
   if (h->h_ring) (void)hipHostFree(h->h_ring);
   if (h->d_items) (void)hipFree(h->d_items);
@@ -1149,6 +1211,21 @@ int mi355_attn_prefill_route_probe(int32_t kv_dtype, int32_t n_layers, int32_t n
   if (split.direct) return MI355_ATTN_ROUTE_DIRECT16;
   a.kchunk = split.kchunk;
   return prefill_takes_plan(a, prefill_work_items(a), compute_units) ? MI355_ATTN_ROUTE_PLANNED16 : MI355_ATTN_ROUTE_TILED32;
+}
+
+int mi355_attn_decode_plan_probe(int32_t kv_dtype, int32_t n_layers, int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
+                                 const int32_t* layer_window, int32_t max_len, int32_t min_len, int32_t num_splits,
+                                 int32_t* merged_in_launch, int32_t* rows, int32_t* fixed_rows) {
+  if (kv_dtype < MI355_ATTN_F32 || kv_dtype > MI355_ATTN_I8 || n_layers < 1 || batch < 1 || batch > 65535 || num_kv_heads < 1 ||
+      num_q_heads < num_kv_heads || num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > kMaxGroup || !layer_window ||
+      min_len < 1 || max_len < min_len || num_splits < 0 || num_splits > kMaxSplits)
+    return -1;
+  const DecodeShape shape{layer_window, n_layers, batch, batch, num_q_heads, num_kv_heads, dtype_size(kv_dtype), max_len, min_len};
+  const DecodePlan plan = plan_decode(shape, num_splits, SIZE_MAX);
+  if (merged_in_launch) *merged_in_launch = plan.merges_itself;
+  if (rows) *rows = (int32_t)std::min<size_t>(plan.rows, INT32_MAX);
+  if (fixed_rows) *fixed_rows = (int32_t)kFixedRows;
+  return plan.num_splits;
 }
 
 int mi355_attn_decode_step(mi355_attn* h, int32_t layer, const int32_t* seq_ids, const int32_t* kv_lens, int32_t batch,
