@@ -285,7 +285,10 @@ int mi355_attn_decode_step(mi355_attn* handle, int32_t layer, const int32_t* seq
  * of more than 4,096 partial results other than this one needs the handle's growable
  * workspace: kFailedPrecondition unless such a call has been made before the capture.
  * What a recorded call writes to stays with the handle until it is destroyed, whatever
- * is called in between.
+ * is called in between. Partial results (of decode calls and of short prefill calls) lie
+ * in memory of the handle, in the order of its stream: replays that run at the same time
+ * as another call or replay of the same handle spoil the results of both (not those of
+ * later calls) - keep them on one stream, or ordered by events.
  */
 int mi355_attn_decode_noalloc(mi355_attn* handle, int32_t layer, const int32_t* seq_ids, const int32_t* kv_lens,
                               int32_t batch, const void* q, void* out, int32_t num_splits, char** error_msg);

@@ -95,8 +95,8 @@ struct DecodeArgs {
   const float* scales;       // int8 cache only
   float* ws_acc;             // [items][hq][num_splits][D] partial accumulators
   float* ws_ml;              // [items][hq][num_splits][2] partial (max, sum)
-  uint32_t* tickets;         // [items][hkv] visible keys whose partials are written, all zero between launches; nullptr:
-                             // the partials are merged by a launch of their own
+  uint32_t* tickets;         // [items][hkv] what the workgroups whose partials are written have added (ticket_share), all zero
+                             // between launches; nullptr: the partials are merged by a launch of their own
   int64_t plane_bytes;       // as in CacheGeom
   int32_t hkv, max_seqs;
   int32_t hq, group;
@@ -172,6 +172,12 @@ inline bool decode_merges_itself(int n_layers, int rule_batch, int hkv, int num_
   return num_splits > 1 && num_splits <= 64 && (int64_t)n_layers * rule_batch * hkv * num_splits <= kLatencyWorkgroups;
 }
 
+// What a workgroup adds to the ticket of its row (or tile) when its part of `part_size` keys (or key blocks) of `total` is
+// written: the size, and the first part the total less. The sum over all parts is 0 and over any fewer is not, so the
+// workgroup that brings the ticket to 0 is the last, and nobody has to clear it. Launches that overlap by a caller's mistake
+// (replays of graphs of one handle) may spoil each other's results, but leave the tickets at 0 for the calls that follow.
+MI355_HD uint32_t ticket_share(int part, int part_size, int total) { return (uint32_t)part_size - (part == 0 ? (uint32_t)total : 0u); }
+
 // Tokens per split-KV partition for a layer with the given window: the same
 // formula runs in the attention kernel and in the merge kernel.
 MI355_HD int decode_span(int max_kv_len, int window, int align) {
@@ -239,7 +245,7 @@ struct PrefillShortArgs {
   const uint8_t* cache;
   const float* scales;  // int8 cache only
   float* ws_acc;        // parts of split tiles: [unit][tile][part][16 columns] x D and x 2 floats, and a ticket per (unit, tile)
-  float* ws_ml;         // that counts key blocks, all zero between launches (used only where parts > 1)
+  float* ws_ml;         // of the parts' key blocks (ticket_share), all zero between launches (used only where parts > 1)
   uint32_t* tickets;
   int64_t plane_bytes;  // as in CacheGeom
   int32_t hkv, max_seqs;

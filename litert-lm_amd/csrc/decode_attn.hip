@@ -705,19 +705,16 @@ decode_attn_kernel(const DecodeArgs a, const DecodeWork<ITEMS, LAYERS> work, con
   }
   if (!tickets) return;
 
-  // The merge of the partials by the workgroup that writes the last of them: every workgroup counts the keys of its
-  // partition once its stores have been acknowledged (device scope: they and the loads below go through to memory, the
+  // The merge of the partials by the workgroup that writes the last of them: every workgroup adds its share of the keys to the
+  // ticket once its stores have been acknowledged (device scope: they and the loads below go through to memory, the
   // workgroups of a row sit on different XCDs, whose L2s are different ones; no cache is written back or invalidated).
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   lds_barrier();
   uint32_t* const sm_last = reinterpret_cast<uint32_t*>(smem);
   if (threadIdx.x == 0) {
     uint32_t* ticket = tickets + item * hkv + kvh;
-    const uint32_t mine = p_hi - p_lo;
-    const uint32_t before = __hip_atomic_fetch_add(ticket, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool last = before + mine == (uint32_t)(kv_len - start);
-    if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-    *sm_last = last;
+    const uint32_t mine = ticket_share(split, p_hi - p_lo, kv_len - start);
+    *sm_last = __hip_atomic_fetch_add(ticket, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine == 0;
   }
   lds_barrier();
   if (!__builtin_amdgcn_readfirstlane((int)*sm_last)) return;

@@ -55,8 +55,8 @@ constexpr int lds_bytes() {
 // compute unit instead of two.
 //
 // A call of few tiles cuts each of them into up to `parts` stretches of its key blocks, a workgroup each (grid z). A part
-// leaves its unnormalised sums, maxima and totals in the workspace by device-scope stores, counts its blocks on the tile's
-// ticket, and the workgroup whose count completes the tile adds the parts up in order (as decode_attn_kernel does).
+// leaves its unnormalised sums, maxima and totals in the workspace by device-scope stores, adds its share of the blocks to the
+// tile's ticket, and the workgroup that completes the tile adds the parts up in order (as decode_attn_kernel does).
 template <int KV, int IO, int D, int NW, bool CAP, int LAYERS>
 __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const PrefillShortArgs a, const PrefillWindows<LAYERS> windows) {
   using io_t = typename IoT<IO>::type;
@@ -285,11 +285,8 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_short_kernel(const Prefill
     uint32_t* const sm_last = reinterpret_cast<uint32_t*>(smem);
     if (threadIdx.x == 0) {
       uint32_t* ticket = a.tickets + unit * tiles + tile;
-      const uint32_t mine = blk_end - blk0;
-      const uint32_t before = __hip_atomic_fetch_add(ticket, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const bool last = before + mine == (uint32_t)tile_blocks;
-      if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-      *sm_last = last;
+      const uint32_t mine = ticket_share(blockIdx.z, blk_end - blk0, tile_blocks);
+      *sm_last = __hip_atomic_fetch_add(ticket, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine == 0;
     }
     lds_barrier();
     if (!__builtin_amdgcn_readfirstlane((int)*sm_last)) return;

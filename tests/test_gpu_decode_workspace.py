@@ -133,3 +133,39 @@ def test_noalloc_calls_of_more_results_than_a_handle_has_room_for_are_ordered_ac
         torch.cuda.synchronize()
         for i in range(2):
             assert all(torch.equal(x, want[i]) for x in got[i])
+
+
+def test_overlapping_replays_leave_later_calls_alone():
+    """Replays of one handle that run at the same time spoil each other's results at most: what follows is right again."""
+    hq, hkv, ctx = 4, 1, 1152
+    side, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(side), handle(A.F32, A.F32, hq, hkv, ctx, 1, side) as at:
+        qd, qp = rnd(1, (1, hq, D), torch.float32), rnd(2, (100, hq, D), torch.float32)
+        assert A.decode_plan(A.F32, hq, hkv, [0], [ctx])[1] and A.decode_plan(A.F32, hq, hkv, [0], [700])[1]
+        calls = [lambda o: at.decode(0, [ctx], qd, o), lambda o: at.decode(0, [700], qd, o), lambda o: at.prefill(0, 0, 1000, 100, qp, o)]
+        want = [torch.empty_like(q) for q in (qd, qd, qp)]
+        for call, o in zip(calls, want):
+            call(o)
+        graphs = []
+        for call, q in zip(calls, (qd, qd, qp)):
+            out = torch.empty_like(q)
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=side):
+                call(out)
+            graphs.append((g, out))
+        side.synchronize()
+        for rep in range(20):
+            for i in range(30):
+                with torch.cuda.stream(side if i % 2 else second):
+                    graphs[(i + rep) % 3][0].replay()
+            torch.cuda.synchronize()
+            for (g, out), call, w in zip(graphs, calls, want):
+                out.fill_(float("nan"))
+                g.replay()
+                side.synchronize()
+                assert torch.equal(out, w), rep
+                out.fill_(float("nan"))
+                call(out)
+                side.synchronize()
+                assert torch.equal(out, w), rep
+        del g, graphs
