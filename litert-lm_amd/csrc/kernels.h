@@ -92,6 +92,7 @@ hipError_t launch_prefill_short(PrefillShortArgs args, const int32_t* window, in
                                 hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
 // Parts that the tiles of a call are cut into: `wgs` tiles in all, the longest of `most` key blocks.
 int prefill_short_parts(int kv_dtype, long wgs, int most);
+int prefill_short_call_parts(int kv_dtype, int group, int hkv, const int32_t* window, int n_layers, int q_pos0, int n);
 
 // Scatter n boundary-layout rows into the cache planes / gather them back.
 hipError_t launch_kv_append(const KvCopyArgs& args, hipStream_t stream);

@@ -1194,8 +1194,10 @@ int mi355_attn_prefill_route_probe(int32_t kv_dtype, int32_t n_layers, int32_t n
   if (parts) *parts = 1;
   if (kv_dtype == MI355_ATTN_I8 && n < kI8MinRows) return MI355_ATTN_ROUTE_ROWWISE;
   if (short_prefill_takes(n_layers, n) &&
-      prefill_short_wanted(kv_dtype, num_q_heads, num_kv_heads, layer_window, n_layers, q_pos0, n))
+      prefill_short_wanted(kv_dtype, num_q_heads, num_kv_heads, layer_window, n_layers, q_pos0, n)) {
+    if (parts) *parts = prefill_short_call_parts(kv_dtype, num_q_heads / num_kv_heads, num_kv_heads, layer_window, n_layers, q_pos0, n);
     return MI355_ATTN_ROUTE_SHORT;
+  }
   if (kv_dtype == MI355_ATTN_F32) return MI355_ATTN_ROUTE_ROWWISE;
   PrefillArgs a{};
   a.n_layers = n_layers;

@@ -401,6 +401,18 @@ int prefill_short_parts(int kv_dtype, long wgs, int most) {
   return best;
 }
 
+int prefill_short_call_parts(int kv_dtype, int group, int hkv, const int32_t* window, int n_layers, int q_pos0, int n) {
+  const int rows_log2 = prefill_short_rows_log2(group);
+  const int vb = kv_dtype == kF32 ? 16 : (kv_dtype == kI8 ? 64 : 32);
+  int most = 0;
+  for (int l = 0; l < n_layers; ++l) {
+    // (a tile at the end of the call sees the most blocks, but where the window cuts them all alike)
+    const int last = q_pos0 + n - 1, lo = window[l] > 0 ? std::max(0, (last >> rows_log2 << rows_log2) - window[l] + 1) : 0;
+    most = std::max(most, last / vb - lo / vb + 1);
+  }
+  return prefill_short_parts(kv_dtype, (long)short_tiles(q_pos0, n, rows_log2) * n_layers * hkv, most);
+}
+
 // Whether the short kernel is expected to finish a call before the tiled kernels of prefill_attn.hip: both sides by
 // formulas fitted to measured times (head_dim 256, MI355X, calls queued back to back, 1,140 shapes spread at random over
 // 16 to 4,096 rows behind 0 to 12,000 cached ones, 1 to 34 layers with and without windows, sixteen head counts). Nine
@@ -532,14 +544,7 @@ hipError_t launch_prefill_short(PrefillShortArgs a, const int32_t* window, int n
   a.rows_log2 = prefill_short_rows_log2(a.group);
   a.tiles = short_tiles(a.q_pos0, a.n, a.rows_log2);
   if (a.tiles > 65535) return hipErrorInvalidValue;
-  const int vb = kv_dtype == kF32 ? 16 : (kv_dtype == kI8 ? 64 : 32);
-  int most = 0;
-  for (int l = 0; l < n_layers; ++l) {
-    // (a tile at the end of the call sees the most blocks, but where the window cuts them all alike)
-    const int last = a.q_pos0 + a.n - 1, lo = window[l] > 0 ? std::max(0, (last >> a.rows_log2 << a.rows_log2) - window[l] + 1) : 0;
-    most = std::max(most, last / vb - lo / vb + 1);
-  }
-  a.parts = prefill_short_parts(kv_dtype, (long)a.tiles * n_layers * a.hkv, most);
+  a.parts = prefill_short_call_parts(kv_dtype, a.group, a.hkv, window, n_layers, a.q_pos0, a.n);
   auto inverse = [](int d) { return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; };
   a.parts_inverse = inverse(a.parts);
   a.hkv_inverse = inverse(a.hkv);

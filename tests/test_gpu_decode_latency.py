@@ -1,7 +1,7 @@
 """GPU parity of decode launches of up to one workgroup a compute unit, whose partials are merged by the workgroup that
 writes the last of them, and of the launches next to them, against the float64 oracle: partitions of one key block up to
-more than the merge has in one trip (16, 32, 64), counts on both sides of what merges itself, contexts that end inside, at
-and behind a block, sequences of unequal lengths (some with a single partition), windows, more different windows than a
+more than the merge has in one trip, contexts that end inside, at and behind a block (exact counts of partitions, up to the
+most, are in test_gpu_decode_partitions.py), sequences of unequal lengths (some with a single partition), windows, more different windows than a
 launch carries, 16 query heads on a KV head, repeated calls (the tickets are zero again), replays of a graph; and the fused
 step against its two calls on both sides of the line between row waves of their own and shared ones.
 

@@ -1,7 +1,8 @@
 """GPU parity of short prefill calls whose tiles are cut over the keys into parts that the launch merges itself, against the
-float64 oracle: from one tile (eight parts) to 128 (two) and one more (none), contexts that leave the last part short or
-missing, windows that cut the tiles unequally, several layers and KV heads, every pair of types, repeated calls (the tickets
-are zero again) and replays of a graph recorded before any eager call.
+float64 oracle: from one tile (eight parts) to 128 (two, which fill the workspace and the tickets to their end) and one more
+(none), contexts that leave the last part short or missing, windows that cut the tiles unequally, several layers and KV heads,
+one to 16 query heads a KV head, soft-capped scores, every pair of types, repeated calls (the tickets are zero again) and
+replays of a graph recorded before any eager call.
 
 Bounds, of the largest value: 1e-5 for a float32 cache, 2e-3 otherwise (half operands; bfloat16 outputs are compared after
 discounting the half ulp of the format).
@@ -63,7 +64,7 @@ def test_parts_of_tiles(kv, io, hq, hkv):
                 stream=torch.cuda.current_stream().cuda_stream) as at:
         at.set_option("prefill_short", 1)
         rows = [fill(at, kv, layer, L, hkv, 10 * layer + 1) for layer in range(len(windows))]
-        # (tiles of 1, 4 or 5 positions: from one of them to more than 128)
+        # (tiles of 4 positions: from one of them to more than 128)
         for q_pos0, n in ((2299, 1), (2049, 3), (1000, 63), (1, 300), (1780, 513)):
             for layers in ((0, 1), (0, 2)):
                 qd, qr = rounded(gen(900 + n, layers[1], n, hq, D), io)
@@ -79,6 +80,32 @@ def test_parts_of_tiles(kv, io, hq, hkv):
                     ref = c_oracle.sdpa_f64(qr[i], k, v, 0.07, q_pos0=q_pos0, window=windows[layers[0] + i], kv_len=q_pos0 + n)
                     err = orc.rel_err_beyond_bf16_rounding(got[i], ref) if io == A.BF16 else float(np.abs(got[i] - ref).max() / np.abs(ref).max())
                     assert err < (1e-5 if kv == A.F32 else 2e-3), (q_pos0, n, layers, i, err)
+
+
+# query heads, KV heads, start, rows, parts of a tile, soft cap
+SHAPES = [(4, 1, 1500, 512, 2, 0.0), (4, 1, 1500, 512, 2, 30.0), (4, 1, 1500, 513, 1, 0.0), (16, 1, 3000, 20, 8, 0.0), (16, 1, 3000, 100, 2, 30.0),
+          (1, 1, 3000, 300, 8, 0.0), (1, 1, 3001, 64, 8, 30.0), (8, 2, 3000, 64, 8, 0.0)]
+
+
+@pytest.mark.parametrize("kv,io", PAIRS)
+@pytest.mark.parametrize("hq,hkv,start,n,parts,softcap", SHAPES)
+def test_counts_of_parts(kv, io, hq, hkv, start, n, parts, softcap):
+    if parts > 1:
+        assert A.prefill_route(kv, hq, hkv, [0], start, n) == (A.ROUTE_SHORT, parts)
+    with A.Attn(1, hq, hkv, D, start + n, 1, kv, io, scale=0.07, softcap=softcap, stream=torch.cuda.current_stream().cuda_stream) as at:
+        at.set_option("prefill_short", 1)
+        k, v = fill(at, kv, 0, start + n, hkv, 3)
+        qd, qr = rounded(gen(n, n, hq, D), io)
+        if io == A.F32 and kv in (A.F16, A.BF16):  # (what the matrix cores take, by definition)
+            qd, qr = rounded(rounded(qr, kv)[1], A.F32)
+        out = torch.full_like(qd, float("nan"))
+        for _ in range(2):  # (the second call finds the tickets as the first has left them)
+            at.prefill(0, 0, start, n, qd, out)
+        torch.cuda.synchronize()
+        got = out.float().cpu().numpy()
+        ref = c_oracle.sdpa_f64(qr, k, v, 0.07, q_pos0=start, softcap=softcap, kv_len=start + n)
+        err = orc.rel_err_beyond_bf16_rounding(got, ref) if io == A.BF16 else float(np.abs(got - ref).max() / np.abs(ref).max())
+        assert err < (1e-5 if kv == A.F32 else 2e-3), err
 
 
 @pytest.mark.parametrize("kv", [A.F16, A.F32, A.I8])

@@ -54,6 +54,8 @@ MEASURED = [
     (A.I8, 8, 2, 1, 0, 3072, 256, 47.0, 31.0),
     (A.I8, 4, 1, 1, 0, 3072, 1024, 42.7, 37.0),
     (A.I8, 8, 4, 2, 512, 31, 762, 37.3, 24.1),
+    # few tiles behind a long context, in parts
+    (A.F16, 8, 1, 1, 0, 6843, 26, 38.4, 17.2),
 ]
 
 
@@ -74,6 +76,13 @@ def test_routes_at_their_limits():
     assert A.prefill_route(A.BF16, 4, 1, windows(26, 512), 0, 1024) == (A.ROUTE_PLANNED16, 1)
     assert A.prefill_route(A.F16, 8, 2, [0], 6157, 2047) == (A.ROUTE_DIRECT16, 4)
     assert A.prefill_route(A.I8, 8, 2, [0], 3072, 1024) == (A.ROUTE_TILED32, 4)
+
+
+def test_parts_of_short_calls():
+    """Few tiles of many key blocks are cut over the keys, into at most eight parts and 256 workgroups."""
+    for kv, hq, hkv, start, n, parts in ((A.F16, 8, 1, 6843, 26, 8), (A.F32, 4, 1, 0, 300, 3), (A.F32, 4, 1, 1000, 100, 8), (A.I8, 8, 2, 3000, 64, 8),
+                                         (A.F32, 4, 1, 1500, 512, 2), (A.F32, 4, 1, 1500, 513, 1), (A.F32, 4, 1, 0, 64, 1)):
+        assert A.prefill_route(kv, hq, hkv, [0], start, n) == (A.ROUTE_SHORT, parts), (kv, start, n)
 
 
 def test_arguments_are_checked():
