@@ -162,6 +162,7 @@ struct DecodeLaunch {
   int32_t max_kv_len = 0;    // max over kv_lens, sizes the partitions
   int32_t min_kv_len = 0;    // min over kv_lens
   int32_t widest_window = 0; // of the launch's layers, 0: a layer without one
+  int32_t rule_splits = 1;   // partitions the launch rules count: those asked for, before empty ones are left out
   int32_t rule_batch = 0;    // sequences the launch rules count: batch, or those of the larger batch this launch is a part of
 };
 // Launches of up to one workgroup a compute unit are bound by latency: they have waves for the rows of the fused step and

@@ -821,10 +821,10 @@ hipError_t launch_typed(const DecodeLaunch& l, const DecodeTuning& t, hipStream_
     // 1,152 tokens in partitions of two blocks: 8.8 us with two waves, 9.4 with
     // one, 9.2 with four; of one block: 7.8, 8.1 with two).
     constexpr int VB = KvT<KV>::VB;
-    const int wgs = l.n_layers * l.rule_batch * a.hkv * a.num_splits;
+    const int heads = l.n_layers * l.rule_batch * a.hkv, wgs = heads * a.num_splits;
     const int blocks = decode_partition_tokens(l.max_kv_len, l.widest_window, a.num_splits, a.align) / VB;
     if (wgs <= kLatencyWorkgroups) waves = blocks >= 3 ? 4 : blocks;
-    else waves = wgs >= 768 || a.num_splits > 1 || blocks <= 2 ? 1 : 2;
+    else waves = heads * l.rule_splits >= 768 || blocks <= 2 ? 1 : 2;
     // ... and four waves for a big launch of whole sequences of unequal lengths: the wave slots of
     // the chip then hold a quarter of the workgroups at a time instead of all of them, and the short
     // sequences, dispatched last, fill in behind the long ones (16 layers x 64 sequences of 256 to

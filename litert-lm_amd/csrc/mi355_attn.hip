@@ -341,14 +341,15 @@ struct NewRows {
 // partition of a 16-bit cache are still better than more workgroups where there are three to eight partitions (16 sequences
 // of 1,200, 8 on 2: 11.6 against 12.4, 40 of 900, 4 on 1, 11.2 against 11.9; with 16 partitions 12.7 against 12.3).
 //
-// Larger launches: about 512 workgroups, 1024 where sequences or layers see unequal lengths (16 layers x 64 sequences are
-// fastest without any split; one layer in 512 / 1024, us, decode and decode step: 64 sequences of 2,000, 8 heads on 2, fp16
-// 43.5 / 46.2 and 47.4 / 52.8, 40 of 3,000, 4 on 1, 23.1 / 24.5 and 24.1 / 26.5, 47 of 7,490, window 512, 13.9 / 14.5 and
-// 15.5 / 17.1, 32 of 2,490, int8, 22.2 / 22.1 and 22.7 / 26.3, 61 ragged ones of up to 5,746 43.4 / 33.7; six layers x 4
-// sequences of 2,496, int8, five with a window of 512: 17.1 / 15.2), partitions of whole 64 tokens (4 layers x 15 float32
-// sequences of 3,170: 53 us in partitions of 176 tokens, 39 of 192), and one for contexts of up to 512 tokens (64 sequences
-// of 256 / 512 tokens, Hq8/Hkv2: 9.7 / 15.4 us against 11.0 / 16.1 split and merged, 256 sequences 26.9 / 46.3 against 32.4 /
-// 51.8).
+// Larger launches: about 1,024 workgroups, in at most 64 partitions a sequence (one or two KV heads have fewer workgroups
+// then), partitions of whole 64 tokens (4 layers x 15 float32 sequences of 3,170: 53 us in partitions of 176 tokens, 39 of
+// 192), and one for contexts of up to 512 tokens (64 sequences of 256 / 512 tokens, Hq8/Hkv2: 9.7 / 15.4 us against 11.0 /
+// 16.1 split and merged, 256 sequences 26.9 / 46.3 against 32.4 / 51.8). Half as many workgroups would make decode steps of
+// equal lengths 4 to 7 % faster (64 sequences of 2,000, 8 on 2, fp16 48.3 against 51.9 us; decode itself 43.5 / 45.6, over an
+// int8 cache 1 % slower, in the mean of 34 shapes as fast), but would lose precision: probabilities enter P.V as halves
+// relative to the maximum of a wave's keys, so the heaviest key of each wave is exact, and with half the waves the error
+// against 64 bits grows (30 layers x 4,096 2.67e-4 to 2.73e-4, 32 int8 sequences 3.40e-4 to 3.44e-4, over 12 seeds each,
+// whose spread is 1e-6).
 //
 // Over a float32 cache a block's 128 matrix instructions of 32 cycles bound a wave: up to one workgroup a compute unit, of
 // four waves, where that still cuts every sequence in two (in 1024 single waves / so, decode and decode step: 20 of 3,000,
@@ -369,8 +370,7 @@ DecodeSplits choose_decode_splits(int max_len, int min_len, int widest, int narr
   const int most = decode_span(max_len, widest, 1), least = decode_span(min_len, narrowest, 1);
   const bool unequal = least * 4 < most * 3;
   if (block == 16 && heads <= kLatencyWorkgroups / 2 && !(unequal && n_layers > 1)) return {kLatencyWorkgroups / heads, kTokenAlign};
-  const int target = unequal || block == 16 ? 1024 : 512;
-  return {std::max(1, std::min({(target + heads - 1) / heads, (max_len + 63) / 64, 64})), kTokenAlign};
+  return {std::max(1, std::min({(1024 + heads - 1) / heads, (max_len + 63) / 64, 64})), kTokenAlign};
 }
 
 // What a decode launch looks like: its partitions, those of them that hold anything, and the partial results they leave.
@@ -383,13 +383,14 @@ struct DecodeShape {
 };
 struct DecodePlan {
   int num_splits, align;
+  int asked;              // partitions before those that hold nothing are left out
   int widest;             // window of its layers, 0: a layer without one
   size_t rows;            // partial results (0: one partition)
   bool merges_itself;
 };
 // num_splits: 0 by rule, then so many that `most_rows` hold their results (at least one).
 DecodePlan plan_decode(const DecodeShape& s, int num_splits, size_t most_rows) {
-  DecodePlan p{num_splits, kTokenAlign, s.window[0], 0, false};
+  DecodePlan p{num_splits, kTokenAlign, num_splits, s.window[0], 0, false};
   int narrowest = p.widest;
   for (int l = 1; l < s.n_layers; ++l) {
     const int w = s.window[l];
@@ -401,14 +402,14 @@ DecodePlan plan_decode(const DecodeShape& s, int num_splits, size_t most_rows) {
     const DecodeSplits splits = choose_decode_splits(s.max_len, s.min_len, p.widest, narrowest, s.n_layers,
                                                      s.n_layers * s.rule_batch * s.hkv, decode_block_tokens(s.esize));
     p.align = splits.align;
-    p.num_splits = std::max(1, (int)std::min((size_t)splits.count, most_rows / heads));
+    p.asked = std::max(1, (int)std::min((size_t)splits.count, most_rows / heads));
   }
   // Partitions are rounded up, so fewer may cover the context than were asked for (4,096 tokens in 18: sixteen of 256): the
   // launch has no workgroups for the others. (Their size stays what it is: any count in between gives the same.)
   int used = 1;
   for (int l = 0; l < s.n_layers; ++l) {
     if (l > 0 && s.window[l] == s.window[l - 1]) continue;
-    const int per = decode_partition_tokens(s.max_len, s.window[l], p.num_splits, p.align);
+    const int per = decode_partition_tokens(s.max_len, s.window[l], p.asked, p.align);
     used = std::max(used, (decode_span(s.max_len, s.window[l], p.align) + per - 1) / per);
   }
   p.num_splits = used;
@@ -563,6 +564,7 @@ int decode_impl(mi355_attn* h, int layer_begin, int n_layers, const int32_t* seq
   launch.min_kv_len = min_len;
   launch.widest_window = plan.widest;
   launch.rule_batch = shape.rule_batch;
+  launch.rule_splits = plan.asked;
   a.num_splits = num_splits;
   a.align = plan.align;
   if (plan.merges_itself) a.tickets = h->d_tickets;

@@ -56,6 +56,14 @@ def test_partitions_that_hold_nothing_are_not_counted():
     assert A.decode_plan(A.F16, 8, 2, [0], [1], 64)[0] == 1
 
 
+@pytest.mark.parametrize("kv,hq,hkv,layers,batch,n,splits", [
+    (A.F16, 8, 2, 30, 1, 4096, 16), (A.I8, 8, 2, 1, 32, 4096, 16), (A.F16, 8, 2, 1, 64, 2000, 8), (A.BF16, 4, 1, 1, 40, 3000, 24),
+    (A.I8, 8, 2, 1, 32, 2490, 13), (A.BF16, 4, 1, 26, 1, 6000, 32), (A.I8, 4, 1, 1, 64, 6000, 16), (A.F16, 8, 2, 6, 8, 2000, 11)])
+def test_large_launches_run_in_about_1024_workgroups(kv, hq, hkv, layers, batch, n, splits):
+    """Half as many lose precision: the heaviest key of a wave is the one whose probability is exact in half."""
+    assert A.decode_plan(kv, hq, hkv, [0] * layers, [n] * batch)[0] == splits
+
+
 def test_arguments_are_checked():
     w = (ctypes.c_int32 * 1)(0)
     probe = A.lib().mi355_attn_decode_plan_probe
