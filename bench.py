@@ -174,7 +174,7 @@ def bench_decode_c3(A, torch, steps, warmup, layers=30, rotation=4, splits=16, c
         def one_launch(r):
             at.decode(r * layers, lens, q[r], out[r], num_splits=splits, n_layers=layers, batch=1)
 
-        def per_layer_chain(r):  # layer l + 1 of a forward pass needs layer l's output: one launch (+ merge) per layer, in order
+        def per_layer_chain(r):  # layer l + 1 of a forward pass needs layer l's output: one launch (its merge inside) per layer, in order
             for layer in range(layers):  # (partition count by the library's own rule for a one-layer launch)
                 at.decode(r * layers + layer, lens, q[r, layer], out[r, layer], num_splits=0, batch=1)
 
@@ -197,7 +197,7 @@ def bench_decode_c3(A, torch, steps, warmup, layers=30, rotation=4, splits=16, c
             graph = {
                 "what": "the headline step replayed from HIP graphs (captured calls of the same C ABI, one graph per cache "
                         "set): `one_launch` = the multi-layer launch + merge; `per_layer_chain` = the 30 layers as 30 "
-                        "launches (+ merges) in dependency order, the shape a forward pass over a model issues",
+                        "launches (each merging its own partials) in dependency order, the shape a forward pass over a model issues",
                 "one_launch": {"us_per_step": round(sec_g1 * 1e6, 2), "GBps": round(step_bytes / sec_g1 / 1e9, 1),
                                "frac_of_hbm_peak": round(step_bytes / sec_g1 / 1e9 / HBM_PEAK_GBS, 4),
                                "equals_eager_output": ok1},
@@ -468,7 +468,7 @@ def pipeline_report(X, device_resident, two_call_decode_step=False):
 
 
 def protocol_layer_latency(A, torch, ctx=1152):
-    """Latency of one decode attention call (attention + merge launches, queued back to back) at the shape of the
+    """Latency of one decode attention call (attention with the merge inside, queued back to back) at the shape of the
     benchmark protocol's decode turn: Hq4 / Hkv1, fp16, about the middle context of the 256 steps."""
     at = A.Attn(1, 4, 1, D, 2048, 1, A.F16, A.F16)
     fill_cache(at, torch, 1, [ctx], 1, torch.float16, seed=7)

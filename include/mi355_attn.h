@@ -364,8 +364,10 @@ void* mi355_attn_stream(mi355_attn* handle);
 
 /*
  * Duration in milliseconds of the kernel of the most recent
- * prefill / decode / pre_attention call, measured with HIP events on the handle's stream
- * (the split-merge pass is excluded). Blocks until that call has finished.
+ * prefill / decode / pre_attention call, measured with HIP events on the handle's stream.
+ * A merge of partial results is included where the kernel does it itself (decode calls of up
+ * to 256 workgroups and 64 partitions, short prefill calls) and excluded where it is a launch
+ * of its own. Blocks until that call has finished.
  * Timing is recorded only after mi355_attn_set_timing(handle, 1).
  */
 int mi355_attn_set_timing(mi355_attn* handle, int32_t enabled);
@@ -381,8 +383,9 @@ float mi355_attn_last_kernel_ms(mi355_attn* handle);
  *                      over more than 64 layers or 65,535 rows and under option
  *                      rowwise_prefill), 0 never, -1 (default): by rule, where none of
  *                      the options below asks for another kernel (an fp32 cache, which
- *                      the tiled kernels do not take: always). It needs no room beside
- *                      the cache, int8 included
+ *                      the tiled kernels do not take: always). It allocates nothing:
+ *                      the parts that it cuts few tiles into go to room that the
+ *                      handle holds from its creation
  *   "prefill_i8_min_rows" int8 cache: prefill calls of fewer rows run row by row
  *                      (default 16) unless prefill_short is 1
  *   "prefill_i8_stage_mib" int8 cache: limit of the staging area for half planes,

@@ -170,17 +170,6 @@ __device__ __forceinline__ void stream_blocks(float sc, float softcap, __amdgpu_
   // The four lanes (g = 0..3) of a head each summed their own tokens.
 }
 
-// Log-sum-exp merge of the split-KV partials: grid (query head, sequence, layer), a wave for every 16 partitions (up to
-// four) that adds up their rows with four channels per lane. A launch of its own for decode launches of more workgroups than
-// compute units, where it takes 4 us and the workgroups of the attention have their slots for the next ones; smaller
-// launches merge themselves (decode_attn_kernel). What neither does is write back and invalidate an L2, the other way to
-// make partials visible to another XCD: a fence pair per workgroup made the launch several times slower.
-//
-// Bound: latency. A launch moves a few hundred KiB; its time is its trips to memory one behind the other, so there are
-// two, the arguments, then all (max, sum) pairs and rows at once, and the instructions of a single wave, so it is
-// straight-line code (rows that hold nothing are read as zeros through a resource that ends in front of them, and weigh 0).
-// INL and the argument loads in front of the first read of the partials: as in decode_attn_kernel.
-
 // What a workgroup works on: its sequence's slot, length and row in q / out, its layer's window and partition size.
 struct Place { int seq, kv_len, row, window, per; };
 template <int ITEMS, int LAYERS>
@@ -236,6 +225,18 @@ using PreBlock = std::conditional_t<PRE != 0, DecodePre, NoBlock>;
 constexpr int kMergeRows = 16;  // partitions of a wave at a time
 MI355_HD int merge_waves(int num_splits) { return num_splits >= 49 ? 4 : (num_splits + kMergeRows - 1) / kMergeRows; }
 
+// Log-sum-exp merge of the split-KV partials: grid (query head, sequence, layer), a wave for every 16 partitions (up to
+// four) that adds up their rows with four channels per lane. A launch of its own for decode launches of more workgroups than
+// compute units or of more than 64 partitions, where it takes 4 to 5 us and the workgroups of the attention have their slots
+// for the next ones; smaller launches merge themselves (decode_attn_kernel). What neither does is write back and invalidate
+// an L2, the other way to make partials visible to another XCD: a fence pair per workgroup made the launch several times
+// slower.
+//
+// Bound: latency. A launch moves a few hundred KiB to a few MiB; its time is its trips to memory one behind the other, so
+// there are two, the arguments, then all (max, sum) pairs and rows at once, and the instructions of a single wave, so it is
+// straight-line code (rows that hold nothing are read as zeros through a resource that ends in front of them, and weigh 0).
+// More than 64 partitions come in further trips of 64.
+// INL and the argument loads in front of the first read of the partials: as in decode_attn_kernel.
 template <int KV, int IO, int D, int ITEMS, int LAYERS, bool INL>
 __global__ void __launch_bounds__(256)
 decode_merge_kernel(const DecodeArgs a, const DecodeWork<ITEMS, LAYERS> work, const TableBlock<INL> tab) {
@@ -315,12 +316,11 @@ decode_merge_kernel(const DecodeArgs a, const DecodeWork<ITEMS, LAYERS> work, co
   else *reinterpret_cast<u2*>(orow) = *reinterpret_cast<const u2*>(o);
 }
 
-// INL: lengths, sequence ids and windows travel in the argument block (the host
-// knows: a.inline_items and n_layers <= kInlineLayers). Then everything in front
-// of the first loads is one round of scalar loads at addresses that depend on
-// the block index only. (With both sources behind one `cond ? a.inline_x[b] :
-// a.x[b]` the compiler selects a pointer and issues vector loads, one after the
-// other, and a wave spent 2 to 4 us before its first K/V load.)
+// INL: lengths, sequence ids and windows travel in the argument block (inline_place; the host
+// knows: DecodeLaunch::inline_items and inline_layers). Then everything in front of the first
+// loads is one round of scalar loads at addresses that depend on the block index only. (With
+// both sources in one kernel, behind a condition per value, the compiler selects a pointer and
+// issues vector loads, one after the other, and a wave spent 2 to 4 us before its first K/V load.)
 //
 // PRE (with INL, one layer): the kernel runs the step before attention for the one new token of its
 // sequence itself (row t = kv_len - 1): every workgroup norms and rotates the query rows of its KV

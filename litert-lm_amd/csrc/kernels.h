@@ -15,8 +15,8 @@ struct DecodeTuning {
 
 bool decode_supported(int kv_dtype, int io_dtype, int head_dim);
 
-// Queues the decode attention kernel (bracketed by ev0/ev1 when non-null) and,
-// for num_splits > 1, the log-sum-exp merge kernel.
+// Queues the decode attention kernel (bracketed by ev0/ev1 when non-null) and, where it leaves partials that it does not
+// merge itself (num_splits > 1 without tickets), the log-sum-exp merge kernel.
 hipError_t launch_decode(const DecodeLaunch& launch, int kv_dtype, int io_dtype, const DecodeTuning& tuning,
                          hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
 

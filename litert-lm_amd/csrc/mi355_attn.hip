@@ -633,7 +633,8 @@ int prefill_impl(mi355_attn* h, int layer_begin, int n_layers, int seq, int q_po
   if (int rc = stage_in(h, 0, q, io_bytes, &dq, error_msg)) return rc;
   if (int rc = stage_out_begin(h, 1, out, io_bytes, &dout, error_msg)) return rc;
   hipEvent_t e0 = h->timing ? h->ev0 : nullptr, e1 = h->timing ? h->ev1 : nullptr;
-  // The short kernel first: it reads the planes as they are and needs no room, neither now nor while a graph is recorded.
+  // The short kernel first: it reads the planes as they are, and the room for its parts and its tickets are there from the
+  // handle's creation, so nothing is allocated, neither now nor while a graph is recorded.
   if (takes_short_prefill(h, layer_begin, n_layers, q_pos0, n)) {
     PrefillShortArgs a{};
     a.q = dq;

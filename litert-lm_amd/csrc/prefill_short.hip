@@ -383,9 +383,9 @@ int prefill_short_rows_log2(int group) {
 
 // Parts of the tiles of a call of `wgs` tiles, the longest of `most` key blocks: as few as end the launch first by the
 // times measured (us: a key block of a workgroup 0.72 over a float32 cache, 0.40 over an int8 one, 0.184 otherwise; the parts'
-// way through the workspace 3), a workgroup a compute unit. 300 rows over a float32 cache, 4 heads on 1: three parts, 17.6 us
-// before, 12 now; 100 rows behind 1,000: eight, 45.6 and 19.5 with the step before; 64 behind 3,000, int8, 8 on 2: 31.4 and
-// 18.3; 26 behind 6,843, fp16, 8 on 1: 17.2 against 38.4 on the tiled kernels.
+// way through the workspace 3), a workgroup a compute unit. Whole tiles / parts, us a call back to back: 300 rows over a float32
+// cache, 4 heads on 1: three parts, 16.6 / 13.6; 100 rows behind 1,000: eight, 42.0 / 15.3; 64 behind 3,000, int8, 8 on 2: eight,
+// 28.2 / 14.4; 26 behind 6,843, fp16, 8 on 1: eight, 66.8 / 16.7, and 38.1 on the tiled kernels.
 int prefill_short_parts(int kv_dtype, long wgs, int most) {
   if (wgs > kShortPartSlots / 2) return 1;
   const double block = kv_dtype == kF32 ? 0.72 : (kv_dtype == kI8 ? 0.40 : 0.184), merge = 3.0;
@@ -415,13 +415,13 @@ int prefill_short_call_parts(int kv_dtype, int group, int hkv, const int32_t* wi
 
 // Whether the short kernel is expected to finish a call before the tiled kernels of prefill_attn.hip: both sides by
 // formulas fitted to measured times (head_dim 256, MI355X, calls queued back to back, 1,140 shapes spread at random over
-// 16 to 4,096 rows behind 0 to 12,000 cached ones, 1 to 34 layers with and without windows, sixteen head counts). Nine
-// tenths of the times are within 15 % of the formulas, and what they choose takes 0.3 % longer than the better side in
-// the mean (on 320 other shapes 0.4 %, five of them by 10 to 15 %). Examples, tiled / short, us: bfloat16, 4 query heads on 1 KV head, one layer of 64 rows 9.9 / 5.1, 256 rows
-// 15.9 / 8.0, 1,024 rows 25.7 / 13.6, 1,370 rows behind 1,338 35 / 38, 17 behind 1,207 19 / 14, 26 layers of 256 rows
-// 20 / 28; 8 heads on 2, 2 layers of 1,768 behind 693 83 / 96. int8 cache, 300 rows 24 / 10, 256 rows behind 3,072
-// 47 / 31. A float32 cache always takes the short kernel: the alternative is one decode item per row, which reads every
-// key once per position instead of once per 16 columns (300 rows 36 / 17, 300 behind 2,000 305 / 81).
+// 16 to 4,096 rows behind 0 to 12,000 cached ones, 1 to 34 layers with and without windows, sixteen head counts; the formula
+// of calls of up to 256 tiles again, with their parts, to 133). On 296 other shapes of both kernels what they choose takes 0.3 %
+// longer than the better side in the mean, three of them by 10 to 31 % (the worst 26 layers of 34 rows behind 249, 16 heads
+// on 2: 25 / 19). Examples, tiled / short, us: bfloat16, 4 query heads on 1 KV head, one layer of 256 rows 17.2 / 7.0, 1,024
+// rows 25.8 / 12.0; 8 heads on 2, 2 layers of 1,768 behind 693 83 / 96. int8 cache, 300 rows 21.8 / 9.5, 64 rows behind 3,000
+// 31.2 / 14.4. A float32 cache always takes the short kernel: the alternative is one decode item per row, which reads every
+// key once per position instead of once per 16 columns (300 rows 36 / 13.6, 300 behind 2,000 305 / 33.5).
 //
 // What decides for the short kernel beside the key blocks themselves is where its workgroups run. They go round the eight
 // XCDs and, within each, round its four engines of eight compute units, with the units (layer x KV head) varying fastest:
