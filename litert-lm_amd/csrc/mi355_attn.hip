@@ -207,7 +207,8 @@ size_t rule_rows(const mi355_attn* h) { return (size_t)2048 * (h->cfg.num_q_head
 // writing to the room that it was recorded with, so that one is kept until the handle goes.
 int ensure_workspace(mi355_attn* h, size_t rows, char** error_msg) {
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  HIP_OR_RETURN(hipStreamIsCapturing(h->stream, &capturing));
+  // (the default stream cannot be captured, and asking about it while another stream is captured is an error)
+  if (h->stream) HIP_OR_RETURN(hipStreamIsCapturing(h->stream, &capturing));
   const bool recording = capturing != hipStreamCaptureStatusNone;
   if (h->ws_rows >= rows) {
     h->ws_recorded |= recording;

@@ -114,6 +114,25 @@ def test_recorded_call_keeps_its_workspace_when_a_later_one_outgrows_it():
         del g
 
 
+def test_large_call_on_the_default_stream_while_another_stream_is_captured():
+    hq, hkv, ctx, B = 8, 2, 1024, 40
+    side = torch.cuda.Stream()
+    with A.Attn(1, hq, hkv, D, ctx, B, A.F16, A.F16, stream=0) as at:
+        for b in range(B):
+            at.kv_append(0, b, 0, rnd(2 * b, (ctx, hkv, D), torch.float16), rnd(2 * b + 1, (ctx, hkv, D), torch.float16))
+        q = rnd(5, (B, hq, D), torch.float16)
+        want, out, x = torch.empty_like(q), torch.empty_like(q), torch.zeros(4, device=DEV)
+        at.decode(0, [ctx] * B, q, want, num_splits=16)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side, capture_error_mode="thread_local"):
+            x += 1
+            at.decode(0, [ctx] * B, q, out, num_splits=16)  # (runs: the handle's stream is not the one captured)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        del g
+
+
 def test_noalloc_calls_of_more_results_than_a_handle_has_room_for_are_ordered_across_streams():
     hq, hkv, ctx, B = 8, 2, 1024, 40
     assert A.decode_plan(A.F16, hq, hkv, [0], [ctx] * B, 16)[2] > A.decode_plan(A.F16, hq, hkv, [0], [ctx] * B, 16)[3]
